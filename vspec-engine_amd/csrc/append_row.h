@@ -25,6 +25,11 @@ struct AppendParams {
     const float* rope_sin;
     uint32_t rope_dim;
     uint32_t max_pos;
+    bool rope_vec;  // the rotary tables' rows may be read 16 bytes at a time
+    // query rows [batch][n_new][hq][head_dim] rotated into q_out (q_in != null)
+    const float* q_in;
+    float* q_out;
+    uint32_t hq;
     // with start_pos and token_item null: source token b goes to position ctx_lens[b] - 1
     // (the decode step's append; a context of 0 appends nothing)
     const int32_t* ctx_lens;
@@ -150,7 +155,25 @@ __device__ __forceinline__ uint32_t int4_v_tile_byte(uint32_t slot, uint32_t c, 
     return (16u * tg + nn) * (D / 8u) + 4u * c + 2u * (tr & 1u) + (tr >> 1);
 }
 
-template <int DT, int SRC>
+// N elements (a multiple of 8) from element el on, as floats
+template <int SRC, int N>
+__device__ __forceinline__ void load_elements(const uint8_t* src, size_t el, float (&x)[N]) {
+    if constexpr (SRC == VSPEC_KV_F32) {
+        const float4* s4 = reinterpret_cast<const float4*>(src + el * 4);
+#pragma unroll
+        for (int j = 0; j < N / 4; ++j) {
+            const float4 w = s4[j];
+            x[4 * j] = w.x; x[4 * j + 1] = w.y; x[4 * j + 2] = w.z; x[4 * j + 3] = w.w;
+        }
+    } else {
+        const uint4* s4 = reinterpret_cast<const uint4*>(src + el * 2);
+#pragma unroll
+        for (int j = 0; j < N / 8; ++j) unpack_f16x8(s4[j], x + 8 * j);
+    }
+}
+
+// ROPE: the launch may carry rotary tables (without it their code and registers go)
+template <int DT, int SRC, bool ROPE = true>
 __device__ __forceinline__ void append_chunk(const AppendParams& p, uint32_t seq, uint32_t pos, uint32_t h,
                                              uint32_t c, int which, size_t src_el, FlagOp* defer = nullptr) {
     constexpr int EPT = append_ept(DT);
@@ -160,25 +183,14 @@ __device__ __forceinline__ void append_chunk(const AppendParams& p, uint32_t seq
     // flight together
     float x[EPT];
     const uint8_t* src = which ? p.v_new : p.k_new;
-    if constexpr (SRC == VSPEC_KV_F32) {
-        const float4* s4 = reinterpret_cast<const float4*>(src + src_el * 4);
-#pragma unroll
-        for (int j = 0; j < EPT / 4; ++j) {
-            const float4 w = s4[j];
-            x[4 * j] = w.x; x[4 * j + 1] = w.y; x[4 * j + 2] = w.z; x[4 * j + 3] = w.w;
-        }
-    } else {
-        const uint4* s4 = reinterpret_cast<const uint4*>(src + src_el * 2);
-#pragma unroll
-        for (int j = 0; j < EPT / 8; ++j) unpack_f16x8(s4[j], x + 8 * j);
-    }
+    load_elements<SRC, EPT>(src, src_el, x);
     const int32_t phys = p.block_tables[(size_t)seq * p.max_blocks + lb];
     if (phys < 0 || (uint32_t)phys >= p.num_blocks) return;
     const uint32_t slot = pos % p.block_tokens;
     const size_t row = ((size_t)phys * p.hkv + h) * p.block_tokens + slot;
     const size_t e0 = (size_t)c * EPT;  // first element of this chunk within the row
 
-    const bool rope = p.rope_cos != nullptr;
+    const bool rope = ROPE && p.rope_cos != nullptr;
     if (rope) {
         if (pos >= p.max_pos) return;  // no table row: the token is not written
         if (!which) {
@@ -190,20 +202,36 @@ __device__ __forceinline__ void append_chunk(const AppendParams& p, uint32_t seq
             const size_t row0 = src_el - e0;  // element 0 of this token-head row
             const float* cr = p.rope_cos + (size_t)pos * half;
             const float* sr = p.rope_sin + (size_t)pos * half;
+            if (p.rope_vec && half % EPT == 0) {
+                // the chunk lies whole in the first or the second half of the rotated
+                // elements, or past them: its partners and table entries are one run each
+                if (e0 < p.rope_dim) {
+                    const bool first = e0 < half;
+                    const uint32_t i0 = first ? (uint32_t)e0 : (uint32_t)e0 - half;
+                    float other[EPT], cv[EPT], sv[EPT];
+                    load_elements<SRC, EPT>(src, row0 + (first ? e0 + half : e0 - half), other);
+                    load_elements<VSPEC_KV_F32, EPT>(reinterpret_cast<const uint8_t*>(cr), i0, cv);
+                    load_elements<VSPEC_KV_F32, EPT>(reinterpret_cast<const uint8_t*>(sr), i0, sv);
 #pragma unroll
-            for (int e = 0; e < EPT; ++e) {
-                const uint32_t d = (uint32_t)e0 + e;
-                if (d >= p.rope_dim) continue;
-                const uint32_t i = d < half ? d : d - half;
-                const size_t pe = row0 + (d < half ? d + half : d - half);
-                float other;
-                if constexpr (SRC == VSPEC_KV_F32) {
-                    other = reinterpret_cast<const float*>(src)[pe];
-                } else {
-                    other = half_bits_to_float(reinterpret_cast<const uint16_t*>(src)[pe]);
+                    for (int e = 0; e < EPT; ++e)
+                        x[e] = first ? x[e] * cv[e] - other[e] * sv[e] : other[e] * sv[e] + x[e] * cv[e];
                 }
-                const float c = cr[i], sn = sr[i];
-                x[e] = d < half ? x[e] * c - other * sn : other * sn + x[e] * c;
+            } else {
+#pragma unroll
+                for (int e = 0; e < EPT; ++e) {
+                    const uint32_t d = (uint32_t)e0 + e;
+                    if (d >= p.rope_dim) continue;
+                    const uint32_t i = d < half ? d : d - half;
+                    const size_t pe = row0 + (d < half ? d + half : d - half);
+                    float other;
+                    if constexpr (SRC == VSPEC_KV_F32) {
+                        other = reinterpret_cast<const float*>(src)[pe];
+                    } else {
+                        other = half_bits_to_float(reinterpret_cast<const uint16_t*>(src)[pe]);
+                    }
+                    const float c = cr[i], sn = sr[i];
+                    x[e] = d < half ? x[e] * c - other * sn : other * sn + x[e] * c;
+                }
             }
         }
     }
@@ -284,6 +312,10 @@ __device__ __forceinline__ AppendParams decode_step_append_params(const DecodePa
     a.rope_sin = nullptr;
     a.rope_dim = 0;
     a.max_pos = 0;
+    a.rope_vec = false;
+    a.q_in = nullptr;
+    a.q_out = nullptr;
+    a.hq = 0;
     a.ctx_lens = p.ctx_lens;
     a.k_new = p.k_new;
     a.v_new = p.v_new;
@@ -303,11 +335,26 @@ __device__ __forceinline__ uint64_t append_items(const AppendParams& p) {
     return (uint64_t)p.batch * p.n_new * p.hkv * (p.head_dim / append_ept(DT)) * 2;
 }
 
+// Where source token b (packed tokens, or sequence b's first token) goes: block-table row
+// and position.  False: nowhere.
+__device__ __forceinline__ bool append_where(const AppendParams& p, uint32_t b, int32_t& item, int32_t& sp) {
+    item = p.token_item ? p.token_item[b] : (int32_t)b;
+    if (p.token_item) {
+        sp = p.token_pos[b];
+    } else if (p.start_pos) {
+        sp = p.start_pos[b];
+    } else {
+        const int32_t cl = p.ctx_lens[b];
+        sp = cl > 0 ? cl - 1 : -1;
+    }
+    return sp >= 0 && item >= 0 && !(p.token_item && (uint32_t)item >= p.n_items);
+}
+
 // One work item of the append kernel (any order; no two items write the same bytes):
 // item `it` = ((token, kv head, chunk) << 1) | which.  Uniform batch (start_pos), packed
 // tokens (token_item / token_pos, items not below n_items skipped) or the decode step's
 // token at ctx_lens[b] - 1.
-template <int DT, int SRC>
+template <int DT, int SRC, bool ROPE = true>
 __device__ __forceinline__ void append_item(const AppendParams& p, uint64_t it) {
     constexpr int EPT = append_ept(DT);
     const uint32_t chunks = p.head_dim / EPT;
@@ -320,19 +367,169 @@ __device__ __forceinline__ void append_item(const AppendParams& p, uint64_t it) 
     const uint32_t i = (uint32_t)(r % p.n_new);
     const uint32_t b = (uint32_t)(r / p.n_new);
 
-    const int32_t item = p.token_item ? p.token_item[b] : (int32_t)b;
-    int32_t sp;
-    if (p.token_item) {
-        sp = p.token_pos[b];
-    } else if (p.start_pos) {
-        sp = p.start_pos[b];
-    } else {
-        const int32_t cl = p.ctx_lens[b];
-        sp = cl > 0 ? cl - 1 : -1;
-    }
-    if (sp < 0 || item < 0 || (p.token_item && (uint32_t)item >= p.n_items)) return;
+    int32_t item, sp;
+    if (!append_where(p, b, item, sp)) return;
     const size_t src_el = (((size_t)b * p.n_new + i) * p.hkv + h) * p.head_dim + (size_t)c * EPT;
-    append_chunk<DT, SRC>(p, (uint32_t)item, (uint32_t)sp + i, h, c, which, src_el);
+    append_chunk<DT, SRC, ROPE>(p, (uint32_t)item, (uint32_t)sp + i, h, c, which, src_el);
+}
+
+// ---------------------------------------------------------------------------
+// f16 and f32 pools, items by section: K chunks, then V chunks, then query chunks (each
+// section a whole number of workgroups).  The K section is one 8-element chunk of one row
+// an item, as append_item's; the V section of f16 pools takes a chunk of a whole group of
+// 4 tokens where the launch holds the group's tokens, since a group's chunk is 64
+// contiguous bytes of the pool while one token's is eight 2-byte pieces.
+// ---------------------------------------------------------------------------
+
+// V items of one sequence per chunk and head: groups of 4 positions that n_new tokens may
+// meet (uniform batches of f16 pools), else tokens
+template <int DT>
+__host__ __device__ __forceinline__ uint32_t append_v_units(uint32_t n_new, bool packed) {
+    return DT == VSPEC_KV_F16 && !packed ? (n_new + 2) / 4 + 1 : n_new;
+}
+
+// One chunk of the 4 tokens of a group (positions pos0 .. pos0 + 3, pos0 a multiple of 4;
+// token j's chunk at source element el0 + j * stride).
+template <int SRC>
+__device__ __forceinline__ void append_v_group(const AppendParams& p, uint32_t seq, uint32_t pos0, uint32_t h, uint32_t c,
+                                               size_t el0, size_t stride) {
+    const uint32_t lb = pos0 / p.block_tokens;
+    if (lb >= p.max_blocks) return;
+    uint32_t w[4][4];  // token, pair of elements
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const size_t el = el0 + j * stride;
+        if constexpr (SRC == VSPEC_KV_F16) {
+            const uint4 s = *reinterpret_cast<const uint4*>(p.v_new + el * 2);
+            w[j][0] = s.x; w[j][1] = s.y; w[j][2] = s.z; w[j][3] = s.w;
+        } else {
+            float x[8];
+            load_elements<SRC, 8>(p.v_new, el, x);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[j][e] = float_to_half_bits(x[2 * e]) | (float_to_half_bits(x[2 * e + 1]) << 16);
+        }
+    }
+    const int32_t phys = p.block_tables[(size_t)seq * p.max_blocks + lb];
+    if (phys < 0 || (uint32_t)phys >= p.num_blocks) return;
+    uint4* d = reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.v) +
+                                        f16_v_index((size_t)phys * p.hkv + h, p.block_tokens, p.head_dim,
+                                                    pos0 % p.block_tokens, 8 * c));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        // elements 2e and 2e + 1: tokens 0..3 of each
+        d[e] = make_uint4((w[0][e] & 0xffffu) | (w[1][e] << 16), (w[2][e] & 0xffffu) | (w[3][e] << 16),
+                          (w[0][e] >> 16) | (w[1][e] & 0xffff0000u), (w[2][e] >> 16) | (w[3][e] & 0xffff0000u));
+    }
+}
+
+// Item `it` of the K section: ((sequence, token), kv head, chunk).
+template <int DT, int SRC, bool ROPE>
+__device__ __forceinline__ void append_k_item(const AppendParams& p, uint32_t it) {
+    const uint32_t chunks = p.head_dim / 8;
+    const uint32_t c = it % chunks, r = it / chunks;
+    const uint32_t h = r % p.hkv, t = r / p.hkv;
+    const uint32_t b = t / p.n_new, i = t % p.n_new;
+    int32_t item, sp;
+    if (!append_where(p, b, item, sp)) return;
+    append_chunk<DT, SRC, ROPE>(p, (uint32_t)item, (uint32_t)sp + i, h, c, 0, ((size_t)t * p.hkv + h) * p.head_dim + 8 * c);
+}
+
+// Item `it` of the V section: ((sequence, group or token), kv head, chunk).
+template <int DT, int SRC, bool ROPE>
+__device__ __forceinline__ void append_v_item(const AppendParams& p, uint32_t it) {
+    const uint32_t chunks = p.head_dim / 8;
+    const uint32_t c = it % chunks, r = it / chunks;
+    const uint32_t h = r % p.hkv, u = r / p.hkv;
+    const size_t stride = (size_t)p.hkv * p.head_dim;
+    const size_t el_hc = (size_t)h * p.head_dim + 8 * c;
+    int32_t item, sp;
+    if constexpr (DT == VSPEC_KV_F16) {
+        if (!p.token_item) {
+            const uint32_t units = append_v_units<DT>(p.n_new, false);
+            const uint32_t b = u / units, g = u % units;
+            if (!append_where(p, b, item, sp)) return;
+            const uint32_t pos0 = ((uint32_t)sp & ~3u) + 4 * g;
+            const size_t el_b = (size_t)b * p.n_new * stride + el_hc;
+            // tokens of the launch in the group: lo .. hi - 1 of 0..3
+            const uint32_t lo = pos0 < (uint32_t)sp ? (uint32_t)sp - pos0 : 0u;
+            const uint32_t end = (uint32_t)sp + p.n_new;
+            const uint32_t hi = pos0 >= end ? 0u : (end - pos0 < 4u ? end - pos0 : 4u);
+            if (lo == 0 && hi == 4 && !(ROPE && p.rope_cos && pos0 + 3 >= p.max_pos)) {
+                append_v_group<SRC>(p, (uint32_t)item, pos0, h, c, el_b + (size_t)(pos0 - (uint32_t)sp) * stride, stride);
+                return;
+            }
+            for (uint32_t j = lo; j < hi; ++j) {
+                append_chunk<DT, SRC, ROPE>(p, (uint32_t)item, pos0 + j, h, c, 1, el_b + (size_t)(pos0 + j - (uint32_t)sp) * stride);
+            }
+            return;
+        }
+        if (!append_where(p, u, item, sp)) return;
+        // the packed tokens around u hold its group, in order: its first token's items
+        // write the group, the others nothing
+        const uint32_t r4 = (uint32_t)sp & 3u;
+        if (u >= r4 && u - r4 + 4 <= p.batch) {
+            const uint32_t u0 = u - r4;
+            bool whole = true;
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j)
+                whole = whole && p.token_item[u0 + j] == item && p.token_pos[u0 + j] == sp - (int32_t)r4 + (int32_t)j;
+            if (whole) {
+                if (r4 == 0) append_v_group<SRC>(p, (uint32_t)item, (uint32_t)sp, h, c, u * stride + el_hc, stride);
+                return;
+            }
+        }
+        append_chunk<DT, SRC, ROPE>(p, (uint32_t)item, (uint32_t)sp, h, c, 1, u * stride + el_hc);
+    } else {
+        const uint32_t b = u / p.n_new, i = u % p.n_new;
+        if (!append_where(p, b, item, sp)) return;
+        append_chunk<DT, SRC, ROPE>(p, (uint32_t)item, (uint32_t)sp + i, h, c, 1, u * stride + el_hc);
+    }
+}
+
+// Query section: an item is 4 elements of the first half of the rotated elements and their
+// partners, or 4 elements past them, of up to kRopeHeads heads of one token (the table
+// entries are read once for them all).  rope_dim / 2 a multiple of 4, rows and tables
+// 16-byte aligned.
+constexpr uint32_t kRopeHeads = 4;
+__host__ __device__ __forceinline__ uint32_t rope_q_chunks(uint32_t head_dim, uint32_t rope_dim) {
+    return rope_dim / 8 + (head_dim - rope_dim) / 4;
+}
+__device__ __forceinline__ void rope_q_item(const AppendParams& p, uint32_t it) {
+    const uint32_t chunks = rope_q_chunks(p.head_dim, p.rope_dim);
+    const uint32_t c = it % chunks, r = it / chunks;
+    const uint32_t hg = (p.hq + kRopeHeads - 1) / kRopeHeads;
+    const uint32_t h0 = (r % hg) * kRopeHeads, t = r / hg;
+    int32_t item, sp;
+    if (!append_where(p, t / p.n_new, item, sp)) return;
+    const uint32_t pos = (uint32_t)sp + t % p.n_new;
+    if (pos >= p.max_pos) return;
+    const uint32_t half = p.rope_dim / 2, d4 = p.head_dim / 4;
+    const uint32_t nh = p.hq - h0 < kRopeHeads ? p.hq - h0 : kRopeHeads;
+    const float4* in = reinterpret_cast<const float4*>(p.q_in) + ((size_t)t * p.hq + h0) * d4;
+    float4* out = reinterpret_cast<float4*>(p.q_out) + ((size_t)t * p.hq + h0) * d4;
+    if (c >= half / 4) {  // past the rotated elements
+        const uint32_t i = c + half / 4;
+        for (uint32_t h = 0; h < nh; ++h) out[h * d4 + i] = in[h * d4 + i];
+        return;
+    }
+    const float4 cv = reinterpret_cast<const float4*>(p.rope_cos + (size_t)pos * half)[c];
+    const float4 sv = reinterpret_cast<const float4*>(p.rope_sin + (size_t)pos * half)[c];
+    float4 x[kRopeHeads], y[kRopeHeads];
+#pragma unroll
+    for (uint32_t h = 0; h < kRopeHeads; ++h) {
+        const uint32_t hh = h < nh ? h : 0;  // loads stay unconditional
+        x[h] = in[hh * d4 + c];
+        y[h] = in[hh * d4 + c + half / 4];
+    }
+#pragma unroll
+    for (uint32_t h = 0; h < kRopeHeads; ++h) {
+#pragma clang fp contract(off)
+        if (h >= nh) break;
+        out[h * d4 + c] = make_float4(x[h].x * cv.x - y[h].x * sv.x, x[h].y * cv.y - y[h].y * sv.y,
+                                      x[h].z * cv.z - y[h].z * sv.z, x[h].w * cv.w - y[h].w * sv.w);
+        out[h * d4 + c + half / 4] = make_float4(x[h].x * sv.x + y[h].x * cv.x, x[h].y * sv.y + y[h].y * cv.y,
+                                                 x[h].z * sv.z + y[h].z * cv.z, x[h].w * sv.w + y[h].w * cv.w);
+    }
 }
 
 // Fused decode-step append of the MFMA decode kernels (p.k_new != null).  Every work

@@ -360,13 +360,42 @@ __global__ __launch_bounds__(D) void decode_combine(DecodeParams p) {
 // ---------------------------------------------------------------------------
 // One work item = EPT consecutive elements of one token-head row of K or V: a whole
 // 32-element quantisation group for int4 pools, 8 elements (16 or 32 bytes) otherwise.
-template <int DT, int SRC>
+template <int DT, int SRC, bool ROPE>
 __global__ __launch_bounds__(256) void kv_append(AppendParams p) {
     const uint64_t total = append_items<DT>(p);
     for (uint64_t it = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; it < total;
          it += (uint64_t)gridDim.x * blockDim.x) {
-        append_item<DT, SRC>(p, it);
+        append_item<DT, SRC, ROPE>(p, it);
     }
+}
+
+// f16 and f32 pools: the K, V and query sections of append_row.h, 256 items a workgroup.
+// Bound by memory: a 4096-token f16 chunk with rotary q and k (32/8 heads of 128) moves
+// 170 MB, in 36 us (4.7 TB/s, the rate of a large copy).  One item per lane keeps whole rows
+// coalesced (16 lanes a row), sections instead of K and V in alternate lanes keep a wave on
+// one path, V goes out in whole 4-token groups, and the rotary tables and partners are read
+// 16 bytes at a time, the tables once for 4 query heads.  Before (V in 2-byte pieces, tables
+// and partners element by element, q rotated one element a lane by a second launch): 114 us.
+template <int DT, int SRC, bool ROPE>
+__global__ __launch_bounds__(256) void kv_append_rows(AppendParams p, uint32_t k_wgs, uint32_t v_wgs, uint32_t k_items,
+                                                      uint32_t v_items, uint32_t q_items) {
+    const uint32_t wg = blockIdx.x;
+    if (wg < k_wgs) {
+        const uint32_t it = wg * 256 + threadIdx.x;
+        if (it < k_items) append_k_item<DT, SRC, ROPE>(p, it);
+    } else if (wg < k_wgs + v_wgs) {
+        const uint32_t it = (wg - k_wgs) * 256 + threadIdx.x;
+        if (it < v_items) append_v_item<DT, SRC, ROPE>(p, it);
+    } else {
+        const uint32_t it = (wg - k_wgs - v_wgs) * 256 + threadIdx.x;
+        if (it < q_items) rope_q_item(p, it);
+    }
+}
+
+// The query section alone (int4 pools, whose K and V items are whole quantisation groups).
+__global__ __launch_bounds__(256) void rope_q_rows(AppendParams p, uint32_t q_items) {
+    const uint32_t it = blockIdx.x * 256 + threadIdx.x;
+    if (it < q_items) rope_q_item(p, it);
 }
 
 // Rotary embedding of the query rows of the appended tokens: q [B][n_new][Hq][D] fp32,
@@ -1151,23 +1180,65 @@ static int append_launch(const char* who, const VspecPagedKV* kv, AppendParams& 
     p.head_dim = kv->head_dim;
     p.block_tokens = kv->block_tokens;
     p.num_blocks = kv->num_blocks;
-    const uint32_t ept = kv->dtype == VSPEC_KV_INT4 ? 32 : 8;
-    const uint64_t items = (uint64_t)p.batch * p.n_new * kv->num_kv_heads * (kv->head_dim / ept) * 2;
-    uint64_t blocks = (items + 255) / 256;
-    if (blocks > 65536) blocks = 65536;
-    const dim3 grid((unsigned)blocks);
+    p.rope_vec = p.rope_cos && ((uintptr_t)p.rope_cos | (uintptr_t)p.rope_sin) % 16 == 0;
     hipStream_t s = (hipStream_t)stream;
-#define VSPEC_APPEND(DT, SRC) hipLaunchKernelGGL((kv_append<DT, SRC>), grid, dim3(256), 0, s, p)
-    if (src_dtype == VSPEC_KV_F32) {
-        if (kv->dtype == VSPEC_KV_F32) VSPEC_APPEND(VSPEC_KV_F32, VSPEC_KV_F32);
-        else if (kv->dtype == VSPEC_KV_F16) VSPEC_APPEND(VSPEC_KV_F16, VSPEC_KV_F32);
-        else VSPEC_APPEND(VSPEC_KV_INT4, VSPEC_KV_F32);
+    const uint64_t tokens = (uint64_t)p.batch * p.n_new;
+    // query rows ride along when their halves and the tables split into 16-byte chunks
+    const bool q_vec = p.q_in && p.rope_vec && p.rope_dim % 8 == 0 && ((uintptr_t)p.q_in | (uintptr_t)p.q_out) % 16 == 0;
+    const uint64_t q_items =
+        q_vec ? tokens * ((p.hq + kRopeHeads - 1) / kRopeHeads) * rope_q_chunks(p.head_dim, p.rope_dim) : 0;
+    const uint64_t k_items = tokens * p.hkv * (p.head_dim / 8);
+    const uint64_t v_items = kv->dtype == VSPEC_KV_F16
+                                 ? (uint64_t)p.batch * append_v_units<VSPEC_KV_F16>(p.n_new, p.token_item != nullptr) *
+                                       p.hkv * (p.head_dim / 8)
+                                 : k_items;
+    // the row kernel counts its items in 32 bits
+    const bool rows = kv->dtype != VSPEC_KV_INT4 && k_items + v_items + q_items + 768 < 0xffffffffull;
+    const bool q_rows = q_items && (rows || q_items + 256 < 0xffffffffull);
+    if (rows) {
+        const uint32_t kw = (uint32_t)((k_items + 255) / 256), vw = (uint32_t)((v_items + 255) / 256);
+        const dim3 grid(kw + vw + (uint32_t)((q_items + 255) / 256));
+#define VSPEC_APPEND_(DT, SRC, ROPE)                                                                         \
+    hipLaunchKernelGGL((kv_append_rows<DT, SRC, ROPE>), grid, dim3(256), 0, s, p, kw, vw, (uint32_t)k_items, \
+                       (uint32_t)v_items, (uint32_t)q_items)
+#define VSPEC_APPEND(DT, SRC) \
+    if (p.rope_cos) VSPEC_APPEND_(DT, SRC, true); \
+    else VSPEC_APPEND_(DT, SRC, false)
+        if (src_dtype == VSPEC_KV_F32) {
+            if (kv->dtype == VSPEC_KV_F32) { VSPEC_APPEND(VSPEC_KV_F32, VSPEC_KV_F32); }
+            else { VSPEC_APPEND(VSPEC_KV_F16, VSPEC_KV_F32); }
+        } else {
+            if (kv->dtype == VSPEC_KV_F32) { VSPEC_APPEND(VSPEC_KV_F32, VSPEC_KV_F16); }
+            else { VSPEC_APPEND(VSPEC_KV_F16, VSPEC_KV_F16); }
+        }
+#undef VSPEC_APPEND_
     } else {
-        if (kv->dtype == VSPEC_KV_F32) VSPEC_APPEND(VSPEC_KV_F32, VSPEC_KV_F16);
-        else if (kv->dtype == VSPEC_KV_F16) VSPEC_APPEND(VSPEC_KV_F16, VSPEC_KV_F16);
-        else VSPEC_APPEND(VSPEC_KV_INT4, VSPEC_KV_F16);
-    }
+        const uint32_t ept = kv->dtype == VSPEC_KV_INT4 ? 32 : 8;
+        const uint64_t items = tokens * p.hkv * (p.head_dim / ept) * 2;
+        uint64_t blocks = (items + 255) / 256;
+        if (blocks > 65536) blocks = 65536;
+        const dim3 grid((unsigned)blocks);
+#define VSPEC_APPEND_(DT, SRC, ROPE) hipLaunchKernelGGL((kv_append<DT, SRC, ROPE>), grid, dim3(256), 0, s, p)
+        if (src_dtype == VSPEC_KV_F32) {
+            if (kv->dtype == VSPEC_KV_F32) { VSPEC_APPEND(VSPEC_KV_F32, VSPEC_KV_F32); }
+            else if (kv->dtype == VSPEC_KV_F16) { VSPEC_APPEND(VSPEC_KV_F16, VSPEC_KV_F32); }
+            else { VSPEC_APPEND(VSPEC_KV_INT4, VSPEC_KV_F32); }
+        } else {
+            if (kv->dtype == VSPEC_KV_F32) { VSPEC_APPEND(VSPEC_KV_F32, VSPEC_KV_F16); }
+            else if (kv->dtype == VSPEC_KV_F16) { VSPEC_APPEND(VSPEC_KV_F16, VSPEC_KV_F16); }
+            else { VSPEC_APPEND(VSPEC_KV_INT4, VSPEC_KV_F16); }
+        }
+        if (q_rows) hipLaunchKernelGGL(rope_q_rows, dim3((unsigned)((q_items + 255) / 256)), dim3(256), 0, s, p, (uint32_t)q_items);
 #undef VSPEC_APPEND
+#undef VSPEC_APPEND_
+    }
+    if (p.q_in && !q_rows) {
+        RopeQParams rq = {p.q_in, p.q_out, p.start_pos, p.rope_cos, p.rope_sin, p.batch, p.n_new, p.hq,
+                          p.head_dim, p.rope_dim, p.max_pos};
+        uint64_t blocks = (tokens * p.hq * p.head_dim + 255) / 256;
+        if (blocks > 65536) blocks = 65536;
+        hipLaunchKernelGGL(rope_q, dim3((unsigned)blocks), dim3(256), 0, s, rq);
+    }
     HIP_CHECK(hipGetLastError(), who);
     return 1;
 }
@@ -1231,17 +1302,10 @@ int vspec_rocm_kv_append_rope(const VspecPagedKV* kv, uint32_t batch, const int3
     p.rope_sin = rope_sin;
     p.rope_dim = rope_dim;
     p.max_pos = max_pos;
-    if (!append_launch("kv_append_rope launch", kv, p, src_dtype, stream)) return 0;
-    if (q_in) {
-        RopeQParams rq = {q_in, q_out, start_pos, rope_cos, rope_sin, batch, n_new, num_q_heads,
-                          kv->head_dim, rope_dim, max_pos};
-        const uint64_t total = (uint64_t)batch * n_new * num_q_heads * kv->head_dim;
-        uint64_t blocks = (total + 255) / 256;
-        if (blocks > 65536) blocks = 65536;
-        hipLaunchKernelGGL(rope_q, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, rq);
-        HIP_CHECK(hipGetLastError(), "rope_q launch");
-    }
-    return 1;
+    p.q_in = q_in;
+    p.q_out = q_out;
+    p.hq = num_q_heads;
+    return append_launch("kv_append_rope launch", kv, p, src_dtype, stream);
 }
 
 int vspec_rocm_kv_append_tokens(const VspecPagedKV* kv, uint32_t n_tokens, const int32_t* token_item,
