@@ -1,0 +1,71 @@
+"""GPU tests of single kernel paths at the sizes where they can go wrong (tile edges,
+remainders), against a general path of the library or a plain torch reference."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    import torch
+
+    if not torch.cuda.is_available():
+        pytest.fail("no GPU visible for a gpu-marked test")
+    return torch.device("cuda:0")
+
+
+@pytest.mark.parametrize("kind,D,H,P", [("f16", 8, 3, 16), ("f16", 24, 2, 48), ("f16", 64, 1, 16), ("f16", 128, 8, 32),
+                                        ("int4", 64, 3, 32), ("int4", 128, 2, 16), ("int4", 96, 2, 16)])
+@pytest.mark.parametrize("mode", ["raw", "f32"])
+def test_gather_units_equal_row_gather(gpu, kind, D, H, P, mode):
+    """kv_gather (units of 4 tokens) against kv_gather_rows (token by token): contexts off
+    multiples of 4, a bound below a context, an invalid block, gaps between the outputs of
+    the sequences that must stay as they were."""
+    import torch
+    import vspec_rocm as vr
+
+    dt = {"f16": vr.KV_F16, "int4": vr.KV_INT4}[kind]
+    lens, bound, gap = [1, 2, 3, 4, 5, 4 * P + 3, 130, 0], 101, 3
+    pool = vr.PagedPool(dt, 96, P, H, D, device=gpu)
+    g = torch.Generator(device=gpu).manual_seed(D + P)
+    nblk = -(-max(lens) // P)
+    tables = torch.randperm(96, generator=torch.Generator().manual_seed(1))[:len(lens) * nblk].view(len(lens), nblk).to(torch.int32)
+    x = [torch.randn((len(lens), nblk * P, H, D), generator=g, device=gpu) for _ in range(2)]
+    vr.kv_append(pool, tables, torch.zeros(len(lens), dtype=torch.int32), *x)
+    tables[6, 1] = -1  # tokens P .. 2P - 1 of sequence 6 are not read
+    ctx = torch.tensor(lens, dtype=torch.int32, device=gpu)
+    counts = [min(n, bound) for n in lens]
+    off = [sum(counts[:b]) + gap * (b + 1) for b in range(len(lens))]
+    total = sum(counts) + gap * (len(lens) + 1)
+    raw = mode == "raw"
+    out = {n: torch.full((total, H, D // 2 if raw and kind == "int4" else D), 7, device=gpu,
+                         dtype=pool.k.dtype if raw else torch.float32) for n in "kv"}
+    sc = {n: torch.full((total, H, max(D // 32, 1)), 7, device=gpu, dtype=torch.int16) for n in "kv"}
+    import ctypes as C
+
+    kv, tab = pool.desc(), tables.to(gpu)
+    offd = torch.tensor(off, dtype=torch.int64, device=gpu)
+    assert vr.lib().vspec_rocm_kv_gather(C.byref(kv), len(lens), tab.data_ptr(), nblk, ctx.data_ptr(), bound, offd.data_ptr(),
+                                         vr.GATHER_RAW if raw else vr.GATHER_F32, out["k"].data_ptr(), out["v"].data_ptr(),
+                                         sc["k"].data_ptr(), sc["v"].data_ptr(), torch.cuda.current_stream().cuda_stream), vr.last_error()
+    # the same tokens through the row-list gather
+    toks = [(b, t) for b, n in enumerate(counts) for t in range(n) if tables[b, t // P] >= 0]
+    where = torch.tensor([off[b] + t for b, t in toks], device=gpu)
+    pages = torch.tensor([int(tables[b, t // P]) for b, t in toks], dtype=torch.int32, device=gpu)
+    slots = torch.tensor([t % P for _, t in toks], dtype=torch.int32, device=gpu)
+    rows = {n: torch.empty((len(toks), H, D), device=gpu) for n in "kv"}
+    assert vr.lib().vspec_rocm_kv_gather_rows(C.byref(kv), len(toks), pages.data_ptr(), slots.data_ptr(), rows["k"].data_ptr(),
+                                              rows["v"].data_ptr(), torch.cuda.current_stream().cuda_stream)
+    for n in "kv":
+        got = out[n]
+        if raw and kind == "int4":
+            s = sc[n].view(torch.float16).float().repeat_interleave(32, -1)
+            c = got.to(torch.int32)
+            codes = torch.stack([((c & 15) ^ 8) - 8, ((c >> 4) ^ 8) - 8], -1).flatten(-2)
+            got = codes.float() * s
+        assert torch.equal(got[where].float(), rows[n])
+        keep = torch.ones(total, dtype=torch.bool, device=gpu)
+        keep[where] = False
+        assert bool((out[n][keep] == 7).all())
+        if raw and kind == "int4":
+            assert bool((sc[n][keep] == 7).all())

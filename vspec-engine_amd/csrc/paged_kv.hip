@@ -545,6 +545,165 @@ __global__ __launch_bounds__(256) void kv_gather(GatherParams p) {
     }
 }
 
+// 16 bytes that this launch does not read again
+__device__ __forceinline__ void store_stream4f(void* p, float a, float b, float c, float d) {
+    typedef float nt_f32x4 __attribute__((ext_vector_type(4)));
+    const nt_f32x4 v = {a, b, c, d};
+    __builtin_nontemporal_store(v, reinterpret_cast<nt_f32x4*>(p));
+}
+
+// f16 and int4 pools (int4: D = 64 or 128): K (blockIdx.z 0) or V (1) of 4 consecutive tokens
+// of one head per lane, the unit in which both pools hold V.  Bound by memory.  f16: a lane
+// takes E elements of each token, so that every store of a wave covers whole rows (f32 out: 4
+// elements, 16 bytes; raw: 8).  int4 V: lane n of 16 takes the tile chunk that holds d = n,
+// 16 + n, ... of the 4 tokens.  Against the row kernel, whose V elements are 2-byte (f16) or
+// byte (int4) loads: 8 sequences of 1k-8k tokens, 32/8 heads of 128: f16 to f32 174 -> 81 us
+// (5.7 TB/s; 85.5 with ordinary stores); 8 sequences of 0.5k-4k: f16 raw 66 -> 31, int4 raw
+// 37 -> 10.5, int4 to f32 69 -> 42 us; 24 short sequences (12-640 tokens) 7.6 us either way.
+template <int DT, int OUTF32, int D>
+__global__ __launch_bounds__(256) void kv_gather_quads(GatherParams p) {
+    const int b = blockIdx.y;
+    const uint32_t head_dim = D ? (uint32_t)D : p.head_dim;
+    const uint32_t tokens = min((uint32_t)max(p.ctx_lens[b], 0), p.max_ctx);
+    constexpr int E = OUTF32 ? 4 : 8;
+    const uint32_t lanes = DT == VSPEC_KV_F16 ? head_dim / E : 16u;  // lanes of a quad of one head
+    const uint32_t it = blockIdx.x * 256 + threadIdx.x;  // the host keeps this below 2^31
+    const uint32_t c = it % lanes, r = it / lanes;
+    const uint32_t h = r % p.hkv, quad = r / p.hkv;
+    // lanes that have nothing to copy stay for the wave's exchange through LDS below
+    bool on = quad < (tokens + 3) / 4;
+    const uint32_t t0 = on ? 4 * quad : 0u;
+    const uint32_t lb = t0 / p.block_tokens;
+    on = on && lb < p.max_blocks;
+    const int32_t phys = on ? p.block_tables[(size_t)b * p.max_blocks + lb] : -1;
+    on = on && phys >= 0 && (uint32_t)phys < p.num_blocks;
+    const uint32_t slot = t0 % p.block_tokens;
+    const size_t bh = (size_t)(on ? phys : 0) * p.hkv + h;
+    const size_t row = bh * p.block_tokens + slot;
+    const size_t orow = ((size_t)p.out_off[b] + t0) * p.hkv + h;  // token j: + j * hkv
+    const uint32_t n = on ? min(4u, tokens - t0) : 0u;
+    const bool v = blockIdx.z != 0;
+    if constexpr (DT == VSPEC_KV_F16) {
+        if (!on) return;
+        uint32_t w[4][E / 2];  // token, pair of elements
+        if (v) {
+            const uint16_t* src = reinterpret_cast<const uint16_t*>(p.v) + f16_v_index(bh, p.block_tokens, head_dim, slot, E * c);
+#pragma unroll
+            for (int e = 0; e < E / 2; ++e) {  // tokens 0..3 of elements 2e and 2e + 1
+                const uint4 x = load_stream4(src + 8 * e);
+                w[0][e] = (x.x & 0xffffu) | (x.z << 16);
+                w[1][e] = (x.x >> 16) | (x.z & 0xffff0000u);
+                w[2][e] = (x.y & 0xffffu) | (x.w << 16);
+                w[3][e] = (x.y >> 16) | (x.w & 0xffff0000u);
+            }
+        } else {
+            const uint16_t* src = reinterpret_cast<const uint16_t*>(p.k) + row * head_dim + E * c;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if constexpr (E == 4) {
+                    const uint2 x = load_stream2(src + (size_t)j * head_dim);
+                    w[j][0] = x.x; w[j][1] = x.y;
+                } else {
+                    const uint4 x = load_stream4(src + (size_t)j * head_dim);
+                    w[j][0] = x.x; w[j][1] = x.y; w[j][2] = x.z; w[j][3] = x.w;
+                }
+            }
+        }
+        uint8_t* dst = v ? p.ov : p.ok;
+        const size_t stride = (size_t)p.hkv * head_dim * (OUTF32 ? 4 : 2);
+        uint8_t* o = dst + orow * head_dim * (OUTF32 ? 4 : 2) + 16 * c;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (j >= (int)n) break;
+            if constexpr (OUTF32) {
+                store_stream4f(o + j * stride, half_bits_to_float(w[j][0] & 0xffffu), half_bits_to_float(w[j][0] >> 16),
+                               half_bits_to_float(w[j][1] & 0xffffu), half_bits_to_float(w[j][1] >> 16));
+            } else {
+                *reinterpret_cast<uint4*>(o + j * stride) = make_uint4(w[j][0], w[j][1], w[j][2], w[j][3]);
+            }
+        }
+    } else {
+        constexpr int G = D ? D / 32 : 1;  // groups of a row, dwords of a lane's chunk
+        if constexpr (OUTF32) {
+            if (!on) return;
+            if (v) {
+                // the 4 tokens' scales are one run; byte 2 * (j & 1) + (j >> 1) of dword q is
+                // token j's d = 32q + c (low nibble) and 32q + 16 + c (high)
+                uint32_t w[G];
+                const uint32_t* src = reinterpret_cast<const uint32_t*>(p.v + bh * ((size_t)p.block_tokens * D / 2) +
+                                                                        (size_t)(slot >> 4) * (8u * D)) + (4 * (slot & 15) + c) * G;
+#pragma unroll
+                for (int q = 0; q < G; ++q) w[q] = src[q];
+                float* o = reinterpret_cast<float*>(p.ov) + orow * D + c;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if (j >= (int)n) break;
+#pragma unroll
+                    for (int q = 0; q < G; ++q) {
+                        const float s = half_bits_to_float(p.vs[(row + j) * G + q]);
+                        const int byte = 2 * (j & 1) + (j >> 1);
+                        o[(size_t)j * p.hkv * D + 32 * q] = nibble(w[q], 2 * byte) * s;
+                        o[(size_t)j * p.hkv * D + 32 * q + 16] = nibble(w[q], 2 * byte + 1) * s;
+                    }
+                }
+            } else {
+                // lane c: elements 4c .. 4c + 3 (and 64 + 4c .. of a 128-element row)
+                const uint16_t* src = reinterpret_cast<const uint16_t*>(p.k + row * (D / 2));
+                float* o = reinterpret_cast<float*>(p.ok) + orow * D + 4 * c;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if (j >= (int)n) break;
+#pragma unroll
+                    for (int q = 0; q < D / 64; ++q) {
+                        const uint32_t w = src[(size_t)j * (D / 4) + 16 * q + c];
+                        const float s = half_bits_to_float(p.ks[int4_ks_index(bh, G, p.block_tokens, slot + j, 2 * q + c / 8)]);
+                        *reinterpret_cast<float4*>(o + (size_t)j * p.hkv * D + 64 * q) =
+                            make_float4(nibble(w, 0) * s, nibble(w, 1) * s, nibble(w, 2) * s, nibble(w, 3) * s);
+                    }
+                }
+            }
+        } else {
+            // canonical packed codes: lane c of a quad writes group c % G of token c / G (D = 64:
+            // lanes 8..15 idle), 16 bytes
+            const uint32_t j = c / G, q = c % G;
+            const bool mine = on && c < 4 * G && j < n;
+            uint4 out = make_uint4(0u, 0u, 0u, 0u);
+            if (v) {
+                // the quad's 16 chunks through LDS (a wave's own accesses, in program order),
+                // then the 16 bytes of (token, group): low nibbles d = 32q + i, high ones + 16
+                __shared__ uint32_t tile[256 / 16][16][G];
+                uint32_t(*mine_tile)[G] = tile[threadIdx.x / 16];
+                if (on) {
+                    const uint32_t* src = reinterpret_cast<const uint32_t*>(p.v + bh * ((size_t)p.block_tokens * D / 2) +
+                                                                            (size_t)(slot >> 4) * (8u * D)) + (4 * (slot & 15) + c) * G;
+#pragma unroll
+                    for (int i = 0; i < G; ++i) mine_tile[c][i] = src[i];
+                }
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                const uint32_t byte = 2 * (j & 1) + (j >> 1);
+                uint32_t lo[2] = {0u, 0u}, hi[2] = {0u, 0u};
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const uint32_t x = reinterpret_cast<const uint8_t*>(&mine_tile[i][q])[byte & 3];
+                    lo[i / 8] |= (x & 0xfu) << (4 * (i % 8));
+                    hi[i / 8] |= (x >> 4) << (4 * (i % 8));
+                }
+                out = make_uint4(lo[0], lo[1], hi[0], hi[1]);
+            } else if (mine) {
+                out = *reinterpret_cast<const uint4*>(p.k + (row + j) * (D / 2) + 16 * q);
+            }
+            if (mine) {
+                const size_t o = orow + (size_t)j * p.hkv;
+                *reinterpret_cast<uint4*>((v ? p.ov : p.ok) + o * (D / 2) + 16 * q) = out;
+                (v ? p.ovs : p.oks)[o * G + q] =
+                    v ? p.vs[(row + j) * G + q] : p.ks[int4_ks_index(bh, G, p.block_tokens, slot + j, q)];
+            }
+        }
+    }
+}
+
 struct GatherRowsParams {
     const uint8_t* k;
     const uint8_t* v;
@@ -1380,6 +1539,24 @@ int vspec_rocm_kv_gather(const VspecPagedKV* kv, uint32_t batch, const int32_t* 
     if (gx > 16384) gx = 16384;
     const dim3 grid((unsigned)gx, batch);
     hipStream_t s = (hipStream_t)stream;
+    // 4-token units (not the row kernel): f16 pools, and int4 ones of the usual head sizes
+    const bool i4 = kv->dtype == VSPEC_KV_INT4, f32_out = out_mode == VSPEC_GATHER_F32;
+    if (kv->dtype == VSPEC_KV_F16 || (i4 && (D == 64 || D == 128))) {
+        const uint64_t lanes = i4 ? 16 : D / (f32_out ? 4 : 8);
+        const uint64_t wgs = (((uint64_t)max_ctx_len + 3) / 4 * kv->num_kv_heads * lanes + 255) / 256;
+        if (wgs <= 0x7fffffffull / 256) {
+            const dim3 qgrid((unsigned)wgs, batch, 2);
+#define VSPEC_GATHER(DT, DIM)                                                                                  \
+    if (f32_out) hipLaunchKernelGGL((kv_gather_quads<DT, 1, DIM>), qgrid, dim3(256), 0, s, p); \
+    else hipLaunchKernelGGL((kv_gather_quads<DT, 0, DIM>), qgrid, dim3(256), 0, s, p)
+            if (!i4) { VSPEC_GATHER(VSPEC_KV_F16, 0); }
+            else if (D == 64) { VSPEC_GATHER(VSPEC_KV_INT4, 64); }
+            else { VSPEC_GATHER(VSPEC_KV_INT4, 128); }
+#undef VSPEC_GATHER
+            HIP_CHECK(hipGetLastError(), "kv_gather launch");
+            return 1;
+        }
+    }
 #define VSPEC_GATHER(DT, OF) hipLaunchKernelGGL((kv_gather<DT, OF>), grid, dim3(256), 0, s, p)
     if (out_mode == VSPEC_GATHER_F32) {
         if (kv->dtype == VSPEC_KV_F32) VSPEC_GATHER(VSPEC_KV_F32, 1);
