@@ -69,3 +69,26 @@ def test_gather_units_equal_row_gather(gpu, kind, D, H, P, mode):
         assert bool((out[n][keep] == 7).all())
         if raw and kind == "int4":
             assert bool((sc[n][keep] == 7).all())
+
+
+@pytest.mark.parametrize("B,H", [(1, 8), (5, 8), (40, 16)])
+def test_fused_step_many_short_items_d64(gpu, monkeypatch, B, H):
+    """f16 pools with 64-element heads, several short work items per workgroup (more than the
+    four whose new token is staged up front): the fused step leaves the bytes of kv_append."""
+    import torch
+    import vspec_rocm as vr
+
+    monkeypatch.setenv("VSPEC_ROCM_DECODE_ITEM_PARTS", "0")
+    D, P, T = 64, 16, 21
+    g = torch.Generator(device=gpu).manual_seed(B)
+    tables = torch.randperm(2 * B, generator=torch.Generator().manual_seed(B)).view(B, 2).to(torch.int32).to(gpu)
+    kv = [torch.randn((B, T, H, D), generator=g, device=gpu).half() for _ in range(2)]
+    new = [torch.randn((B, H, D), generator=g, device=gpu).half() for _ in range(2)]
+    q = torch.randn((B, H, D), generator=g, device=gpu)
+    pools = [vr.PagedPool(vr.KV_F16, 2 * B, P, H, D, device=gpu) for _ in range(2)]
+    zero = torch.zeros(B, dtype=torch.int32)
+    for pool in pools:
+        vr.kv_append(pool, tables, zero, *kv)
+    vr.kv_append(pools[0], tables, zero + T, *(x[:, None].contiguous() for x in new))
+    vr.paged_decode_step(pools[1], tables, torch.full((B,), T + 1, dtype=torch.int32), q, *new)
+    assert torch.equal(pools[0].k, pools[1].k) and torch.equal(pools[0].v, pools[1].v)

@@ -108,6 +108,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
     };
     auto newrow_load = [&](const ItemCursor& c) -> NewRow {
         NewRow r = {0u, 0u, make_float2(0.f, 0.f), make_float2(0.f, 0.f)};
+        if (D < 128 && lane >= D / 2) return r;  // (a row has D / 2 pairs)
         const size_t el = ((size_t)c.b * p.hkv + c.y / (int)p.gsplit) * D + 2 * lane;
         if (p.append_src == VSPEC_KV_F32) {
             r.kf = *reinterpret_cast<const float2*>(p.k_new + el * 4);
@@ -124,6 +125,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
             kw = float_to_half_bits(r.kf.x) | (float_to_half_bits(r.kf.y) << 16);
             vw = float_to_half_bits(r.vf.x) | (float_to_half_bits(r.vf.y) << 16);
         }
+        if (D < 128 && lane >= D / 2) return;
         newtok[row][0][lane] = kw;
         newtok[row][1][lane] = vw;
     };
