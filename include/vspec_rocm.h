@@ -147,8 +147,8 @@ typedef struct VspecPagedAttnDesc {
     const int32_t* block_used;
     /* Optional host lower bound of ctx_lens (0: none).  When it equals max_ctx_len (every
      * context the same) the host knows the work split exactly: it skips the merge launch
-     * if no work item spans two workgroups (e.g. 64 x 4097 tokens on 256 CUs), and f16
-     * batches whose work items about fill the CUs run one whole item per 8-wave workgroup.
+     * if no work item spans two workgroups (e.g. 64 x 4097 tokens on 256 CUs), and may cut
+     * long items into parts for workgroups of their own whatever their length.
      * A context below a non-zero bound is a caller error (its output may be left
      * unwritten). */
     uint32_t min_ctx_len;

@@ -92,3 +92,88 @@ def test_fused_step_many_short_items_d64(gpu, monkeypatch, B, H):
     vr.kv_append(pools[0], tables, zero + T, *(x[:, None].contiguous() for x in new))
     vr.paged_decode_step(pools[1], tables, torch.full((B,), T + 1, dtype=torch.int32), q, *new)
     assert torch.equal(pools[0].k, pools[1].k) and torch.equal(pools[0].v, pools[1].v)
+
+
+def _decode_setup(gpu, kind, lens, Hq, H, D, P, used=False, seed=0):
+    import torch
+    import vspec_rocm as vr
+
+    dt = {"f32": vr.KV_F32, "f16": vr.KV_F16, "int4": vr.KV_INT4}[kind]
+    nblk = max(1, -(-max(lens) // P))
+    g = torch.Generator(device=gpu).manual_seed(seed + D + P + sum(lens))
+    n = len(lens) * nblk
+    tables = torch.randperm(n + 3, generator=torch.Generator().manual_seed(seed))[:n].view(len(lens), nblk).to(torch.int32).to(gpu)
+    x = [torch.randn((len(lens), nblk * P, H, D), generator=g, device=gpu).half() for _ in range(2)]
+    pools = []
+    for _ in range(2):
+        pool = vr.PagedPool(dt, n + 3, P, H, D, device=gpu)
+        vr.kv_append(pool, tables, torch.zeros(len(lens), dtype=torch.int32), *x)
+        pools.append(pool)
+    q = torch.randn((len(lens), Hq, D), generator=g, device=gpu)
+    new = [torch.randn((len(lens), H, D), generator=g, device=gpu).half() for _ in range(2)]
+    ctx = torch.tensor(lens, dtype=torch.int32, device=gpu)
+    bu = None
+    if used:  # some middle blocks partly filled; the last entry's count ends the span
+        bu = torch.full((len(lens), nblk), P, dtype=torch.int32, device=gpu)
+        bu[:, ::3] = max(1, P - 5)
+        for b, t in enumerate(lens):
+            if t:
+                bu[b, (t - 1) // P] = (t - 1) % P + 1
+    return vr, pools, tables, ctx, q, new, bu
+
+
+def _same_pools(a, b):
+    import torch
+
+    return all(torch.equal(x.view(torch.uint8), y.view(torch.uint8)) for x, y in
+               ((a.k, b.k), (a.v, b.v), (a.ks, b.ks), (a.vs, b.vs), (a.kf, b.kf)) if x is not None)
+
+
+@pytest.mark.parametrize("kind", ["f16", "int4"])
+@pytest.mark.parametrize("lens,Hq,H,D,P,used", [
+    ([1], 8, 8, 64, 16, False), ([16, 17, 0, 1], 8, 2, 128, 16, False), ([64, 65, 80, 81, 3], 6, 2, 64, 48, False),
+    ([129], 24, 2, 128, 16, False), ([1000, 31, 515], 4, 2, 128, 32, True), ([300] * 5, 16, 4, 64, 16, True),
+    ([4100, 77], 8, 2, 128, 16, False)])
+def test_item_split_equals_balanced_split(gpu, monkeypatch, kind, lens, Hq, H, D, P, used):
+    """One work item's part per workgroup, for several part counts, against the balanced split:
+    the fused step's pool bytes are the same and the outputs differ only by rounding (f16: f32
+    sums of weights <= 1 against |v| < 6 in another order, below 16 * 2^-24 * 6; int4 also
+    rounds each weight x scale once to fp16 on either side, 2 * 2^-12 * 6)."""
+    import torch
+
+    vr, pools, tables, ctx, q, new, bu = _decode_setup(gpu, kind, lens, Hq, H, D, P, used)
+    tol = 2 * 6 * 2.0 ** -12 if kind == "int4" else 6e-6
+    for same in (False, True):
+        if same and len(set(lens)) > 1:
+            continue
+        hint = dict(max_ctx_len=max(lens), min_ctx_len=max(lens) if same else 0, block_used=bu)
+        for numerics in (vr.NUMERICS_PLAIN, vr.NUMERICS_3BIT):
+            monkeypatch.setenv("VSPEC_ROCM_DECODE_ITEM_PARTS", "0")
+            want = vr.paged_decode_step(pools[0], tables, ctx, q, *new, numerics=numerics, **hint)
+            plain = vr.paged_decode(pools[0], tables, ctx, q, numerics=numerics, **hint)
+            for parts in ("1", "2", "5", "64"):
+                monkeypatch.setenv("VSPEC_ROCM_DECODE_ITEM_PARTS", parts)
+                out = torch.full_like(q, float("nan"))
+                vr.paged_decode_step(pools[1], tables, ctx, q, *new, numerics=numerics, out=out, **hint)
+                assert _same_pools(*pools)
+                assert float((out - want).abs().max()) <= tol
+                out = vr.paged_decode(pools[1], tables, ctx, q, numerics=numerics, **hint)
+                assert float((out - plain).abs().max()) <= tol
+
+
+def test_item_split_keeps_the_workspace_plan(gpu, monkeypatch):
+    """The item split fits the workspace that the balanced split's plan asks for, at every size
+    below the one the caller sized its workspace for."""
+    import ctypes as C
+
+    vr, pools, tables, ctx, q, new, _ = _decode_setup(gpu, "f16", [2049] * 2, 8, 2, 128, 16)
+    import torch
+
+    out = torch.empty_like(q)
+    big = vr.make_decode_desc(pools[0], tables, ctx, q, out, 2049)
+    ws = torch.empty(vr.decode_workspace_bytes(big), dtype=torch.uint8, device=gpu)
+    for bound in list(range(1, 400, 13)) + [640, 1000, 1024, 1500, 2000, 2049]:
+        cl = torch.full((2,), bound, dtype=torch.int32, device=gpu)
+        d = vr.make_decode_desc(pools[0], tables, cl, q, out, bound, workspace=ws)
+        assert vr.lib().vspec_rocm_paged_decode_attention(C.byref(d)), vr.last_error()
+    torch.cuda.synchronize()

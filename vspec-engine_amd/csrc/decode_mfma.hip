@@ -51,14 +51,19 @@ struct Frags {
 // old one to an LDS merge slot, resets it and prepares the new item's q operands from
 // q rows staged in LDS up front.  The last of the waves to hand in an item's state
 // merges them all; no barrier stops the ring.
-template <int D, int GW, int PB, int NB, bool USED, int NW>
+// ITEMS: the workgroup takes one part of one work item instead (item_part), with nothing to
+// scan and one item's set-up: what bounds short and few contexts is the chain of dependent
+// round trips (context scan, q rows, table entries, tiles, merge), 17-34 us of kernel plus a
+// 5-7 us merge launch at 1 x 21 and 53 x 19 tokens against 7.4 and 8.2 us in all here.
+template <int D, int GW, int PB, int NB, bool USED, int NW, bool ITEMS>
 __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams p) {
     constexpr int NQK = D / 32;   // QK MFMAs per tile (each on 32 d)
     constexpr int NDT = D / 16;   // PV d-tiles
-    constexpr int kQStage = 4;    // item segments whose q rows are staged up front
-    constexpr int kSlots = 2;     // item segments being merged at once
-    __shared__ float qraw[kQStage][GW][D];
-    __shared__ float qs[NW][GW][D];  // per wave: q' of its current item
+    constexpr int kQStage = ITEMS ? 1 : 4;  // item segments whose q rows are staged up front
+    constexpr int kSlots = ITEMS ? 1 : 2;   // item segments being merged at once
+    __shared__ float qraw[ITEMS ? 1 : kQStage][ITEMS ? 1 : GW][ITEMS ? 1 : D];
+    __shared__ float qs[ITEMS ? 1 : NW][GW][D];  // per wave: q' of its current item (ITEMS: for all)
+    __shared__ int qexp[GW];                     // ITEMS: per head, the q' operand shift (qnorm_shift)
     // per wave: QK B operands (hi, lo for each 32-wide d chunk), read back every tile
     __shared__ float comb[kSlots][NW][GW][D + 2];
     __shared__ float patch_val[NW][kTile][4];
@@ -80,9 +85,16 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
     const int n = lane & 15;   // column / token within the tile
 
     const int ips = (int)(p.hkv * p.gsplit);  // work items per sequence
-    const WorkSplit ws = work_split<kSplitRagged, NW>(p, ips, split_sh);
+    WorkSplit ws = {};
+    ItemCursor first;
+    if constexpr (ITEMS) {
+        first = item_part(p, ws.lo, ws.hi);
+    } else {
+        ws = work_split<kSplitRagged, NW>(p, ips, split_sh);
+    }
     if (ws.lo >= ws.hi) return;
-    const ItemCursor first = cursor_at(p, ws);
+    if constexpr (!ITEMS) first = cursor_at(p, ws);
+    const int qrow_set = ITEMS ? 0 : wave;  // this wave's rows of qs
 
 
     // ---- q' = clip(q) * scale * log2(e) of work item c (segment s) for this wave, and
@@ -130,48 +142,29 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
         newtok[row][1][lane] = vw;
     };
 
-    auto qprep = [&](const int s, const ItemCursor& c) {
+    // q row x (the lane's elements of head h) into row h of the wave's qs; returns its shift
+    auto qhead = [&](const int h, const float (&x)[D / 64]) -> int {
         constexpr int E = D / 64;
-        if (s >= kQStage) {
-            // rows past the staged ones go through this wave's qs first, so that only this
-            // rare branch waits for a global load (the other path keeps the ring's loads
-            // in flight)
+        float sm = 0.f;
 #pragma unroll
-            for (int h = 0; h < GW; ++h) {
-                const float* qrow = p.q + ((size_t)c.b * p.hq + (size_t)c.y * GW + h) * D;
+        for (int e = 0; e < E; ++e) sm += x[e];
+        const float mean = wave_sum(sm) * (1.0f / D);
+        float v = 0.f;
 #pragma unroll
-                for (int e = 0; e < E; ++e) qs[wave][h][lane * E + e] = qrow[lane * E + e];
-            }
-            if (p.k_new) newrow_store(newrow_load(c), kQStage + wave);
+        for (int e = 0; e < E; ++e) v = fmaf(x[e] - mean, x[e] - mean, v);
+        v = wave_sum(v);
+        const float th = fminf(fmaxf(1e-6f, p.alpha * sqrtf(v * (1.0f / D))), p.input_clip);
+        float am = 0.f;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const float y = fminf(fmaxf(x[e], -th), th) * p.qscale;
+            qs[qrow_set][h][lane * E + e] = y;
+            am = fmaxf(am, fabsf(y));
         }
-        float (*src)[D] = s < kQStage ? qraw[s] : qs[wave];
-        int eh[GW];
-#pragma unroll
-        for (int h = 0; h < GW; ++h) {
-            float x[E];
-#pragma unroll
-            for (int e = 0; e < E; ++e) x[e] = src[h][lane * E + e];
-            float sm = 0.f;
-#pragma unroll
-            for (int e = 0; e < E; ++e) sm += x[e];
-            const float mean = wave_sum(sm) * (1.0f / D);
-            float v = 0.f;
-#pragma unroll
-            for (int e = 0; e < E; ++e) v = fmaf(x[e] - mean, x[e] - mean, v);
-            v = wave_sum(v);
-            const float th = fminf(fmaxf(1e-6f, p.alpha * sqrtf(v * (1.0f / D))), p.input_clip);
-            float am = 0.f;
-#pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const float y = fminf(fmaxf(x[e], -th), th) * p.qscale;
-                qs[wave][h][lane * E + e] = y;
-                am = fmaxf(am, fabsf(y));
-            }
-            eh[h] = __builtin_amdgcn_readfirstlane(qnorm_shift(wave_max(am)));
-        }
-        int en = 0;
-#pragma unroll
-        for (int h = 0; h < GW; ++h) en = n == h ? eh[h] : en;
+        return __builtin_amdgcn_readfirstlane(qnorm_shift(wave_max(am)));
+    };
+    // the lane's MFMA operands and score units from qs, en: the shift of head n
+    auto qoperands = [&](const int en) {
         qfac = pow2i(-en);
         qinv = pow2i(en);
         thr_raw = 8.0f * qinv;
@@ -187,7 +180,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
             h8_t hi8, lo8;
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                const float qv = qs[wave][hn][32 * i + 8 * g + j] * qin;
+                const float qv = qs[qrow_set][hn][32 * i + 8 * g + j] * qin;
                 const _Float16 hi = (_Float16)qv;
                 hi8[j] = hi;
                 lo8[j] = (_Float16)(qv - (float)hi);
@@ -195,6 +188,34 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
             qreg[i][0] = hi8;
             qreg[i][1] = lo8;
         }
+    };
+    auto qprep = [&](const int s, const ItemCursor& c) {
+        constexpr int E = D / 64;
+        if (s >= kQStage) {
+            // rows past the staged ones go through this wave's qs first, so that only this
+            // rare branch waits for a global load (the other path keeps the ring's loads
+            // in flight)
+#pragma unroll
+            for (int h = 0; h < GW; ++h) {
+                const float* qrow = p.q + ((size_t)c.b * p.hq + (size_t)c.y * GW + h) * D;
+#pragma unroll
+                for (int e = 0; e < E; ++e) qs[wave][h][lane * E + e] = qrow[lane * E + e];
+            }
+            if (p.k_new) newrow_store(newrow_load(c), kQStage + wave);
+        }
+        float (*src)[D] = s < kQStage ? reinterpret_cast<float (*)[D]>(qraw[s]) : qs[wave];
+        int eh[GW];
+#pragma unroll
+        for (int h = 0; h < GW; ++h) {
+            float x[E];
+#pragma unroll
+            for (int e = 0; e < E; ++e) x[e] = src[h][lane * E + e];
+            eh[h] = qhead(h, x);
+        }
+        int en = 0;
+#pragma unroll
+        for (int h = 0; h < GW; ++h) en = n == h ? eh[h] : en;
+        qoperands(en);
     };
 
     const int P = PB ? PB : (int)p.block_tokens;
@@ -209,15 +230,8 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
     // `lc` is the work item of the tiles being loaded (it runs NB tiles ahead).  Returns
     // how many of the tile's tokens its block holds (16, or block_used's cap; 0: none).
     ItemCursor lc = first;
-    auto load = [&](int t, Frags<D>& f) -> int {
-        t = __builtin_amdgcn_readfirstlane(t);
-        const bool in_range = t < ws.hi;
-        if (in_range) {
-            while (t >= lc.item0 + lc.U) cursor_next(p, ips, lc);
-        }
-        const int tile = in_range ? t - lc.item0 : 0;
-        const size_t row = (size_t)lc.b * p.max_blocks + tile / tiles_per_block;
-        const int entry = as_const(p.block_tables)[row];
+    auto load_entry = [&](const int t, const bool in_range, const int tile, const size_t row, const int entry,
+                          Frags<D>& f) -> int {
         const bool ok = in_range && entry >= 0 && (uint32_t)entry < p.num_blocks;
         const size_t tidx = (size_t)(ok ? entry : 0) * p.hkv + lc.y / (int)p.gsplit;
         const int slot0 = (tile % tiles_per_block) * kTile;
@@ -230,6 +244,16 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
         for (int j = 0; j < NDT; ++j) f.v[j] = load_stream2(vt + 64 * j);
         if constexpr (USED) return ok ? used_cap(as_const(p.block_used)[row], slot0) : 0;
         return ok ? kTile : 0;
+    };
+    auto load = [&](int t, Frags<D>& f) -> int {
+        t = __builtin_amdgcn_readfirstlane(t);
+        const bool in_range = t < ws.hi;
+        if (!ITEMS && in_range) {
+            while (t >= lc.item0 + lc.U) cursor_next(p, ips, lc);
+        }
+        const int tile = in_range ? t - lc.item0 : 0;
+        const size_t row = (size_t)lc.b * p.max_blocks + tile / tiles_per_block;
+        return load_entry(t, in_range, tile, row, as_const(p.block_tables)[row], f);
     };
 
     f4_t acc[NDT];
@@ -318,7 +342,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     const float x = half_bits_to_float((w4[e / 2] >> (16 * (e % 2))) & 0xffffu);
-                    a = fmaf(qs[wave][h][32 * i + 8 * g + e], fminf(fmaxf(x, -th), th), a);
+                    a = fmaf(qs[qrow_set][h][32 * i + 8 * g + e], fminf(fmaxf(x, -th), th), a);
                 }
             }
             part[h] = add_rows(a);
@@ -528,6 +552,78 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
     const int nt = wave < len ? (len - wave + NW - 1) / NW : 0;
     Frags<D> f[NB];
     int ok[NB];
+    if constexpr (ITEMS) {
+        // One work item's part (item_part): its q rows and new token are read by different
+        // waves, each wave's first tiles are on their way while head w is prepared by wave w,
+        // one barrier publishes them, and all waves merge after another.
+        static_assert(GW <= NW, "one wave per head");
+        constexpr int E = D / 64;
+        float x[E];
+        if (wave < GW) {
+            const float* qrow = p.q + ((size_t)pc.b * p.hq + (size_t)pc.y * GW + wave) * D;
+#pragma unroll
+            for (int e = 0; e < E; ++e) x[e] = qrow[lane * E + e];
+        }
+        // the first tiles' table entries and the context in one scalar round trip
+        int entry[NB];
+        size_t erow[NB];
+#pragma unroll
+        for (int u = 0; u < NB; ++u) {
+            erow[u] = (size_t)pc.b * p.max_blocks + min(t0 + u * NW, ws.hi - 1) / tiles_per_block;
+            entry[u] = as_const(p.block_tables)[erow[u]];
+        }
+        const int tnew = papp >= 0 ? min(papp / kTile, pc.U - 1) : -1;  // the tile whose wave stores the token
+        const bool stage = tnew >= ws.lo && tnew < ws.hi && wave == NW - 1;
+        NewRow row;
+        if (stage) row = newrow_load(pc);
+#pragma unroll
+        for (int u = 0; u < NB; ++u) {
+            if (u < nt) ok[u] = load_entry(t0 + u * NW, true, t0 + u * NW, erow[u], entry[u], f[u]);
+        }
+        if (wave < GW) {
+            const int e = qhead(wave, x);
+            if (lane == 0) qexp[wave] = e;
+        }
+        if (stage) newrow_store(row, 0);
+        __syncthreads();
+        reset();
+        qoperands(n < GW ? qexp[n < GW ? n : 0] : 0);
+        auto step = [&](const int u, const int t) {
+            if (t == tnew) {
+                if (t == papp / kTile) patch_new(f[u], 0, papp % kTile);
+                store_new(pc, 0, papp);
+            }
+            process(f[u], ok[u], t, pctx);
+        };
+        int k = 0;
+        for (; k + NB < nt; k += NB) {
+#pragma unroll
+            for (int u = 0; u < NB; ++u) {
+                const int t = t0 + (k + u) * NW;
+                step(u, t);
+                ok[u] = load(t + NB * NW, f[u]);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < NB; ++u) {
+            if (k + u < nt) step(u, t0 + (k + u) * NW);
+        }
+        const float l = add_rows(l_run);
+        if (n < GW) {
+#pragma unroll
+            for (int j = 0; j < NDT; ++j) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) comb[0][wave][n][2 + 16 * j + 4 * g + r] = acc[j][r];
+            }
+            if (g == 0) {
+                comb[0][wave][n][0] = mf;
+                comb[0][wave][n][1] = l;
+            }
+        }
+        __syncthreads();
+        finish_item<D, GW, NW>(p, comb[0], pc, ws.hi - ws.lo == pc.U);
+        return;
+    }
     // Set-up.  Wave 0 loads the q rows of the range's first kQStage segments (rows GW*y ..
     // GW*y + GW - 1 of sequence b are contiguous; merge slot s serves segment s first) and,
     // for a fused decode step, their new token rows, waits for these loads only, stages
@@ -572,7 +668,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
 #pragma unroll
                 for (int j = 0; j < QPL; ++j) {
                     const int i = lane + 64 * j;
-                    if (i < GW * D) qraw[s][i / D][i % D] = qreg[s][j];
+                    if (i < GW * D) (&qraw[0][0][0])[s * GW * D + i] = qreg[s][j];
                 }
                 if (p.k_new) newrow_store(nrow[s], s);
             }
@@ -625,29 +721,29 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
 #define VSPEC_F16_TILES_IN_FLIGHT 2
 #endif
 
-template <int D, int GW, bool USED>
-void launch_used(const DecodeParams& p, dim3 grid, hipStream_t s) {
+template <int D, int GW, bool USED, int PB>
+void launch_pb(const DecodeParams& p, dim3 grid, hipStream_t s) {
     constexpr int NB = VSPEC_F16_TILES_IN_FLIGHT;
-    if (p.wide) {
-        // one work item per workgroup of 8 waves (no item spans two workgroups)
-        if (p.block_tokens == 16) {
-            hipLaunchKernelGGL((decode_mfma_f16<D, GW, 16, NB, USED, 8>), grid, dim3(512), 0, s, p);
-        } else {
-            hipLaunchKernelGGL((decode_mfma_f16<D, GW, 0, NB, USED, 8>), grid, dim3(512), 0, s, p);
-        }
-    } else if (p.block_tokens == 16) {
-        hipLaunchKernelGGL((decode_mfma_f16<D, GW, 16, NB, USED, kWaves>), grid, dim3(256), 0, s, p);
+    if (p.item_parts) {
+        hipLaunchKernelGGL((decode_mfma_f16<D, GW, PB, NB, USED, kWaves, true>), grid, dim3(kWaves * 64), 0, s, p);
     } else {
-        hipLaunchKernelGGL((decode_mfma_f16<D, GW, 0, NB, USED, kWaves>), grid, dim3(256), 0, s, p);
+        hipLaunchKernelGGL((decode_mfma_f16<D, GW, PB, NB, USED, kWaves, false>), grid, dim3(kWaves * 64), 0, s, p);
     }
 }
 
 template <int D, int GW>
 void launch(const DecodeParams& p, dim3 grid, hipStream_t s) {
-    if (p.block_used) launch_used<D, GW, true>(p, grid, s);
-    else launch_used<D, GW, false>(p, grid, s);
-    // items split over several workgroups (same split: the f16 kernel's pair shares)
-    if (p.merge) {
+    if (p.block_used) {
+        if (p.block_tokens == 16) launch_pb<D, GW, true, 16>(p, grid, s);
+        else launch_pb<D, GW, true, 0>(p, grid, s);
+    } else {
+        if (p.block_tokens == 16) launch_pb<D, GW, false, 16>(p, grid, s);
+        else launch_pb<D, GW, false, 0>(p, grid, s);
+    }
+    if (p.item_parts > 1) {
+        hipLaunchKernelGGL((decode_merge_items<D, GW>), dim3(p.hkv * p.gsplit, p.batch), dim3(256), 0, s, p);
+    } else if (!p.item_parts && p.merge) {
+        // items split over several workgroups (same split: the f16 kernel's pair shares)
         const dim3 merge_grid(p.batch * p.hkv * p.gsplit);
         hipLaunchKernelGGL((decode_merge_split<D, GW, kSplitRagged>), merge_grid, dim3(kWaves * 64), 0, s, p);
     }
@@ -666,11 +762,15 @@ int launch_gw(uint32_t gw, const DecodeParams& p, dim3 grid, hipStream_t s) {
 
 }  // namespace
 
-int launch_decode_mfma_f16(const DecodeParams& p, uint32_t head_dim, uint32_t gw, dim3 grid,
-                           hipStream_t stream) {
-    if (head_dim == 64) return launch_gw<64>(gw, p, grid, stream);
-    if (head_dim == 128) return launch_gw<128>(gw, p, grid, stream);
-    return 0;
+// one head size per object file (VSPEC_HEAD_DIM), so that they build side by side
+#if VSPEC_HEAD_DIM == 64
+int launch_decode_mfma_f16_d64(const DecodeParams& p, uint32_t gw, dim3 grid, hipStream_t stream) {
+    return launch_gw<64>(gw, p, grid, stream);
 }
+#else
+int launch_decode_mfma_f16_d128(const DecodeParams& p, uint32_t gw, dim3 grid, hipStream_t stream) {
+    return launch_gw<128>(gw, p, grid, stream);
+}
+#endif
 
 }  // namespace vkv

@@ -163,8 +163,9 @@ struct I4NewToken {
 // ST: tile pairs in flight per wave (LDS stages); FL: the tile loop takes the pool's clamp
 // flags (and screens only what they cannot say); without FL it screens every tile, a
 // lighter loop for short per-workgroup shares.  USED: per-block used counts cap each tile
-// (block_used).
-template <int D, int GW, int PB, int ST, bool FL, bool USED>
+// (block_used); ITEMS: one part of one work item per workgroup (item_part), else a range of
+// the work split.
+template <int D, int GW, int PB, int ST, bool FL, bool USED, bool ITEMS>
 __global__ __launch_bounds__(256, VSPEC_I4_MIN_WG_PER_CU) void decode_mfma_i4(DecodeParams p) {
     constexpr int NQ = D / 32;   // code dwords per lane = QK MFMAs per tile = groups
     constexpr int NG = D / 32;
@@ -188,7 +189,15 @@ __global__ __launch_bounds__(256, VSPEC_I4_MIN_WG_PER_CU) void decode_mfma_i4(De
     const int n = lane & 15;
 
     const int ips = (int)(p.hkv * p.gsplit);  // work items per sequence
-    const WorkSplit ws = work_split<kSplitAlways>(p, ips, split_sh);
+    WorkSplit ws = {};
+    ItemCursor c0 = {0, 0, 1, 0, 0};
+    if constexpr (ITEMS) {
+        c0 = item_part(p, ws.lo, ws.hi);
+        ws.b = c0.b;
+        if (ws.lo >= ws.hi) return;
+    } else {
+        ws = work_split<kSplitAlways>(p, ips, split_sh);
+    }
     // q rows of a work item (wave w < GW: head w), loaded ahead of the item's set-up
     constexpr int E = D / 64;
     float q_rows[E];
@@ -200,9 +209,8 @@ __global__ __launch_bounds__(256, VSPEC_I4_MIN_WG_PER_CU) void decode_mfma_i4(De
             for (int e = 0; e < E; ++e) q_rows[e] = qrow[lane * E + e];
         }
     };
-    ItemCursor c0 = {0, 0, 1, 0, 0};
     if (ws.lo < ws.hi) {
-        c0 = cursor_at(p, ws);
+        if constexpr (!ITEMS) c0 = cursor_at(p, ws);
         load_q(c0.b, c0.y);
     }
     const bool appending = p.k_new != nullptr && ws.lo < ws.hi;
@@ -302,7 +310,9 @@ __global__ __launch_bounds__(256, VSPEC_I4_MIN_WG_PER_CU) void decode_mfma_i4(De
         }
         return r;
     };
-    if (appending && wave == 0 && nt_in && lane < kNtLanes) {
+    // (ITEMS: every lane, lanes past kNtLanes repeat the V row's; without the lane test the
+    // compiler keeps the block-table reads below on the scalar unit)
+    if (appending && wave == 0 && nt_in && (ITEMS || lane < kNtLanes)) {
         float x[4];
         load_token(c0.b, (uint32_t)c0.y / p.gsplit, x);
         // a vector load (the barriers wait for scalar ones), used after the tile loop
@@ -323,7 +333,7 @@ __global__ __launch_bounds__(256, VSPEC_I4_MIN_WG_PER_CU) void decode_mfma_i4(De
     // The range's further appended items (short ones), the j-th of them by wave j % kWaves,
     // are written to the pool at once (the same bytes as the append kernel's), and their
     // tiles are read after the first barrier: these waves wait for their stores.
-    if (appending) {
+    if (!ITEMS && appending) {
         const uint32_t P0 = PB ? (uint32_t)PB : p.block_tokens;
         ItemCursor c = c0;
         bool direct = false;
@@ -367,17 +377,17 @@ __global__ __launch_bounds__(256, VSPEC_I4_MIN_WG_PER_CU) void decode_mfma_i4(De
     int b = ws.b;
     int seq0 = ws.seq0;
     for (int pos = ws.lo; pos < ws.hi;) {
-        const int U = item_tiles(p, b);
-        if (pos >= seq0 + U * ips) {
+        const int U = ITEMS ? c0.U : item_tiles(p, b);
+        if (!ITEMS && pos >= seq0 + U * ips) {
             seq0 += U * ips;
             ++b;
             continue;
         }
-        const int y = (pos - seq0) / U;
-        const int item0 = seq0 + y * U;
+        const int y = ITEMS ? c0.y : (pos - seq0) / U;
+        const int item0 = ITEMS ? 0 : seq0 + y * U;
         const int tile_begin = pos - item0;
         const int tile_end = min(ws.hi, item0 + U) - item0;
-        const int hk = y / (int)p.gsplit;
+        const int hk = ITEMS ? __builtin_amdgcn_readfirstlane(y / (int)p.gsplit) : y / (int)p.gsplit;
         const int hq0 = hk * ((int)p.gsplit * GW) + (y % (int)p.gsplit) * GW;
         const int ctx = min(max(as_const(p.ctx_lens)[b], 0), (int)(p.max_blocks * p.block_tokens));
 
@@ -501,6 +511,13 @@ __global__ __launch_bounds__(256, VSPEC_I4_MIN_WG_PER_CU) void decode_mfma_i4(De
 
         const int step = 2 * kWaves;
         const int t0 = tile_begin + 2 * wave;
+        // the ring's first table reads go out together (ITEMS: before the q rows are waited
+        // for, so that the two round trips overlap)
+        Look first_look[ST];
+        if constexpr (ITEMS) {
+#pragma unroll
+            for (int u = 0; u < ST; ++u) first_look[u] = lookup(t0 + u * step);
+        }
 
         // ---- q' = clip(q) * scale * log2(e): wave w prepares head w ----
         if (wave < GW) {
@@ -530,10 +547,10 @@ __global__ __launch_bounds__(256, VSPEC_I4_MIN_WG_PER_CU) void decode_mfma_i4(De
         }
         // The first ST pairs are on their way while the q operands are prepared (after the
         // q rows are in registers: a wait for those would also wait for these).
-        // the ring's first table reads go out together
-        Look first_look[ST];
+        if constexpr (!ITEMS) {
 #pragma unroll
-        for (int u = 0; u < ST; ++u) first_look[u] = lookup(t0 + u * step);
+            for (int u = 0; u < ST; ++u) first_look[u] = lookup(t0 + u * step);
+        }
 #pragma unroll
         for (int u = 0; u < ST; ++u) issue(t0 + u * step, u, first_look[u]);
         Look next = lookup(t0 + ST * step);
@@ -974,6 +991,10 @@ __global__ __launch_bounds__(256, VSPEC_I4_MIN_WG_PER_CU) void decode_mfma_i4(De
             comb[wave][n][1] = l_run;
         }
         __syncthreads();
+        if constexpr (ITEMS) {
+            finish_item<D, GW, kWaves>(p, comb, c0, tile_end - tile_begin == U);
+            return;
+        }
         finish_segment<D, GW>(p, comb, b, hq0, U, tile_begin, tile_end, pos == ws.lo ? 0 : 1);
         __syncthreads();  // the wave states are read before the next item's loads refill the ring
         pos = item0 + tile_end;
@@ -984,28 +1005,32 @@ __global__ __launch_bounds__(256, VSPEC_I4_MIN_WG_PER_CU) void decode_mfma_i4(De
 #define VSPEC_I4_STAGES 2
 #endif
 
-template <int D, int GW, bool USED>
-void launch_used(const DecodeParams& p, dim3 grid, hipStream_t s) {
+template <int D, int GW, int PB, bool FL, bool USED>
+void launch_fl(const DecodeParams& p, dim3 grid, hipStream_t s) {
     constexpr int ST = VSPEC_I4_STAGES;
-    if (p.read_flags) {
-        if (p.block_tokens == 16)
-            hipLaunchKernelGGL((decode_mfma_i4<D, GW, 16, ST, true, USED>), grid, dim3(256), 0, s, p);
-        else
-            hipLaunchKernelGGL((decode_mfma_i4<D, GW, 0, ST, true, USED>), grid, dim3(256), 0, s, p);
+    if (p.item_parts) hipLaunchKernelGGL((decode_mfma_i4<D, GW, PB, ST, FL, USED, true>), grid, dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((decode_mfma_i4<D, GW, PB, ST, FL, USED, false>), grid, dim3(256), 0, s, p);
+}
+
+template <int D, int GW, int PB>
+void launch_pb(const DecodeParams& p, dim3 grid, hipStream_t s) {
+    if (p.block_used) {
+        if (p.read_flags) launch_fl<D, GW, PB, true, true>(p, grid, s);
+        else launch_fl<D, GW, PB, false, true>(p, grid, s);
     } else {
-        if (p.block_tokens == 16)
-            hipLaunchKernelGGL((decode_mfma_i4<D, GW, 16, ST, false, USED>), grid, dim3(256), 0, s, p);
-        else
-            hipLaunchKernelGGL((decode_mfma_i4<D, GW, 0, ST, false, USED>), grid, dim3(256), 0, s, p);
+        if (p.read_flags) launch_fl<D, GW, PB, true, false>(p, grid, s);
+        else launch_fl<D, GW, PB, false, false>(p, grid, s);
     }
 }
 
 template <int D, int GW>
 void launch(const DecodeParams& p, dim3 grid, hipStream_t s) {
-    if (p.block_used) launch_used<D, GW, true>(p, grid, s);
-    else launch_used<D, GW, false>(p, grid, s);
-    // items split over several workgroups (same split: equal shares)
-    if (p.merge) {
+    if (p.block_tokens == 16) launch_pb<D, GW, 16>(p, grid, s);
+    else launch_pb<D, GW, 0>(p, grid, s);
+    if (p.item_parts > 1) {
+        hipLaunchKernelGGL((decode_merge_items<D, GW>), dim3(p.hkv * p.gsplit, p.batch), dim3(256), 0, s, p);
+    } else if (!p.item_parts && p.merge) {
+        // items split over several workgroups (same split: equal shares)
         const dim3 merge_grid(p.batch * p.hkv * p.gsplit);
         hipLaunchKernelGGL((decode_merge_split<D, GW, kSplitAlways>), merge_grid, dim3(kWaves * 64), 0, s, p);
     }
@@ -1024,11 +1049,15 @@ int launch_gw(uint32_t gw, const DecodeParams& p, dim3 grid, hipStream_t s) {
 
 }  // namespace
 
-int launch_decode_mfma_int4(const DecodeParams& p, uint32_t head_dim, uint32_t gw, dim3 grid,
-                            hipStream_t stream) {
-    if (head_dim == 64) return launch_gw<64>(gw, p, grid, stream);
-    if (head_dim == 128) return launch_gw<128>(gw, p, grid, stream);
-    return 0;
+// one head size per object file (VSPEC_HEAD_DIM), so that they build side by side
+#if VSPEC_HEAD_DIM == 64
+int launch_decode_mfma_int4_d64(const DecodeParams& p, uint32_t gw, dim3 grid, hipStream_t stream) {
+    return launch_gw<64>(gw, p, grid, stream);
 }
+#else
+int launch_decode_mfma_int4_d128(const DecodeParams& p, uint32_t gw, dim3 grid, hipStream_t stream) {
+    return launch_gw<128>(gw, p, grid, stream);
+}
+#endif
 
 }  // namespace vkv

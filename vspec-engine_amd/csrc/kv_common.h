@@ -266,21 +266,20 @@ struct DecodeParams {
     // tiles per work item when the host knows every context to be the same (min_ctx_len ==
     // max_ctx_len), else 0: the split then needs no pass over ctx_lens
     uint32_t uniform_tiles;
-    // f16 pools: workgroups of 8 waves, each taking whole work items (chunk_tiles is a
-    // multiple of the uniform tiles per item), for batches with few, short items
-    bool wide;
     // balanced split of a ragged batch: each work item also costs this many tiles (its
     // set-up and merge in every workgroup that starts it), 0: tiles only
     uint32_t seg_cost;
+    // item split: parts of a work item (grid (hkv * gsplit * item_parts, batch)), 0: the ranges above
+    uint32_t item_parts;
 };
 
 // Launch the MFMA decode kernels for f16 pools (decode_mfma.hip) and int4 pools
-// (decode_mfma_int4.hip), each followed by its merge launch (decode_merge_split); they
-// return 0 when no instantiation matches (head_dim, heads per work item).
-int launch_decode_mfma_f16(const DecodeParams& p, uint32_t head_dim, uint32_t gw, dim3 grid,
-                           hipStream_t stream);
-int launch_decode_mfma_int4(const DecodeParams& p, uint32_t head_dim, uint32_t gw, dim3 grid,
-                            hipStream_t stream);
+// (decode_mfma_int4.hip) of head_dim 64 or 128, each followed by its merge launch; they
+// return 0 when no instantiation matches (heads per work item).
+int launch_decode_mfma_f16_d64(const DecodeParams& p, uint32_t gw, dim3 grid, hipStream_t stream);
+int launch_decode_mfma_f16_d128(const DecodeParams& p, uint32_t gw, dim3 grid, hipStream_t stream);
+int launch_decode_mfma_int4_d64(const DecodeParams& p, uint32_t gw, dim3 grid, hipStream_t stream);
+int launch_decode_mfma_int4_d128(const DecodeParams& p, uint32_t gw, dim3 grid, hipStream_t stream);
 
 // Merge the kWaves per-wave softmax states of a workgroup (comb[w][h] = {max, sum,
 // acc[D]}) and write the output row (one partition) or the split-K partial.
@@ -758,6 +757,130 @@ __device__ __forceinline__ void finish_segment(const DecodeParams& p, const floa
             }
         }
     }
+}
+
+// ---------------------------------------------------------------------------
+// Item split (DecodeParams.item_parts): workgroup (y * parts + part, b) takes part `part` of
+// work item y of sequence b.  An item of U tiles is cut into n = min(parts, ceil(U / 4)) parts
+// (a part has work for the 4 waves), of tiles [part * U / n, (part + 1) * U / n).  No pass over ctx_lens, no workgroup with two
+// items; an item in one part goes straight to the output, and the partial states of the
+// others lie at item * parts + part, where decode_merge_items finds them without redoing a
+// split.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ int item_parts_of(const DecodeParams& p, int U) { return min((int)p.item_parts, (U + 3) / 4); }
+
+// this workgroup's item (tile positions count from the item's first tile) and tiles [lo, hi);
+// lo = hi when it has none
+__device__ __forceinline__ ItemCursor item_part(const DecodeParams& p, int& lo, int& hi) {
+    ItemCursor c;
+    c.b = (int)blockIdx.y;
+    c.seq0 = 0;
+    c.item0 = 0;
+    c.U = item_tiles(p, c.b);
+    int part = 0;
+    c.y = (int)blockIdx.x;
+    if (p.item_parts > 1) {
+        c.y = (int)((uint32_t)blockIdx.x / p.item_parts);
+        part = (int)blockIdx.x - c.y * (int)p.item_parts;
+    }
+    const int n = item_parts_of(p, c.U);
+    const int l = part < n ? (int)((uint32_t)part * (uint32_t)c.U / (uint32_t)n) : 0;
+    const int h = part < n ? (int)((uint32_t)(part + 1) * (uint32_t)c.U / (uint32_t)n) : 0;
+    // wave-uniform values on the scalar unit (the divisions run on the vector one)
+    c.y = __builtin_amdgcn_readfirstlane(c.y);
+    c.U = __builtin_amdgcn_readfirstlane(c.U);
+    lo = __builtin_amdgcn_readfirstlane(l);
+    hi = __builtin_amdgcn_readfirstlane(h);
+    return c;
+}
+
+// Block-wide: merge the NW wave states of an item part and write the output rows (whole) or
+// the part's partial state.
+template <int D, int GW, int NW>
+__device__ __forceinline__ void finish_item(const DecodeParams& p, const float (*st)[GW][D + 2], const ItemCursor& c,
+                                            bool whole) {
+    const size_t slot = (size_t)c.b * gridDim.x + blockIdx.x;
+    const size_t row0 = (size_t)c.b * p.hq + (size_t)c.y * GW;
+    for (int idx = (int)threadIdx.x; idx < GW * D; idx += NW * 64) {
+        const int h = idx / D;
+        const int d = idx % D;
+        float M = -INFINITY;
+#pragma unroll
+        for (int v = 0; v < NW; ++v) M = fmaxf(M, st[v][h][0]);
+        float a = 0.f, l = 0.f;
+#pragma unroll
+        for (int v = 0; v < NW; ++v) {
+            const float f = exp2f(st[v][h][0] - M);
+            a = fmaf(st[v][h][2 + d], f, a);
+            l = fmaf(st[v][h][1], f, l);
+        }
+        if (whole) {
+            p.out[(row0 + h) * D + d] = l > 0.f ? a / l : 0.f;
+        } else {
+            p.part_acc[slot * (GW * D) + idx] = a;
+            if (d == 0) {
+                p.part_ml[(slot * GW + h) * 2] = M;
+                p.part_ml[(slot * GW + h) * 2 + 1] = l;
+            }
+        }
+    }
+}
+
+// Merge launch of an item split, one workgroup per work item (grid = (hkv * gsplit, batch)):
+// a lane takes 4 outputs of one head and every PS-th part; the PS sets meet in LDS.
+template <int D, int GW>
+__global__ __launch_bounds__(256) void decode_merge_items(DecodeParams p) {
+    constexpr int Q = GW * D / 4;   // lanes that cover the outputs once
+    constexpr int PS = 256 / Q;     // part sets
+    constexpr int NBATCH = 4;
+    static_assert(Q * PS <= 256, "lanes");
+    __shared__ float4 sa[PS][Q];
+    __shared__ float2 sml[PS][Q];
+    const int b = (int)blockIdx.y, y = (int)blockIdx.x;
+    const int n = item_parts_of(p, item_tiles(p, b));
+    if (n <= 1) return;  // written by the split kernel
+    const int o = (int)threadIdx.x % Q, ps = (int)threadIdx.x / Q;
+    const int h = 4 * o / D;
+    const size_t slot0 = ((size_t)b * gridDim.x + y) * p.item_parts;
+    const float4* acc = reinterpret_cast<const float4*>(p.part_acc) + slot0 * Q + o;
+    const float2* ml = reinterpret_cast<const float2*>(p.part_ml) + slot0 * GW + h;
+    // -1e30 (not -inf) keeps exp2 finite
+    float M = -1e30f, L = 0.f;
+    float4 A = make_float4(0.f, 0.f, 0.f, 0.f);
+    auto add = [&](float m, float l, float4 a) {
+        const float nm = fmaxf(M, m);
+        const float fo = exp2f(M - nm), fn = exp2f(m - nm);
+        A.x = fmaf(a.x, fn, A.x * fo);
+        A.y = fmaf(a.y, fn, A.y * fo);
+        A.z = fmaf(a.z, fn, A.z * fo);
+        A.w = fmaf(a.w, fn, A.w * fo);
+        L = fmaf(l, fn, L * fo);
+        M = nm;
+    };
+    for (int i = ps; ps < PS && i < n; i += PS * NBATCH) {
+        float2 mlv[NBATCH];
+        float4 av[NBATCH];
+#pragma unroll
+        for (int k = 0; k < NBATCH; ++k) {
+            const int j = min(i + k * PS, n - 1);
+            mlv[k] = ml[(size_t)j * GW];
+            av[k] = acc[(size_t)j * Q];
+        }
+#pragma unroll
+        for (int k = 0; k < NBATCH; ++k) {
+            if (i + k * PS < n) add(mlv[k].x, mlv[k].y, av[k]);
+        }
+    }
+    if (ps > 0 && ps < PS) {
+        sa[ps][o] = A;
+        sml[ps][o] = make_float2(M, L);
+    }
+    __syncthreads();
+    if (ps != 0) return;
+#pragma unroll
+    for (int s = 1; s < PS; ++s) add(sml[s][o].x, sml[s][o].y, sa[s][o]);
+    reinterpret_cast<float4*>(p.out + ((size_t)b * p.hq + (size_t)y * GW) * D)[o] =
+        L > 0.f ? make_float4(A.x / L, A.y / L, A.z / L, A.w / L) : make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
 // Merge launch of a split decode: one workgroup per work item (grid = batch * hkv *

@@ -988,19 +988,70 @@ uint32_t decode_min_tiles_per_wg(uint64_t items) {
     return items <= 8 ? 16u : 1u;
 }
 
-// f16 batches whose contexts the host knows to be the same, whose work items about fill the
-// CUs (between 15/16 of them and all of them) and hold at least 96 tiles each run one whole
-// item per workgroup of 8 waves instead of splitting items over workgroups and merging
-// their partial states in a second launch.  VSPEC_ROCM_DECODE_WIDE (read on every call): 0
-// never, 2 whenever the items fit the CUs, else (default, 1) the rule above.  Measured at
-// B = 32 (256 items), whole against split: 1025 tokens 33.6 / 32.3 us, 2049 53.9 / 57.4,
-// 4097 94.0 / 97.6, 8193 174.1 / 177.4, 32769 665 / 669; B = 30 at 4097: 90.4 / 97.1.
-// With fewer items the split over all CUs wins (C2, 128 items: 36.0 split, 44.0 whole).
-bool decode_wide(uint64_t items, uint64_t cus, uint64_t tiles) {
-    const char* e = getenv("VSPEC_ROCM_DECODE_WIDE");
-    const long x = e ? strtol(e, nullptr, 10) : 1;
-    if (x == 0 || items > cus) return false;
-    return x == 2 || (items * 16 >= cus * 15 && tiles >= 96);
+// An explicitly set knob of the balanced split (the functions around here) selects it.
+bool balanced_split_env() {
+    for (const char* k : {"VSPEC_ROCM_DECODE_WGS_PER_CU", "VSPEC_ROCM_DECODE_OLD_PERMILLE", "VSPEC_ROCM_DECODE_OLD_PERMILLE_INT4",
+                          "VSPEC_ROCM_DECODE_MIN_TILES_PER_WG", "VSPEC_ROCM_DECODE_SEGMENT_COST",
+                          "VSPEC_ROCM_DECODE_SEGMENT_COST_INT4"}) {
+        if (getenv(k)) return true;
+    }
+    return false;
+}
+
+// Parts of a work item under the item split (kv_common.h item_part), or 0 for the balanced
+// split of all items' tiles.  Read on every call: VSPEC_ROCM_DECODE_ITEM_PARTS 0 never, 1..64
+// that many (as far as the workspace holds them); VSPEC_ROCM_DECODE_WIDE=2 whole items
+// wherever they fit the CUs.
+//
+// Else the cheaper one by a cost model in us, fitted to both splits over 30 shapes (1-128
+// sequences of 19-16k tokens): `slots` workgroups run at a time; with k of them running, a
+// part of n tiles takes n * hypot(lat, k * bw), lat being a tile's share of one workgroup's
+// dependent round trips and bw its share of the memory rate (f16) or of the issue rate
+// (int4); a set-up `pro` is paid once, a merge launch with more than one part.  The balanced
+// split pays more set-up (its pass over the contexts, several items per workgroup one after
+// the other, a merge launch that redoes the split) and no last round of few workgroups.
+// Measured, balanced -> item split, f16: 1 x 21 tokens 38.4 -> 7.4 us, 1 x 4097 22.1 -> 15.1,
+// 16 x 2049 36.2 -> 27.8, 61 x 102 30.8 -> 11.7, 64 x 1025 50.4 -> 45.3, 64 x 4097 168.5 -> 166.1,
+// 65 x 4097 187 -> 218 (not taken); int4: 1 x 4097 17.9 -> 15.1, 16 x 2049 22.2 -> 18.5, 64 x 1025
+// 22.8 -> 21.8, 100 x 2000 68.1 -> 59.9, 65 x 4097 74 -> 89 (not taken).  A batch whose
+// contexts may differ takes the item split only up to 72 tiles a part, since the launch ends
+// with its longest part (64 sequences of 128-8192 tokens, 2 parts of up to 256 tiles: 162.5
+// -> 183.8 us).  The parts never need more workspace than the balanced split's plan.
+struct SplitCost {
+    double lat, bw, pro, bal_tile, bal;
+};
+uint32_t plan_item_parts(const VspecPagedAttnDesc* d, uint64_t items, uint64_t tiles, uint64_t slots, uint64_t max_wgs,
+                         bool same) {
+    if (d->batch > 65535u || items / d->batch * 64 > 0x7fffffu) return 0;
+    const uint64_t most = max_wgs / items > 1 ? max_wgs / items : 1;
+    const char* e = getenv("VSPEC_ROCM_DECODE_ITEM_PARTS");
+    if (e && *e) {
+        const long x = strtol(e, nullptr, 10);
+        return x <= 0 ? 0u : (uint32_t)((uint64_t)x < most ? (x < 64 ? x : 64) : (most < 64 ? most : 64));
+    }
+    if (balanced_split_env()) return 0;
+    e = getenv("VSPEC_ROCM_DECODE_WIDE");
+    if (e && strtol(e, nullptr, 10) == 2 && same && items <= slots / 2) return 1;
+    const bool i4 = d->kv.dtype == VSPEC_KV_INT4;
+    const double size = d->kv.head_dim / 128.0;
+    const SplitCost c = i4 ? SplitCost{0.15, 2.6e-4 * (1 + size) / 2, 7.0, 4.2e-4 * (1 + size) / 2, 19.0}
+                           : SplitCost{0.215, 1.26e-3 * size, 6.5, 1.26e-3 * size, 22.0};
+    const double busy = sqrt(c.lat * c.lat + (double)(slots * slots) * c.bw * c.bw);
+    double best = (double)(items * tiles) * c.bal_tile * (same ? 1.0 : 0.75) + c.bal;
+    uint32_t parts = 0;
+    for (const uint32_t p : {1u, 2u, 3u, 4u, 6u, 8u, 12u, 16u, 24u, 32u, 48u, 64u}) {
+        if (p > 1 && (p > most || (uint64_t)p * 4 > tiles + 3)) break;
+        const uint64_t n = (tiles + p - 1) / p;
+        if (!same && n > 72) continue;
+        const double full = (double)(items * p / slots), rem = (double)(items * p % slots);
+        const double t = (double)n * (full * busy + (rem > 0 ? sqrt(c.lat * c.lat + rem * rem * c.bw * c.bw) : 0.0)) + c.pro +
+                         (p > 1 ? 5.0 + 0.12 * p : 0.0);
+        if (t < best) {
+            best = t;
+            parts = p;
+        }
+    }
+    return parts;
 }
 
 // Balanced split of ragged f16 batches: every work item also costs this many tiles
@@ -1045,7 +1096,7 @@ uint32_t decode_flag_min_tiles() {
 
 struct DecodePlan {
     bool merge;  // split MFMA kernels: some work item may span two workgroups (merge launch)
-    bool wide;   // f16: one whole work item per workgroup of 8 waves (no merge launch)
+    uint32_t item_parts;  // item split (kv_common.h): parts of a work item, 0: ranges of all items' tiles
     uint32_t gw;
     uint32_t gsplit;
     uint32_t tiles_per_part;
@@ -1134,7 +1185,7 @@ int plan_decode(const VspecPagedAttnDesc* d, DecodePlan* pl) {
     }
     const uint32_t max_tiles = (uint32_t)((ctx_bound + kTile - 1) / kTile);
     pl->split = d->kv.dtype != VSPEC_KV_F32;
-    pl->wide = false;
+    pl->item_parts = 0;
     pl->min_tiles = decode_min_tiles_per_wg((uint64_t)d->batch * hkv * pl->gsplit);
     if (pl->split) {
         // every workgroup streams an equal share of all work items' tiles
@@ -1151,13 +1202,6 @@ int plan_decode(const VspecPagedAttnDesc* d, DecodePlan* pl) {
             }
             pl->chunk_tiles = d->partition_tokens / kTile;
             grid = (bound + pl->chunk_tiles - 1) / pl->chunk_tiles;
-        } else if (d->kv.dtype == VSPEC_KV_F16 && d->min_ctx_len && d->min_ctx_len >= ctx_bound &&
-                   decode_wide((uint64_t)d->batch * hkv * pl->gsplit, (uint64_t)num_cus(), max_tiles)) {
-            // whole items on 8-wave workgroups: every context is the same (the host says so),
-            // so chunks of one item's tiles are exactly the items
-            pl->wide = true;
-            pl->chunk_tiles = 0;  // set below from the items' tiles
-            grid = (uint64_t)d->batch * hkv * pl->gsplit;
         } else {
             pl->chunk_tiles = 0;
             // two workgroups per CU; small f16 batches (under 64 tiles per workgroup at two
@@ -1185,9 +1229,13 @@ int plan_decode(const VspecPagedAttnDesc* d, DecodePlan* pl) {
         // unequal pair shares need the grid of two workgroups per CU (g and g + G/2 share one)
         pl->old_permille = !pl->chunk_tiles && pl->grid_x == 2u * (uint32_t)num_cus()
                                ? decode_old_permille(d->kv.dtype) : 500u;
-        if (pl->wide) pl->chunk_tiles = uniform_item_tiles(d, pl, ctx_bound);
         pl->merge = uniform_split_has_partials(d, pl, ctx_bound);
         pl->uniform_tiles = uniform_item_tiles(d, pl, ctx_bound);
+        // (a partial state of the balanced split's plan per part: 2 slots per workgroup)
+        if (!pl->chunk_tiles && d->batch) {
+            pl->item_parts = plan_item_parts(d, (uint64_t)d->batch * hkv * pl->gsplit, max_tiles ? max_tiles : 1,
+                                             2ull * (uint64_t)num_cus(), 2ull * pl->grid_x, pl->uniform_tiles != 0);
+        }
         // the workspace stays even without a merge launch: a context below min_ctx_len (a
         // caller error) then leaves its partial states in valid memory, not its output
         pl->ws_bytes = (size_t)pl->grid_x * 2 * pl->gw * (2 + d->kv.head_dim) * sizeof(float);
@@ -1748,7 +1796,7 @@ int paged_decode(const VspecPagedAttnDesc* desc, const void* k_new, const void* 
     p.split_old_permille = pl.split ? pl.old_permille : 500u;
     p.uniform_tiles = pl.split ? pl.uniform_tiles : 0u;
     p.min_tiles = pl.split && !pl.chunk_tiles ? pl.min_tiles : 1u;
-    p.wide = pl.wide;
+    p.item_parts = pl.item_parts;
     p.seg_cost = !pl.split || pl.chunk_tiles ? 0u
                  : desc->kv.dtype == VSPEC_KV_F16 ? decode_segment_cost()
                  : desc->kv.dtype == VSPEC_KV_INT4 ? decode_segment_cost_int4() : 0u;
@@ -1782,12 +1830,22 @@ int paged_decode(const VspecPagedAttnDesc* desc, const void* k_new, const void* 
         // partial slots [grid][2][GW] of (max, sum) then of acc[D]
         p.part_acc = (float*)ws + (size_t)pl.grid_x * 2 * pl.gw * 2;
     }
-    const dim3 grid = pl.split ? dim3(pl.grid_x) : dim3(pl.max_parts, desc->kv.num_kv_heads * pl.gsplit, desc->batch);
+    if (pl.item_parts) {
+        // partial slots [batch][item][part][GW]: acc[D] of all, then (max, sum)
+        p.part_acc = (float*)ws;
+        p.part_ml = (float*)ws + (size_t)desc->batch * desc->kv.num_kv_heads * pl.gsplit * pl.item_parts * pl.gw * D;
+    }
+    const dim3 grid = pl.item_parts ? dim3(desc->kv.num_kv_heads * pl.gsplit * pl.item_parts, desc->batch)
+                      : pl.split ? dim3(pl.grid_x) : dim3(pl.max_parts, desc->kv.num_kv_heads * pl.gsplit, desc->batch);
     int ok = 0;
     switch (desc->kv.dtype) {
         case VSPEC_KV_F32: ok = dispatch_d<VSPEC_KV_F32>(D, pl.gw, p, grid, s); break;
-        case VSPEC_KV_F16: ok = launch_decode_mfma_f16(p, D, pl.gw, grid, s); break;
-        default: ok = launch_decode_mfma_int4(p, D, pl.gw, grid, s); break;
+        case VSPEC_KV_F16:
+            ok = D == 64 ? launch_decode_mfma_f16_d64(p, pl.gw, grid, s) : launch_decode_mfma_f16_d128(p, pl.gw, grid, s);
+            break;
+        default:
+            ok = D == 64 ? launch_decode_mfma_int4_d64(p, pl.gw, grid, s) : launch_decode_mfma_int4_d128(p, pl.gw, grid, s);
+            break;
     }
     if (!ok) {
         set_err("paged_decode: no kernel for head_dim %u, group %u", D, pl.gw);
