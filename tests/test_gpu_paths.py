@@ -177,3 +177,30 @@ def test_item_split_keeps_the_workspace_plan(gpu, monkeypatch):
         d = vr.make_decode_desc(pools[0], tables, cl, q, out, bound, workspace=ws)
         assert vr.lib().vspec_rocm_paged_decode_attention(C.byref(d)), vr.last_error()
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("lens,Hq,H,D,P,used,src", [
+    ([1], 8, 8, 64, 16, False, "f16"), ([16, 17, 0, 1], 8, 2, 128, 16, False, "f32"), ([64, 65, 80, 81, 3], 6, 2, 64, 48, False, "f32"),
+    ([257], 24, 2, 128, 16, False, "f16"), ([1000, 31, 515], 32, 4, 128, 32, True, "f32"), ([300] * 5, 16, 2, 64, 16, True, "f16")])
+def test_f32_step_parts(gpu, monkeypatch, lens, Hq, H, D, P, used, src):
+    """f32 pools: the fused step (token patched into the tile that holds it, by every group of
+    query heads) against kv_append and the plain decode in one part, for several part counts:
+    the same pool bytes; outputs within the rounding of f32 sums in another order (weights
+    <= 1 against |v| < 6: 16 * 2^-24 * 6)."""
+    import torch
+
+    vr, pools, tables, ctx, q, new, bu = _decode_setup(gpu, "f32", lens, Hq, H, D, P, used)
+    if src == "f32":
+        new = [x.float() * 1.001 for x in new]
+    live = [b for b, t in enumerate(lens) if t]
+    at = torch.tensor([lens[b] - 1 for b in live], dtype=torch.int32)
+    vr.kv_append(pools[0], tables[live].contiguous(), at, *(x[live][:, None].contiguous() for x in new))
+    hint = dict(max_ctx_len=max(lens), block_used=bu)
+    for numerics in (vr.NUMERICS_PLAIN, vr.NUMERICS_3BIT):
+        monkeypatch.setenv("VSPEC_ROCM_DECODE_ITEM_PARTS", "1")
+        want = vr.paged_decode(pools[0], tables, ctx, q, numerics=numerics, **hint)
+        for parts in ("", "1", "2", "5", "64"):
+            monkeypatch.setenv("VSPEC_ROCM_DECODE_ITEM_PARTS", parts)
+            got = vr.paged_decode_step(pools[1], tables, ctx, q, *new, numerics=numerics, **hint)
+            assert _same_pools(*pools)
+            assert float((got - want).abs().max()) <= 6e-6

@@ -1,0 +1,307 @@
+// decode_f32.hip -- single-query GQA decode attention over f32 paged KV on the vector ALUs
+// (fp32 products throughout: the matrix cores' f32 form measured no faster), with the
+// reference numerics (per-key std clamp, attention_ref.c:50-62).
+//
+// One workgroup of 4 waves per part of a work item (item_part); wave w takes the part's
+// tiles w, w + 4, ...  D/16 lanes hold one key, 16 elements each (chunks of 4 elements
+// sub + j * D/16); D/8 lanes hold one token of V, 8 elements each.  The decode step's token is
+// taken from its source rows by every wave that reads its tile, so no launch precedes this one.
+//
+// Bound by the memory rate at full batches (16 x 2049 tokens: 269 MB in 55.3 us with the merge
+// launch, 61 us with an append launch ahead and ordinary loads) and by a wave's chain of round
+// trips per tile (about 3 us) at small ones.
+#include "kv_common.h"
+
+namespace vkv {
+namespace {
+
+template <bool ONCE>
+__device__ __forceinline__ float4 load_row4(const float* p) {
+    if constexpr (!ONCE) return *reinterpret_cast<const float4*>(p);
+    const uint4 w = load_stream4(p);
+    return make_float4(__builtin_bit_cast(float, w.x), __builtin_bit_cast(float, w.y), __builtin_bit_cast(float, w.z),
+                       __builtin_bit_cast(float, w.w));
+}
+
+// 4 elements of a new token's row in its source type
+__device__ __forceinline__ float4 load_new4(const uint8_t* src, size_t el, int32_t type) {
+    if (type == VSPEC_KV_F32) return *reinterpret_cast<const float4*>(src + el * 4);
+    const uint2 w = *reinterpret_cast<const uint2*>(src + el * 2);
+    return make_float4(half_bits_to_float(w.x & 0xffffu), half_bits_to_float(w.x >> 16), half_bits_to_float(w.y & 0xffffu),
+                       half_bits_to_float(w.y >> 16));
+}
+
+// Clip a row held by LPK lanes (16 elements each) to +-max(1e-6, alpha*std),
+// then to +-input_clip (three_bit_runtime_modules.c:175-203, :138-173).
+template <int LPK, int D>
+__device__ __forceinline__ void clamp_row(float* x, float alpha, float input_clip) {
+    float s = 0.f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) s += x[e];
+    const float mean = group_sum<LPK>(s) * (1.0f / D);
+    float v = 0.f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        const float d = x[e] - mean;
+        v = fmaf(d, d, v);
+    }
+    const float var = group_sum<LPK>(v) * (1.0f / D);
+    const float th = fminf(fmaxf(1e-6f, alpha * sqrtf(var)), input_clip);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) x[e] = fminf(fmaxf(x[e], -th), th);
+}
+
+// ONCE: each tile is read by one work item, past the caches (16 x 2049 tokens 55.6 us, 59.0 with
+// ordinary loads); else the gsplit items of a kv head share it in their XCD's L2 (25 x 37-2392
+// tokens, 8 heads per kv head: 54.8 us, 57.5 past the caches)
+template <int D, int GW, bool ONCE>
+__global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
+    constexpr int LPK = D / 16;           // lanes per key
+    constexpr int KPP = 64 / LPK;         // keys per K pass
+    constexpr int KPASS = kTile / KPP;    // K passes per tile
+    constexpr int VLPT = D / 8;           // lanes per token on the V side
+    constexpr int VTPP = 64 / VLPT;       // tokens per V pass
+    constexpr int VPASS = kTile / VTPP;   // V passes per tile
+    static_assert(KPASS >= 1 && VPASS >= 1, "tile geometry");
+
+    __shared__ float p_lds[kWaves][2][kTile][GW];
+    __shared__ float comb[kWaves][GW][D + 2];
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int lo, hi;
+    size_t part_slot;
+    const ItemCursor c = item_part(p, lo, hi, part_slot);
+    if (lo >= hi) return;
+    const int hk = __builtin_amdgcn_readfirstlane(c.y / (int)p.gsplit);
+    const int hq0 = c.y * GW;
+    const int tiles_per_block = (int)p.block_tokens / kTile;
+    const int ctx_cap = (int)(p.max_blocks * p.block_tokens);
+    const const_i32* table = as_const(p.block_tables) + (size_t)c.b * p.max_blocks;
+
+    const int kk = lane / LPK;      // key within a K pass
+    const int sub = lane % LPK;     // lane within the key
+    const int vc = lane % VLPT;     // V chunk
+    const int vt = lane / VLPT;     // token within a V pass
+
+    // q' = clip(q) * scale * log2(e), in the K-side lane layout
+    float qv[GW][16];
+#pragma unroll
+    for (int h = 0; h < GW; ++h) {
+        const float* qrow = p.q + ((size_t)c.b * p.hq + hq0 + h) * D;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float4 w = *reinterpret_cast<const float4*>(qrow + 4 * (sub + j * LPK));
+            qv[h][4 * j] = w.x; qv[h][4 * j + 1] = w.y; qv[h][4 * j + 2] = w.z; qv[h][4 * j + 3] = w.w;
+        }
+    }
+    int tile = lo + wave;
+    int entry = table[min(tile, hi - 1) / tiles_per_block];
+    const int raw_ctx = as_const(p.ctx_lens)[c.b];
+    const int ctx = min(max(raw_ctx, 0), ctx_cap);
+    // the decode step's new token: its position, and the decoded tile whose wave stores it
+    const int papp = p.k_new && raw_ctx >= 1 && raw_ctx <= ctx_cap ? raw_ctx - 1 : -1;
+    const int tnew = papp >= 0 ? min(papp / kTile, c.U - 1) : -1;
+#pragma unroll
+    for (int h = 0; h < GW; ++h) {
+        clamp_row<LPK, D>(qv[h], p.alpha, p.input_clip);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) qv[h][e] *= p.qscale;
+    }
+
+    float m_run[GW], l_run[GW], acc[GW][8];
+#pragma unroll
+    for (int h = 0; h < GW; ++h) {
+        m_run[h] = -INFINITY;
+        l_run[h] = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[h][e] = 0.f;
+    }
+
+    const bool v_early = D == 64 || hi - lo <= kWaves;
+    int buf = 0;
+    for (; tile < hi; tile += kWaves) {
+        const int phys = entry;
+        const int lblock = tile / tiles_per_block;
+        entry = table[min(tile + kWaves, hi - 1) / tiles_per_block];  // the wave's next tile's
+        const bool ok = phys >= 0 && (uint32_t)phys < p.num_blocks;  // else the tile is skipped
+        const int tok0 = tile * kTile;
+        const int slot0 = (tile % tiles_per_block) * kTile;
+        const size_t row0 = ((size_t)(ok ? phys : 0) * p.hkv + hk) * p.block_tokens + slot0;
+        const float* krow = reinterpret_cast<const float*>(p.k) + row0 * D;
+        const float* vrow = reinterpret_cast<const float*>(p.v) + row0 * D;
+        // the new token: taken from its source rows wherever the tile is read, and written to
+        // the pool here (its block may be another one where the context exceeds the bound)
+        const bool here = tile == tnew;
+        const int ts = here && tile == papp / kTile ? papp % kTile : -1;  // its slot in this tile
+        const size_t new_el = ((size_t)c.b * p.hkv + hk) * D;
+        if (here && c.y % (int)p.gsplit == 0) {
+            const int e = table[papp / (int)p.block_tokens];
+            if (e >= 0 && (uint32_t)e < p.num_blocks && lane < D / 4) {
+                const size_t row = ((size_t)e * p.hkv + hk) * p.block_tokens + papp % (int)p.block_tokens;
+                *reinterpret_cast<float4*>(const_cast<uint8_t*>(p.k) + (row * D + 4 * lane) * 4) = load_new4(p.k_new, new_el + 4 * lane, p.append_src);
+                *reinterpret_cast<float4*>(const_cast<uint8_t*>(p.v) + (row * D + 4 * lane) * 4) = load_new4(p.v_new, new_el + 4 * lane, p.append_src);
+            }
+        }
+        if (!ok) continue;
+        // valid slots of this tile: below the context and, with block_used, below its
+        // block's used count (a prefix of the block's slots)
+        const int lim = p.block_used ? min(ctx - tok0, used_cap(as_const(p.block_used)[(size_t)c.b * p.max_blocks + lblock], slot0))
+                                     : ctx - tok0;
+
+        // V goes out with K where a wave's chain of round trips, not the memory rate, is what
+        // it waits for: one tile per wave (89 x 1-26 tokens 19.2 -> 17.4 us), and 64-element
+        // heads (36 x 649-5195 67.0 -> 62.6 us); with 128 and longer parts it only costs
+        // registers (16 x 2049 55.7 -> 56.2 us)
+        float4 va[VPASS], vb[VPASS];
+        auto load_v = [&]() {
+#pragma unroll
+            for (int vp = 0; vp < VPASS; ++vp) {
+                va[vp] = load_row4<ONCE>(vrow + (size_t)(vp * VTPP + vt) * D + 8 * vc);
+                vb[vp] = load_row4<ONCE>(vrow + (size_t)(vp * VTPP + vt) * D + 8 * vc + 4);
+            }
+        };
+        if (v_early) load_v();
+        // ---- scores ----
+        float s[KPASS][GW];
+#pragma unroll
+        for (int kp = 0; kp < KPASS; ++kp) {
+            const int slot = kp * KPP + kk;
+            float x[16];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                float4 w = load_row4<ONCE>(krow + (size_t)slot * D + 4 * (sub + j * LPK));
+                if (slot == ts) w = load_new4(p.k_new, new_el + 4 * (sub + j * LPK), p.append_src);
+                x[4 * j] = w.x; x[4 * j + 1] = w.y; x[4 * j + 2] = w.z; x[4 * j + 3] = w.w;
+            }
+            clamp_row<LPK, D>(x, p.alpha, p.input_clip);
+            const bool valid = slot < lim;
+#pragma unroll
+            for (int h = 0; h < GW; ++h) {
+                float d = 0.f;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) d = fmaf(qv[h][e], x[e], d);
+                d = group_sum<LPK>(d);
+                d = fminf(fmaxf(d, -p.logit_clip), p.logit_clip);
+                s[kp][h] = valid ? d : -INFINITY;
+            }
+        }
+
+        // ---- online softmax (rescale only when the max grows by > 2^8) ----
+#pragma unroll
+        for (int h = 0; h < GW; ++h) {
+            float mt = s[0][h];
+#pragma unroll
+            for (int kp = 1; kp < KPASS; ++kp) mt = fmaxf(mt, s[kp][h]);
+            mt = max_across_groups<LPK>(mt);
+            // uniform across the wave after the reduction: keep it in an SGPR
+            mt = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, mt)));
+            if (mt > m_run[h] + 8.0f) {
+                const float f = exp2f(m_run[h] - mt);
+                l_run[h] *= f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) acc[h][e] *= f;
+                m_run[h] = mt;
+            }
+        }
+#pragma unroll
+        for (int kp = 0; kp < KPASS; ++kp) {
+            if (sub < GW) {
+                float sv = s[kp][0], mv = m_run[0];
+#pragma unroll
+                for (int h = 1; h < GW; ++h) {
+                    if (sub == h) {
+                        sv = s[kp][h];
+                        mv = m_run[h];
+                    }
+                }
+                p_lds[wave][buf][kp * KPP + kk][sub] = exp2f(sv - mv);
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+
+        // ---- P.V ----
+        if (!v_early) load_v();
+        const bool tail = lim < kTile;
+#pragma unroll
+        for (int vp = 0; vp < VPASS; ++vp) {
+            const int slot = vp * VTPP + vt;
+            float4 a = va[vp], b = vb[vp];
+            if (slot == ts) {
+                a = load_new4(p.v_new, new_el + 8 * vc, p.append_src);
+                b = load_new4(p.v_new, new_el + 8 * vc + 4, p.append_src);
+            }
+            float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+            if (tail && slot >= lim) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[e] = 0.f;
+            }
+            float pv[GW];
+#pragma unroll
+            for (int h = 0; h < GW; ++h) pv[h] = p_lds[wave][buf][slot][h];
+#pragma unroll
+            for (int h = 0; h < GW; ++h) {
+                l_run[h] += pv[h];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) acc[h][e] = fmaf(pv[h], x[e], acc[h][e]);
+            }
+        }
+        buf ^= 1;
+    }
+
+    // ---- reduce the token groups of the V layout (lanes with equal chunk) ----
+#pragma unroll
+    for (int h = 0; h < GW; ++h) {
+#pragma unroll
+        for (int off = VLPT; off < 64; off <<= 1) {
+            l_run[h] += __shfl_xor(l_run[h], off);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[h][e] += __shfl_xor(acc[h][e], off);
+        }
+    }
+    if (lane < VLPT) {
+#pragma unroll
+        for (int h = 0; h < GW; ++h) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) comb[wave][h][2 + 8 * vc + e] = acc[h][e];
+            if (vc == 0) {
+                comb[wave][h][0] = fmaxf(m_run[h], -1e30f);  // (finite: a wave without tokens)
+                comb[wave][h][1] = l_run[h];
+            }
+        }
+    }
+    __syncthreads();
+    finish_item<D, GW, kWaves>(p, comb, c, part_slot, hi - lo == c.U);
+}
+
+template <int D, int GW>
+void launch(const DecodeParams& p, dim3 grid, hipStream_t s) {
+    if (p.gsplit == 1) hipLaunchKernelGGL((decode_f32<D, GW, true>), grid, dim3(kWaves * 64), 0, s, p);
+    else hipLaunchKernelGGL((decode_f32<D, GW, false>), grid, dim3(kWaves * 64), 0, s, p);
+    if (p.item_parts > 1) {
+        hipLaunchKernelGGL((decode_merge_items<D, GW>), dim3(p.hkv * p.gsplit, p.batch), dim3(256), 0, s, p);
+    }
+}
+
+template <int D>
+int launch_gw(uint32_t gw, const DecodeParams& p, dim3 grid, hipStream_t s) {
+    switch (gw) {
+        case 1: launch<D, 1>(p, grid, s); return 1;
+        case 2: launch<D, 2>(p, grid, s); return 1;
+        case 3: launch<D, 3>(p, grid, s); return 1;
+        case 4: launch<D, 4>(p, grid, s); return 1;
+        default: return 0;
+    }
+}
+
+}  // namespace
+
+int launch_decode_f32(const DecodeParams& p, uint32_t head_dim, uint32_t gw, dim3 grid, hipStream_t stream) {
+    if (head_dim == 64) return launch_gw<64>(gw, p, grid, stream);
+    if (head_dim == 128) return launch_gw<128>(gw, p, grid, stream);
+    return 0;
+}
+
+}  // namespace vkv

@@ -66,7 +66,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
     __shared__ int qexp[GW];                     // ITEMS: per head, the q' operand shift (qnorm_shift)
     // per wave: QK B operands (hi, lo for each 32-wide d chunk), read back every tile
     __shared__ float comb[kSlots][NW][GW][D + 2];
-    __shared__ float patch_val[NW][kTile][4];
+    __shared__ float patch_val[NW][kTile][GW];
     __shared__ int patch_flag[NW][kTile];
     __shared__ int slot_cnt[kSlots];
     __shared__ int slot_seg[kSlots];
@@ -86,9 +86,10 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
 
     const int ips = (int)(p.hkv * p.gsplit);  // work items per sequence
     WorkSplit ws = {};
+    size_t part_slot = 0;  // ITEMS
     ItemCursor first;
     if constexpr (ITEMS) {
-        first = item_part(p, ws.lo, ws.hi);
+        first = item_part(p, ws.lo, ws.hi, part_slot);
     } else {
         ws = work_split<kSplitRagged, NW>(p, ips, split_sh);
     }
@@ -556,13 +557,17 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
         // One work item's part (item_part): its q rows and new token are read by different
         // waves, each wave's first tiles are on their way while head w is prepared by wave w,
         // one barrier publishes them, and all waves merge after another.
-        static_assert(GW <= NW, "one wave per head");
         constexpr int E = D / 64;
-        float x[E];
-        if (wave < GW) {
-            const float* qrow = p.q + ((size_t)pc.b * p.hq + (size_t)pc.y * GW + wave) * D;
+        constexpr int HPW = (GW + NW - 1) / NW;  // heads per wave: w, w + NW
+        float x[HPW][E];
 #pragma unroll
-            for (int e = 0; e < E; ++e) x[e] = qrow[lane * E + e];
+        for (int i = 0; i < HPW; ++i) {
+            const int h = wave + i * NW;
+            if (h < GW) {
+                const float* qrow = p.q + ((size_t)pc.b * p.hq + (size_t)pc.y * GW + h) * D;
+#pragma unroll
+                for (int e = 0; e < E; ++e) x[i][e] = qrow[lane * E + e];
+            }
         }
         // the first tiles' table entries and the context in one scalar round trip
         int entry[NB];
@@ -580,9 +585,13 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
         for (int u = 0; u < NB; ++u) {
             if (u < nt) ok[u] = load_entry(t0 + u * NW, true, t0 + u * NW, erow[u], entry[u], f[u]);
         }
-        if (wave < GW) {
-            const int e = qhead(wave, x);
-            if (lane == 0) qexp[wave] = e;
+#pragma unroll
+        for (int i = 0; i < HPW; ++i) {
+            const int h = wave + i * NW;
+            if (h < GW) {
+                const int e = qhead(h, x[i]);
+                if (lane == 0) qexp[h] = e;
+            }
         }
         if (stage) newrow_store(row, 0);
         __syncthreads();
@@ -621,7 +630,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
             }
         }
         __syncthreads();
-        finish_item<D, GW, NW>(p, comb[0], pc, ws.hi - ws.lo == pc.U);
+        finish_item<D, GW, NW>(p, comb[0], pc, part_slot, ws.hi - ws.lo == pc.U);
         return;
     }
     // Set-up.  Wave 0 loads the q rows of the range's first kQStage segments (rows GW*y ..

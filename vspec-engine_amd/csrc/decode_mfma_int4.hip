@@ -190,9 +190,10 @@ __global__ __launch_bounds__(256, VSPEC_I4_MIN_WG_PER_CU) void decode_mfma_i4(De
 
     const int ips = (int)(p.hkv * p.gsplit);  // work items per sequence
     WorkSplit ws = {};
+    size_t part_slot = 0;  // ITEMS
     ItemCursor c0 = {0, 0, 1, 0, 0};
     if constexpr (ITEMS) {
-        c0 = item_part(p, ws.lo, ws.hi);
+        c0 = item_part(p, ws.lo, ws.hi, part_slot);
         ws.b = c0.b;
         if (ws.lo >= ws.hi) return;
     } else {
@@ -992,7 +993,7 @@ __global__ __launch_bounds__(256, VSPEC_I4_MIN_WG_PER_CU) void decode_mfma_i4(De
         }
         __syncthreads();
         if constexpr (ITEMS) {
-            finish_item<D, GW, kWaves>(p, comb, c0, tile_end - tile_begin == U);
+            finish_item<D, GW, kWaves>(p, comb, c0, part_slot, tile_end - tile_begin == U);
             return;
         }
         finish_segment<D, GW>(p, comb, b, hq0, U, tile_begin, tile_end, pos == ws.lo ? 0 : 1);

@@ -230,15 +230,13 @@ struct DecodeParams {
     const int32_t* block_used;  // [B][max_blocks] tokens per table entry's block, or null (full)
     const float* q;
     float* out;
-    float* part_ml;    // [B][Hq][max_parts][2] (max in log2 units, sum)
-    float* part_acc;   // [B][Hq][max_parts][D]
+    float* part_ml;    // partial states: (max in log2 units, sum) and acc[D] of each slot and head
+    float* part_acc;
     uint32_t hq;
     uint32_t hkv;
     uint32_t block_tokens;
     uint32_t max_blocks;
     uint32_t num_blocks;
-    uint32_t tiles_per_part;
-    uint32_t max_parts;
     uint32_t gsplit;   // work items per kv head (Hq/Hkv/GW)
     float qscale;      // softmax scale * log2(e)
     float alpha;       // std-clamp alpha
@@ -271,50 +269,17 @@ struct DecodeParams {
     uint32_t seg_cost;
     // item split: parts of a work item (grid (hkv * gsplit * item_parts, batch)), 0: the ranges above
     uint32_t item_parts;
+    uint32_t part_tiles;  // least tiles per part
 };
 
-// Launch the MFMA decode kernels for f16 pools (decode_mfma.hip) and int4 pools
-// (decode_mfma_int4.hip) of head_dim 64 or 128, each followed by its merge launch; they
+// Launch the decode kernels for f32 pools (decode_f32.hip), f16 pools (decode_mfma.hip) and
+// int4 pools (decode_mfma_int4.hip) of head_dim 64 or 128, each followed by its merge launch; they
 // return 0 when no instantiation matches (heads per work item).
+int launch_decode_f32(const DecodeParams& p, uint32_t head_dim, uint32_t gw, dim3 grid, hipStream_t stream);
 int launch_decode_mfma_f16_d64(const DecodeParams& p, uint32_t gw, dim3 grid, hipStream_t stream);
 int launch_decode_mfma_f16_d128(const DecodeParams& p, uint32_t gw, dim3 grid, hipStream_t stream);
 int launch_decode_mfma_int4_d64(const DecodeParams& p, uint32_t gw, dim3 grid, hipStream_t stream);
 int launch_decode_mfma_int4_d128(const DecodeParams& p, uint32_t gw, dim3 grid, hipStream_t stream);
-
-// Merge the kWaves per-wave softmax states of a workgroup (comb[w][h] = {max, sum,
-// acc[D]}) and write the output row (one partition) or the split-K partial.
-template <int D, int GW>
-__device__ __forceinline__ void merge_waves(const DecodeParams& p, const float (*comb)[GW][D + 2], int b,
-                                            int hq0, int part, int nparts) {
-    for (int idx = threadIdx.x; idx < GW * D; idx += kWaves * 64) {
-        const int h = idx / D;
-        const int d = idx % D;
-        float M = -INFINITY;
-#pragma unroll
-        for (int w = 0; w < kWaves; ++w) M = fmaxf(M, comb[w][h][0]);
-        float a = 0.f, l = 0.f;
-#pragma unroll
-        for (int w = 0; w < kWaves; ++w) {
-            const float mw = comb[w][h][0];
-            if (mw != -INFINITY) {
-                const float f = exp2f(mw - M);
-                a = fmaf(comb[w][h][2 + d], f, a);
-                l = fmaf(comb[w][h][1], f, l);
-            }
-        }
-        const size_t hq = (size_t)b * p.hq + hq0 + h;
-        if (nparts == 1) {
-            p.out[hq * D + d] = l > 0.f ? a / l : 0.f;
-        } else {
-            const size_t slot = hq * p.max_parts + part;
-            p.part_acc[slot * D + d] = a;
-            if (d == 0) {
-                p.part_ml[2 * slot] = M;
-                p.part_ml[2 * slot + 1] = l;
-            }
-        }
-    }
-}
 
 // ---------------------------------------------------------------------------
 // Work split of the MFMA decode kernels.
@@ -761,36 +726,56 @@ __device__ __forceinline__ void finish_segment(const DecodeParams& p, const floa
 
 // ---------------------------------------------------------------------------
 // Item split (DecodeParams.item_parts): workgroup (y * parts + part, b) takes part `part` of
-// work item y of sequence b.  An item of U tiles is cut into n = min(parts, ceil(U / 4)) parts
-// (a part has work for the 4 waves), of tiles [part * U / n, (part + 1) * U / n).  No pass over ctx_lens, no workgroup with two
+// work item y of sequence b.  An item of U tiles is cut into n = min(parts, ceil(U / part_tiles))
+// parts, of tiles [part * U / n, (part + 1) * U / n).  No pass over ctx_lens, no workgroup with two
 // items; an item in one part goes straight to the output, and the partial states of the
 // others lie at item * parts + part, where decode_merge_items finds them without redoing a
 // split.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ int item_parts_of(const DecodeParams& p, int U) { return min((int)p.item_parts, (U + 3) / 4); }
+__device__ __forceinline__ int item_parts_of(const DecodeParams& p, int U) { return min((int)p.item_parts, (U + (int)p.part_tiles - 1) / (int)p.part_tiles); }
 
 // this workgroup's item (tile positions count from the item's first tile) and tiles [lo, hi);
-// lo = hi when it has none
-__device__ __forceinline__ ItemCursor item_part(const DecodeParams& p, int& lo, int& hi) {
+// lo = hi when it has none; slot: the part's partial state
+__device__ __forceinline__ ItemCursor item_part(const DecodeParams& p, int& lo, int& hi, size_t& slot) {
     ItemCursor c;
-    c.b = (int)blockIdx.y;
     c.seq0 = 0;
     c.item0 = 0;
-    c.U = item_tiles(p, c.b);
-    int part = 0;
-    c.y = (int)blockIdx.x;
-    if (p.item_parts > 1) {
-        c.y = (int)((uint32_t)blockIdx.x / p.item_parts);
-        part = (int)blockIdx.x - c.y * (int)p.item_parts;
+    uint32_t b = blockIdx.y, x = blockIdx.x, g = 0;
+    if (p.gsplit > 1) {
+        // The gsplit items of one kv head read the same tiles: 8 workgroups apart they run on
+        // one XCD side by side, and its L2 can serve all but the first (workgroups go to the 8
+        // XCDs in turn).  Units of (sequence, kv head, part), 8 at a time; the last few as they come.
+        const uint32_t per = p.hkv * p.item_parts, units = p.batch * per / 8 * 8;
+        const uint32_t id = blockIdx.y * gridDim.x + blockIdx.x;
+        if (id < units * p.gsplit) {
+            const uint32_t w = 8 * p.gsplit, j = id % w;
+            g = j / 8;
+            x = id / w * 8 + j % 8;
+        } else {
+            x = units + (id - units * p.gsplit) / p.gsplit;
+            g = (id - units * p.gsplit) % p.gsplit;
+        }
+        b = x / per;
+        x -= b * per;
     }
+    uint32_t part = 0;
+    if (p.item_parts > 1) {
+        const uint32_t k = x / p.item_parts;
+        part = x - k * p.item_parts;
+        x = k;
+    }
+    c.b = __builtin_amdgcn_readfirstlane((int)b);
+    c.y = (int)(x * p.gsplit + g);
+    c.U = item_tiles(p, c.b);
     const int n = item_parts_of(p, c.U);
-    const int l = part < n ? (int)((uint32_t)part * (uint32_t)c.U / (uint32_t)n) : 0;
-    const int h = part < n ? (int)((uint32_t)(part + 1) * (uint32_t)c.U / (uint32_t)n) : 0;
+    const int l = (int)part < n ? (int)(part * (uint32_t)c.U / (uint32_t)n) : 0;
+    const int h = (int)part < n ? (int)((part + 1) * (uint32_t)c.U / (uint32_t)n) : 0;
     // wave-uniform values on the scalar unit (the divisions run on the vector one)
     c.y = __builtin_amdgcn_readfirstlane(c.y);
     c.U = __builtin_amdgcn_readfirstlane(c.U);
     lo = __builtin_amdgcn_readfirstlane(l);
     hi = __builtin_amdgcn_readfirstlane(h);
+    slot = (size_t)c.b * gridDim.x + (uint32_t)c.y * p.item_parts + part;
     return c;
 }
 
@@ -798,8 +783,7 @@ __device__ __forceinline__ ItemCursor item_part(const DecodeParams& p, int& lo, 
 // the part's partial state.
 template <int D, int GW, int NW>
 __device__ __forceinline__ void finish_item(const DecodeParams& p, const float (*st)[GW][D + 2], const ItemCursor& c,
-                                            bool whole) {
-    const size_t slot = (size_t)c.b * gridDim.x + blockIdx.x;
+                                            size_t slot, bool whole) {
     const size_t row0 = (size_t)c.b * p.hq + (size_t)c.y * GW;
     for (int idx = (int)threadIdx.x; idx < GW * D; idx += NW * 64) {
         const int h = idx / D;
@@ -878,7 +862,10 @@ __global__ __launch_bounds__(256) void decode_merge_items(DecodeParams p) {
     __syncthreads();
     if (ps != 0) return;
 #pragma unroll
-    for (int s = 1; s < PS; ++s) add(sml[s][o].x, sml[s][o].y, sa[s][o]);
+    for (int s = 1; s < PS; ++s) {
+        if (s >= n) break;  // (sets past the parts are empty)
+        add(sml[s][o].x, sml[s][o].y, sa[s][o]);
+    }
     reinterpret_cast<float4*>(p.out + ((size_t)b * p.hq + (size_t)y * GW) * D)[o] =
         L > 0.f ? make_float4(A.x / L, A.y / L, A.z / L, A.w / L) : make_float4(0.f, 0.f, 0.f, 0.f);
 }
@@ -894,7 +881,7 @@ template <int D, int GW, int UNEVEN>
 __global__ __launch_bounds__(kWaves * 64) void decode_merge_split(DecodeParams p) {
     constexpr int NT = kWaves * 64;
     constexpr int K = (GW * D + NT - 1) / NT;  // outputs per thread: idx = tid + NT * k
-    constexpr int NBATCH = 16;
+    constexpr int NBATCH = K > 2 ? 8 : 16;
     __shared__ SplitShared sh;
     const int ips = (int)(p.hkv * p.gsplit);
     const int b = (int)blockIdx.x / ips;

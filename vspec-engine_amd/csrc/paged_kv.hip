@@ -4,8 +4,6 @@
 //   kv_append      block-table append of new K/V; int4 pools quantise on write
 //   kv_gather      block-table gather into [T][H][D] (raw bytes or dequantised f32)
 //   kv_compact     whole-block moves (compaction after eviction)
-//   decode_partial single-query GQA attention, split-K over 16-token tiles
-//   decode_combine log-sum-exp merge of the split-K partials
 //
 // The C-ABI is declared in include/vspec_rocm.h.
 #include <hip/hip_runtime.h>
@@ -59,301 +57,6 @@ struct Row {
     static constexpr int kBytes = DT == VSPEC_KV_F32 ? D * 4 : (DT == VSPEC_KV_F16 ? D * 2 : D / 2);
     static constexpr int kScales = DT == VSPEC_KV_INT4 ? D / 32 : 0;
 };
-
-// K-side layout of the VALU decode kernel (f32 and f16 pools): LPK lanes hold one
-// key, 16 elements per lane.
-//   f16:  chunks of 8 elements (16 B), lane chunks sub, sub+LPK
-//   f32:  chunks of 4 elements (16 B), lane chunks sub + j*LPK, j < 4
-template <int DT, int D>
-__device__ __forceinline__ int k_elem(int sub, int e) {
-    static_assert(DT != VSPEC_KV_INT4, "int4 pools decode on the matrix cores");
-    constexpr int LPK = D / 16;
-    if constexpr (DT == VSPEC_KV_F16) {
-        return 8 * (sub + (e / 8) * LPK) + (e % 8);
-    } else {
-        return 4 * (sub + (e / 4) * LPK) + (e % 4);
-    }
-}
-
-template <int DT, int D>
-__device__ __forceinline__ void load_k16(const DecodeParams& p, size_t row, int sub, float* x) {
-    constexpr int LPK = D / 16;
-    if constexpr (DT == VSPEC_KV_F16) {
-        const uint4* src = reinterpret_cast<const uint4*>(p.k + row * (size_t)(D * 2));
-        unpack_f16x8(src[sub], x);
-        unpack_f16x8(src[sub + LPK], x + 8);
-    } else {
-        const float4* src = reinterpret_cast<const float4*>(p.k + row * (size_t)(D * 4));
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const float4 w = src[sub + j * LPK];
-            x[4 * j] = w.x;
-            x[4 * j + 1] = w.y;
-            x[4 * j + 2] = w.z;
-            x[4 * j + 3] = w.w;
-        }
-    }
-}
-
-// V-side layout of the VALU decode kernel (f32 pools: token-major rows): D/8 lanes per
-// token, lane chunk c holds elements 8c..8c+7.
-template <int DT, int D>
-__device__ __forceinline__ void load_v8(const DecodeParams& p, size_t row, int c, float* x) {
-    static_assert(DT == VSPEC_KV_F32, "the VALU decode kernel serves f32 pools");
-    const float4* src = reinterpret_cast<const float4*>(p.v + row * (size_t)(D * 4));
-    const float4 a = src[2 * c];
-    const float4 b = src[2 * c + 1];
-    x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
-    x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
-}
-
-// Clip a row held by LPK lanes (16 elements each) to +-max(1e-6, alpha*std),
-// then to +-input_clip (three_bit_runtime_modules.c:175-203, :138-173).
-template <int LPK, int D>
-__device__ __forceinline__ void clamp_row(float* x, float alpha, float input_clip) {
-    float s = 0.f;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) s += x[e];
-    const float mean = group_sum<LPK>(s) * (1.0f / D);
-    float v = 0.f;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-        const float d = x[e] - mean;
-        v = fmaf(d, d, v);
-    }
-    const float var = group_sum<LPK>(v) * (1.0f / D);
-    const float th = fminf(fmaxf(1e-6f, alpha * sqrtf(var)), input_clip);
-#pragma unroll
-    for (int e = 0; e < 16; ++e) x[e] = fminf(fmaxf(x[e], -th), th);
-}
-
-template <int DT, int D, int GW>
-__global__ __launch_bounds__(256, 2) void decode_partial(DecodeParams p) {
-    constexpr int LPK = D / 16;           // lanes per key
-    constexpr int KPP = 64 / LPK;         // keys per K pass
-    constexpr int KPASS = kTile / KPP;    // K passes per tile
-    constexpr int VLPT = D / 8;           // lanes per token on the V side
-    constexpr int VTPP = 64 / VLPT;       // tokens per V pass
-    constexpr int VPASS = kTile / VTPP;   // V passes per tile
-    static_assert(KPASS >= 1 && VPASS >= 1, "tile geometry");
-
-    __shared__ float p_lds[kWaves][2][kTile][GW];
-    __shared__ float comb[kWaves][GW][D + 2];
-
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int part = blockIdx.x;
-    const int b = blockIdx.z;
-    const int hk = blockIdx.y / p.gsplit;
-    const int hq0 = hk * (p.gsplit * GW) + (blockIdx.y % p.gsplit) * GW;
-
-    // tiles beyond the block table or the planned partitions are never read
-    const int tiles_per_block = (int)p.block_tokens / kTile;
-    const int ctx = min(max(p.ctx_lens[b], 0), (int)(p.max_blocks * p.block_tokens));
-    const int ntiles = min((ctx + kTile - 1) / kTile, (int)(p.max_parts * p.tiles_per_part));
-    const int nparts = max(1, (ntiles + (int)p.tiles_per_part - 1) / (int)p.tiles_per_part);
-    if (part >= nparts) return;
-    const int tile_begin = part * (int)p.tiles_per_part;
-    const int tile_end = min(ntiles, tile_begin + (int)p.tiles_per_part);
-
-    const int kk = lane / LPK;      // key within a K pass
-    const int sub = lane % LPK;     // lane within the key
-    const int vc = lane % VLPT;     // V chunk
-    const int vt = lane / VLPT;     // token within a V pass
-
-    // q' = clip(q) * scale * log2(e), in the K-side lane layout
-    float qv[GW][16];
-#pragma unroll
-    for (int h = 0; h < GW; ++h) {
-        const float* qrow = p.q + ((size_t)b * p.hq + hq0 + h) * D;
-        float x[16];
-#pragma unroll
-        for (int e = 0; e < 16; ++e) x[e] = qrow[k_elem<DT, D>(sub, e)];
-        clamp_row<LPK, D>(x, p.alpha, p.input_clip);
-#pragma unroll
-        for (int e = 0; e < 16; ++e) qv[h][e] = x[e] * p.qscale;
-    }
-
-    float m_run[GW], l_run[GW], acc[GW][8];
-#pragma unroll
-    for (int h = 0; h < GW; ++h) {
-        m_run[h] = -INFINITY;
-        l_run[h] = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[h][e] = 0.f;
-    }
-
-    const int32_t* table = p.block_tables + (size_t)b * p.max_blocks;
-    int buf = 0;
-    for (int tile = tile_begin + wave; tile < tile_end; tile += kWaves) {
-        const int lblock = tile / tiles_per_block;
-        const int phys = table[lblock];
-        if (phys < 0 || (uint32_t)phys >= p.num_blocks) continue;  // invalid entry: tile skipped
-        const size_t row0 = ((size_t)phys * p.hkv + hk) * p.block_tokens +
-                            (size_t)(tile % tiles_per_block) * kTile;
-        const int tok0 = tile * kTile;
-        // valid slots of this tile: below the context and, with block_used, below its
-        // block's used count (a prefix of the block's slots)
-        const int lim = p.block_used ? min(ctx - tok0, used_cap(p.block_used[(size_t)b * p.max_blocks + lblock],
-                                                                (tile % tiles_per_block) * kTile))
-                                     : ctx - tok0;
-
-        // ---- scores ----
-        float s[KPASS][GW];
-#pragma unroll
-        for (int kp = 0; kp < KPASS; ++kp) {
-            const int slot = kp * KPP + kk;
-            float x[16];
-            load_k16<DT, D>(p, row0 + slot, sub, x);
-            clamp_row<LPK, D>(x, p.alpha, p.input_clip);
-            const bool valid = slot < lim;
-#pragma unroll
-            for (int h = 0; h < GW; ++h) {
-                float d = 0.f;
-#pragma unroll
-                for (int e = 0; e < 16; ++e) d = fmaf(qv[h][e], x[e], d);
-                d = group_sum<LPK>(d);
-                d = fminf(fmaxf(d, -p.logit_clip), p.logit_clip);
-                s[kp][h] = valid ? d : -INFINITY;
-            }
-        }
-
-        // ---- online softmax (rescale only when the max grows by > 2^8) ----
-#pragma unroll
-        for (int h = 0; h < GW; ++h) {
-            float mt = s[0][h];
-#pragma unroll
-            for (int kp = 1; kp < KPASS; ++kp) mt = fmaxf(mt, s[kp][h]);
-            mt = max_across_groups<LPK>(mt);
-            // uniform across the wave after the reduction: keep it in an SGPR
-            mt = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, mt)));
-            if (mt > m_run[h] + 8.0f) {
-                const float f = exp2f(m_run[h] - mt);
-                l_run[h] *= f;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) acc[h][e] *= f;
-                m_run[h] = mt;
-            }
-        }
-#pragma unroll
-        for (int kp = 0; kp < KPASS; ++kp) {
-            if (sub < GW) {
-                float sv = s[kp][0], mv = m_run[0];
-#pragma unroll
-                for (int h = 1; h < GW; ++h) {
-                    if (sub == h) {
-                        sv = s[kp][h];
-                        mv = m_run[h];
-                    }
-                }
-                p_lds[wave][buf][kp * KPP + kk][sub] = exp2f(sv - mv);
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-
-        // ---- P.V ----
-        const bool tail = lim < kTile;
-#pragma unroll
-        for (int vp = 0; vp < VPASS; ++vp) {
-            const int slot = vp * VTPP + vt;
-            float x[8];
-            load_v8<DT, D>(p, row0 + slot, vc, x);
-            if (tail && slot >= lim) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) x[e] = 0.f;
-            }
-            float pv[GW];
-#pragma unroll
-            for (int h = 0; h < GW; ++h) pv[h] = p_lds[wave][buf][slot][h];
-#pragma unroll
-            for (int h = 0; h < GW; ++h) {
-                l_run[h] += pv[h];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) acc[h][e] = fmaf(pv[h], x[e], acc[h][e]);
-            }
-        }
-        buf ^= 1;
-    }
-
-    // ---- reduce the token groups of the V layout (lanes with equal chunk) ----
-#pragma unroll
-    for (int h = 0; h < GW; ++h) {
-#pragma unroll
-        for (int off = VLPT; off < 64; off <<= 1) {
-            l_run[h] += __shfl_xor(l_run[h], off);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) acc[h][e] += __shfl_xor(acc[h][e], off);
-        }
-    }
-    if (lane < VLPT) {
-#pragma unroll
-        for (int h = 0; h < GW; ++h) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) comb[wave][h][2 + 8 * vc + e] = acc[h][e];
-            if (vc == 0) {
-                comb[wave][h][0] = m_run[h];
-                comb[wave][h][1] = l_run[h];
-            }
-        }
-    }
-    __syncthreads();
-
-    // ---- merge the waves of this workgroup ----
-    for (int idx = threadIdx.x; idx < GW * D; idx += 256) {
-        const int h = idx / D;
-        const int d = idx % D;
-        float M = -INFINITY;
-#pragma unroll
-        for (int w = 0; w < kWaves; ++w) M = fmaxf(M, comb[w][h][0]);
-        float a = 0.f, l = 0.f;
-#pragma unroll
-        for (int w = 0; w < kWaves; ++w) {
-            const float mw = comb[w][h][0];
-            if (mw != -INFINITY) {
-                const float f = exp2f(mw - M);
-                a = fmaf(comb[w][h][2 + d], f, a);
-                l = fmaf(comb[w][h][1], f, l);
-            }
-        }
-        const size_t hq = (size_t)b * p.hq + hq0 + h;
-        if (nparts == 1) {
-            p.out[hq * D + d] = l > 0.f ? a / l : 0.f;
-        } else {
-            const size_t slot = hq * p.max_parts + part;
-            p.part_acc[slot * D + d] = a;
-            if (d == 0) {
-                p.part_ml[2 * slot] = M;
-                p.part_ml[2 * slot + 1] = l;
-            }
-        }
-    }
-}
-
-template <int D>
-__global__ __launch_bounds__(D) void decode_combine(DecodeParams p) {
-    const int b = blockIdx.y;
-    const int hq = blockIdx.x;
-    const int d = threadIdx.x;
-    const int ctx = min(max(p.ctx_lens[b], 0), (int)(p.max_blocks * p.block_tokens));
-    const int ntiles = min((ctx + kTile - 1) / kTile, (int)(p.max_parts * p.tiles_per_part));
-    const int nparts = max(1, (ntiles + (int)p.tiles_per_part - 1) / (int)p.tiles_per_part);
-    if (nparts == 1) return;
-    const size_t base = ((size_t)b * p.hq + hq) * p.max_parts;
-    float M = -INFINITY;
-    for (int i = 0; i < nparts; ++i) M = fmaxf(M, p.part_ml[2 * (base + i)]);
-    float a = 0.f, l = 0.f;
-    for (int i = 0; i < nparts; ++i) {
-        const float mi = p.part_ml[2 * (base + i)];
-        if (mi != -INFINITY) {
-            const float f = exp2f(mi - M);
-            a = fmaf(p.part_acc[(base + i) * D + d], f, a);
-            l = fmaf(p.part_ml[2 * (base + i) + 1], f, l);
-        }
-    }
-    p.out[((size_t)b * p.hq + hq) * D + d] = l > 0.f ? a / l : 0.f;
-}
 
 // ---------------------------------------------------------------------------
 // append (quantise-on-write for int4)
@@ -1094,13 +797,54 @@ uint32_t decode_flag_min_tiles() {
     return x >= 0 && x <= 4096 ? (uint32_t)x : kDefaultFlagMinTiles;
 }
 
+// Parts of a work item of f32 pools (always the item split).  Where the host knows every
+// context to be the same, by the same kind of model: a part of n tiles takes n * hypot(0.8, k *
+// 16 KB / 5.9 TB/s) us with k workgroups running.  Else up to three workgroups for each place on
+// the card, of at least 8 tiles: workgroups that end early make room for the others, and an
+// item's parts follow from its own context, not from the host's bound.  *ws_parts:
+// what the workspace is sized for, which never falls as the bound on the contexts rises, so
+// that a workspace for the longest contexts serves every shorter one.
+// Measured at 1 / 2 / 4 / 8 / 16 / 32 parts: 1 x 4097 tokens (8 items) 227 / 122 / 69 / 42 / 29 / 24
+// us, 16 x 2049 (128) 126 / 75 / 56 / 65, 36 x 649-5195 (144, D = 64) 189 / 107 / 76 / 64, 64 x 1025
+// (512) 95 / 107.
+uint32_t plan_f32_parts(uint64_t items, uint64_t tiles, uint32_t head_dim, uint64_t slots, bool same, uint32_t* ws_parts,
+                        uint32_t* part_tiles) {
+    uint64_t most = 4 * slots / items;
+    if (most > (tiles + 3) / 4) most = (tiles + 3) / 4;
+    if (most > 128) most = 128;
+    if (most < 1) most = 1;
+    *ws_parts = (uint32_t)most;
+    const char* e = getenv("VSPEC_ROCM_DECODE_ITEM_PARTS");
+    const long x = e ? strtol(e, nullptr, 10) : 0;
+    if (x > 0) return (uint32_t)((uint64_t)x < most ? (uint64_t)x : most);
+    if (!same) {
+        *part_tiles = 8;
+        const uint64_t p = 3 * slots / items > 1 ? 3 * slots / items : 1, by_tiles = (tiles + 7) / 8;
+        return (uint32_t)(p < most ? (p < by_tiles ? p : by_tiles) : (most < by_tiles ? most : by_tiles));
+    }
+    const double lat = 0.8, bw = 2.75e-3 * head_dim / 128.0;
+    const double busy = sqrt(lat * lat + (double)(slots * slots) * bw * bw);
+    double best = 0;
+    uint32_t parts = 0;
+    for (const uint32_t p : {1u, 2u, 3u, 4u, 6u, 8u, 12u, 16u, 24u, 32u, 48u, 64u, 96u, 128u}) {
+        if (p > most) break;
+        const double full = (double)(items * p / slots), rem = (double)(items * p % slots);
+        const double t = (double)((tiles + p - 1) / p) * (full * busy + (rem > 0 ? sqrt(lat * lat + rem * rem * bw * bw) : 0.0)) +
+                         (p > 1 ? 5.0 + 0.12 * p : 0.0);
+        if (!parts || t < best) {
+            best = t;
+            parts = p;
+        }
+    }
+    return parts;
+}
+
 struct DecodePlan {
     bool merge;  // split MFMA kernels: some work item may span two workgroups (merge launch)
+    uint32_t part_tiles;  // least tiles per part of the item split
     uint32_t item_parts;  // item split (kv_common.h): parts of a work item, 0: ranges of all items' tiles
     uint32_t gw;
     uint32_t gsplit;
-    uint32_t tiles_per_part;
-    uint32_t max_parts;
     size_t ws_bytes;
     // MFMA kernels (f16 / int4 pools): tiles of all work items split over grid_x workgroups
     bool split;
@@ -1186,6 +930,7 @@ int plan_decode(const VspecPagedAttnDesc* d, DecodePlan* pl) {
     const uint32_t max_tiles = (uint32_t)((ctx_bound + kTile - 1) / kTile);
     pl->split = d->kv.dtype != VSPEC_KV_F32;
     pl->item_parts = 0;
+    pl->part_tiles = 4;  // one for each wave
     pl->min_tiles = decode_min_tiles_per_wg((uint64_t)d->batch * hkv * pl->gsplit);
     if (pl->split) {
         // every workgroup streams an equal share of all work items' tiles
@@ -1224,8 +969,6 @@ int plan_decode(const VspecPagedAttnDesc* d, DecodePlan* pl) {
         pl->grid_x = (uint32_t)(grid ? grid : 1);
         pl->split_tiles = bound;
         pl->max_tiles = max_tiles;
-        pl->tiles_per_part = 0;
-        pl->max_parts = 1;
         // unequal pair shares need the grid of two workgroups per CU (g and g + G/2 share one)
         pl->old_permille = !pl->chunk_tiles && pl->grid_x == 2u * (uint32_t)num_cus()
                                ? decode_old_permille(d->kv.dtype) : 500u;
@@ -1241,56 +984,27 @@ int plan_decode(const VspecPagedAttnDesc* d, DecodePlan* pl) {
         pl->ws_bytes = (size_t)pl->grid_x * 2 * pl->gw * (2 + d->kv.head_dim) * sizeof(float);
         return 1;
     }
-    uint32_t tpp;
+    pl->uniform_tiles = 0;
+    pl->max_tiles = max_tiles;
+    pl->item_parts = 1;
+    uint32_t ws_parts = 0;  // the workspace holds this many parts per work item
     if (d->partition_tokens) {
         if (d->partition_tokens % kTile) {
             set_err("paged_decode: partition_tokens must be a multiple of %d", kTile);
             return 0;
         }
-        tpp = d->partition_tokens / kTile;
-    } else {
-        // split each (sequence, kv head) only as far as needed to occupy every resident
-        // workgroup slot once (two 4-wave workgroups per CU at the kernels' register
-        // use); extra partitions only add combine traffic and per-workgroup setup
-        const uint64_t items = (uint64_t)d->batch * hkv * pl->gsplit;
-        const uint64_t target = 2ull * (uint64_t)num_cus();
-        uint64_t parts = items ? (target + items - 1) / items : 1;
-        if (parts < 1) parts = 1;
-        tpp = (uint32_t)((max_tiles + parts - 1) / parts);
-        if (tpp < 16) tpp = 16;
-        tpp = (tpp + kWaves - 1) / kWaves * kWaves;
+        const uint32_t tpp = d->partition_tokens / kTile;
+        if (max_tiles) pl->item_parts = (max_tiles + tpp - 1) / tpp;
+    } else if (d->batch) {
+        pl->item_parts = plan_f32_parts((uint64_t)d->batch * hkv * pl->gsplit, max_tiles ? max_tiles : 1, d->kv.head_dim,
+                                        2ull * (uint64_t)num_cus(), uniform_item_tiles(d, pl, ctx_bound) != 0, &ws_parts,
+                                        &pl->part_tiles);
     }
-    if (tpp == 0) tpp = 1;
-    pl->tiles_per_part = tpp;
-    pl->max_parts = max_tiles ? (max_tiles + tpp - 1) / tpp : 1;
-    if (pl->max_parts == 0) pl->max_parts = 1;
-    pl->ws_bytes = pl->max_parts > 1
-                       ? (size_t)d->batch * d->num_q_heads * pl->max_parts * (2 + d->kv.head_dim) * sizeof(float)
+    if (!ws_parts) ws_parts = pl->item_parts;
+    pl->ws_bytes = ws_parts > 1
+                       ? (size_t)d->batch * d->num_q_heads * ws_parts * (2 + d->kv.head_dim) * sizeof(float)
                        : 0;
     return 1;
-}
-
-template <int DT, int D, int GW>
-void launch_partial(const DecodeParams& p, dim3 grid, hipStream_t s) {
-    hipLaunchKernelGGL((decode_partial<DT, D, GW>), grid, dim3(256), 0, s, p);
-}
-
-template <int DT, int D>
-int dispatch_gw(uint32_t gw, const DecodeParams& p, dim3 grid, hipStream_t s) {
-    switch (gw) {
-        case 1: launch_partial<DT, D, 1>(p, grid, s); return 1;
-        case 2: launch_partial<DT, D, 2>(p, grid, s); return 1;
-        case 3: launch_partial<DT, D, 3>(p, grid, s); return 1;
-        case 4: launch_partial<DT, D, 4>(p, grid, s); return 1;
-        default: return 0;
-    }
-}
-
-template <int DT>
-int dispatch_d(uint32_t d, uint32_t gw, const DecodeParams& p, dim3 grid, hipStream_t s) {
-    if (d == 64) return dispatch_gw<DT, 64>(gw, p, grid, s);
-    if (d == 128) return dispatch_gw<DT, 128>(gw, p, grid, s);
-    return 0;
 }
 
 }  // namespace
@@ -1772,14 +1486,11 @@ int paged_decode(const VspecPagedAttnDesc* desc, const void* k_new, const void* 
     p.q = desc->q;
     p.out = desc->out;
     p.part_ml = (float*)ws;
-    p.part_acc = ws ? (float*)ws + (size_t)desc->batch * desc->num_q_heads * pl.max_parts * 2 : nullptr;
     p.hq = desc->num_q_heads;
     p.hkv = desc->kv.num_kv_heads;
     p.block_tokens = desc->kv.block_tokens;
     p.max_blocks = desc->max_blocks_per_seq;
     p.num_blocks = desc->kv.num_blocks;
-    p.tiles_per_part = pl.tiles_per_part;
-    p.max_parts = pl.max_parts;
     p.gsplit = pl.gsplit;
     p.qscale = scale * kLog2e;
     p.alpha = desc->clamp_alpha > 0.f ? desc->clamp_alpha : 4.5f;
@@ -1789,43 +1500,20 @@ int paged_decode(const VspecPagedAttnDesc* desc, const void* k_new, const void* 
     p.merge = pl.split && pl.merge;
     p.batch = desc->batch;
     p.max_tiles = pl.max_tiles;
-    p.chunk_tiles = pl.chunk_tiles;
-    p.k_new = nullptr;
-    p.v_new = nullptr;
+    p.chunk_tiles = pl.split ? pl.chunk_tiles : 0u;
     p.append_src = src_dtype;
     p.split_old_permille = pl.split ? pl.old_permille : 500u;
     p.uniform_tiles = pl.split ? pl.uniform_tiles : 0u;
     p.min_tiles = pl.split && !pl.chunk_tiles ? pl.min_tiles : 1u;
     p.item_parts = pl.item_parts;
+    p.part_tiles = pl.part_tiles;
     p.seg_cost = !pl.split || pl.chunk_tiles ? 0u
                  : desc->kv.dtype == VSPEC_KV_F16 ? decode_segment_cost()
                  : desc->kv.dtype == VSPEC_KV_INT4 ? decode_segment_cost_int4() : 0u;
 
     hipStream_t s = (hipStream_t)desc->stream;
-    if (k_new) {
-        if (pl.split) {
-            p.k_new = (const uint8_t*)k_new;
-            p.v_new = (const uint8_t*)v_new;
-        } else {
-            AppendParams a = {};
-            a.k = (uint8_t*)desc->kv.k_data;
-            a.v = (uint8_t*)desc->kv.v_data;
-            a.ks = desc->kv.k_scales;
-            a.vs = desc->kv.v_scales;
-            a.block_tables = desc->block_tables;
-            a.ctx_lens = desc->ctx_lens;
-            a.k_new = (const uint8_t*)k_new;
-            a.v_new = (const uint8_t*)v_new;
-            a.batch = desc->batch;
-            a.n_new = 1;
-            a.hkv = desc->kv.num_kv_heads;
-            a.head_dim = desc->kv.head_dim;
-            a.block_tokens = desc->kv.block_tokens;
-            a.max_blocks = desc->max_blocks_per_seq;
-            a.num_blocks = desc->kv.num_blocks;
-            if (!append_launch("paged_decode_step append launch", &desc->kv, a, src_dtype, s)) return 0;
-        }
-    }
+    p.k_new = (const uint8_t*)k_new;
+    p.v_new = (const uint8_t*)v_new;
     if (pl.split) {
         // partial slots [grid][2][GW] of (max, sum) then of acc[D]
         p.part_acc = (float*)ws + (size_t)pl.grid_x * 2 * pl.gw * 2;
@@ -1836,10 +1524,10 @@ int paged_decode(const VspecPagedAttnDesc* desc, const void* k_new, const void* 
         p.part_ml = (float*)ws + (size_t)desc->batch * desc->kv.num_kv_heads * pl.gsplit * pl.item_parts * pl.gw * D;
     }
     const dim3 grid = pl.item_parts ? dim3(desc->kv.num_kv_heads * pl.gsplit * pl.item_parts, desc->batch)
-                      : pl.split ? dim3(pl.grid_x) : dim3(pl.max_parts, desc->kv.num_kv_heads * pl.gsplit, desc->batch);
+                                    : dim3(pl.grid_x);
     int ok = 0;
     switch (desc->kv.dtype) {
-        case VSPEC_KV_F32: ok = dispatch_d<VSPEC_KV_F32>(D, pl.gw, p, grid, s); break;
+        case VSPEC_KV_F32: ok = launch_decode_f32(p, D, pl.gw, grid, s); break;
         case VSPEC_KV_F16:
             ok = D == 64 ? launch_decode_mfma_f16_d64(p, pl.gw, grid, s) : launch_decode_mfma_f16_d128(p, pl.gw, grid, s);
             break;
@@ -1852,12 +1540,6 @@ int paged_decode(const VspecPagedAttnDesc* desc, const void* k_new, const void* 
         return 0;
     }
     HIP_CHECK(hipGetLastError(), "decode launch");
-    if (!pl.split && pl.max_parts > 1) {
-        const dim3 cg(desc->num_q_heads, desc->batch);
-        if (D == 64) hipLaunchKernelGGL(decode_combine<64>, cg, dim3(64), 0, s, p);
-        else hipLaunchKernelGGL(decode_combine<128>, cg, dim3(128), 0, s, p);
-        HIP_CHECK(hipGetLastError(), "decode_combine launch");
-    }
     return 1;
 }
 
