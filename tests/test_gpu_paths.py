@@ -133,7 +133,7 @@ def _same_pools(a, b):
 @pytest.mark.parametrize("lens,Hq,H,D,P,used", [
     ([1], 8, 8, 64, 16, False), ([16, 17, 0, 1], 8, 2, 128, 16, False), ([64, 65, 80, 81, 3], 6, 2, 64, 48, False),
     ([129], 24, 2, 128, 16, False), ([1000, 31, 515], 4, 2, 128, 32, True), ([300] * 5, 16, 4, 64, 16, True),
-    ([4100, 77], 8, 2, 128, 16, False)])
+    ([4100, 77], 8, 2, 128, 16, False), ([130, 33, 700], 32, 2, 128, 16, True), ([47], 8, 1, 64, 48, False)])
 def test_item_split_equals_balanced_split(gpu, monkeypatch, kind, lens, Hq, H, D, P, used):
     """One work item's part per workgroup, for several part counts, against the balanced split:
     the fused step's pool bytes are the same and the outputs differ only by rounding (f16: f32

@@ -765,6 +765,7 @@ int launch_gw(uint32_t gw, const DecodeParams& p, dim3 grid, hipStream_t s) {
         case 2: launch<D, 2>(p, grid, s); return 1;
         case 3: launch<D, 3>(p, grid, s); return 1;
         case 4: launch<D, 4>(p, grid, s); return 1;
+        case 8: launch<D, 8>(p, grid, s); return 1;
         default: return 0;
     }
 }

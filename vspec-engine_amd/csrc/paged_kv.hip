@@ -913,6 +913,12 @@ int plan_decode(const VspecPagedAttnDesc* d, DecodePlan* pl) {
     if (g <= 4) {
         pl->gw = g;
         pl->gsplit = 1;
+    } else if (g % 8 == 0 && d->kv.dtype == VSPEC_KV_F16) {
+        // f16: the score MFMA's 16 columns hold 8 heads as well as 4, so that a tile is read
+        // and multiplied once for all of them (64 x 4097 tokens, 32/4 heads: 172 us with two
+        // items of 4 heads, 142 with the two on one XCD, 89.5 with one of 8)
+        pl->gw = 8;
+        pl->gsplit = g / 8;
     } else if (g % 4 == 0) {
         pl->gw = 4;
         pl->gsplit = g / 4;
