@@ -237,6 +237,10 @@ struct DecodeParams {
     uint32_t block_tokens;
     uint32_t max_blocks;
     uint32_t num_blocks;
+    // item split: parts of a work item (grid (hkv * gsplit * item_parts, batch)), 0: the ranges of
+    // the work split
+    uint32_t item_parts;
+    uint32_t part_tiles;  // least tiles per part, for the first near_parts of them
     uint32_t gsplit;   // work items per kv head (Hq/Hkv/GW)
     float qscale;      // softmax scale * log2(e)
     float alpha;       // std-clamp alpha
@@ -267,9 +271,8 @@ struct DecodeParams {
     // balanced split of a ragged batch: each work item also costs this many tiles (its
     // set-up and merge in every workgroup that starts it), 0: tiles only
     uint32_t seg_cost;
-    // item split: parts of a work item (grid (hkv * gsplit * item_parts, batch)), 0: the ranges above
-    uint32_t item_parts;
-    uint32_t part_tiles;  // least tiles per part
+    uint32_t near_parts;
+    uint32_t far_tiles;  // least tiles per part with more parts
 };
 
 // Launch the decode kernels for f32 pools (decode_f32.hip), f16 pools (decode_mfma.hip) and
@@ -726,13 +729,17 @@ __device__ __forceinline__ void finish_segment(const DecodeParams& p, const floa
 
 // ---------------------------------------------------------------------------
 // Item split (DecodeParams.item_parts): workgroup (y * parts + part, b) takes part `part` of
-// work item y of sequence b.  An item of U tiles is cut into n = min(parts, ceil(U / part_tiles))
-// parts, of tiles [part * U / n, (part + 1) * U / n).  No pass over ctx_lens, no workgroup with two
+// work item y of sequence b.  An item of U tiles is cut into n <= parts parts (item_parts_of),
+// of tiles [part * U / n, (part + 1) * U / n).  No pass over ctx_lens, no workgroup with two
 // items; an item in one part goes straight to the output, and the partial states of the
 // others lie at item * parts + part, where decode_merge_items finds them without redoing a
 // split.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ int item_parts_of(const DecodeParams& p, int U) { return min((int)p.item_parts, (U + (int)p.part_tiles - 1) / (int)p.part_tiles); }
+__device__ __forceinline__ int item_parts_of(const DecodeParams& p, int U) {
+    const uint32_t u = (uint32_t)U;
+    const uint32_t near = min(p.near_parts, (u + p.part_tiles - 1) / p.part_tiles);
+    return (int)min(p.item_parts, max(near, (u + p.far_tiles - 1) / p.far_tiles));
+}
 
 // this workgroup's item (tile positions count from the item's first tile) and tiles [lo, hi);
 // lo = hi when it has none; slot: the part's partial state
@@ -767,9 +774,12 @@ __device__ __forceinline__ ItemCursor item_part(const DecodeParams& p, int& lo, 
     c.b = __builtin_amdgcn_readfirstlane((int)b);
     c.y = (int)(x * p.gsplit + g);
     c.U = item_tiles(p, c.b);
-    const int n = item_parts_of(p, c.U);
-    const int l = (int)part < n ? (int)(part * (uint32_t)c.U / (uint32_t)n) : 0;
-    const int h = (int)part < n ? (int)((part + 1) * (uint32_t)c.U / (uint32_t)n) : 0;
+    int l = 0, h = c.U;
+    if (p.item_parts > 1) {
+        const uint32_t n = (uint32_t)item_parts_of(p, c.U);
+        l = part < n ? (int)(part * (uint32_t)c.U / n) : 0;
+        h = part < n ? (int)((part + 1) * (uint32_t)c.U / n) : 0;
+    }
     // wave-uniform values on the scalar unit (the divisions run on the vector one)
     c.y = __builtin_amdgcn_readfirstlane(c.y);
     c.U = __builtin_amdgcn_readfirstlane(c.U);

@@ -797,18 +797,41 @@ uint32_t decode_flag_min_tiles() {
     return x >= 0 && x <= 4096 ? (uint32_t)x : kDefaultFlagMinTiles;
 }
 
+struct DecodePlan {
+    bool merge;  // split MFMA kernels: some work item may span two workgroups (merge launch)
+    uint32_t part_tiles;  // item split: least tiles per part, for the first near_parts of them
+    uint32_t near_parts;
+    uint32_t far_tiles;  // least tiles per part with more parts
+    uint32_t item_parts;  // item split (kv_common.h): parts of a work item, 0: ranges of all items' tiles
+    uint32_t gw;
+    uint32_t gsplit;
+    size_t ws_bytes;
+    // MFMA kernels (f16 / int4 pools): tiles of all work items split over grid_x workgroups
+    bool split;
+    uint32_t grid_x;
+    uint32_t chunk_tiles;
+    uint64_t split_tiles;  // tiles the balanced split spreads over grid_x (upper bound)
+    uint32_t min_tiles;    // least tiles per workgroup of the balanced split
+    uint32_t max_tiles;
+    uint32_t old_permille;  // pair share of the first-half workgroups (500: equal shares)
+    uint32_t uniform_tiles; // tiles per work item when every context is known to be the same
+};
+
 // Parts of a work item of f32 pools (always the item split).  Where the host knows every
 // context to be the same, by the same kind of model: a part of n tiles takes n * hypot(0.8, k *
-// 16 KB / 5.9 TB/s) us with k workgroups running.  Else up to three workgroups for each place on
-// the card, of at least 8 tiles: workgroups that end early make room for the others, and an
-// item's parts follow from its own context, not from the host's bound.  *ws_parts:
+// 16 KB / 5.9 TB/s) us with k workgroups running.  Else an item's parts follow from its own
+// context, not from the host's bound: enough workgroups of at least 8 tiles to fill the card
+// once, and where that cuts an item in fewer than 6, up to three times as many of at least 16
+// tiles, so that the longest context's parts do not outlast the others (36 x 649-5195 tokens,
+// 144 items: 76 us with 3 parts, 61 with 10; 8 x 773-4188, 64 items: 49 us with 8, 56-66 with
+// more; 35 x 128-1024: 25 us, 31 in parts of 8 tiles).  *ws_parts:
 // what the workspace is sized for, which never falls as the bound on the contexts rises, so
 // that a workspace for the longest contexts serves every shorter one.
 // Measured at 1 / 2 / 4 / 8 / 16 / 32 parts: 1 x 4097 tokens (8 items) 227 / 122 / 69 / 42 / 29 / 24
 // us, 16 x 2049 (128) 126 / 75 / 56 / 65, 36 x 649-5195 (144, D = 64) 189 / 107 / 76 / 64, 64 x 1025
 // (512) 95 / 107.
 uint32_t plan_f32_parts(uint64_t items, uint64_t tiles, uint32_t head_dim, uint64_t slots, bool same, uint32_t* ws_parts,
-                        uint32_t* part_tiles) {
+                        DecodePlan* pl) {
     uint64_t most = 4 * slots / items;
     if (most > (tiles + 3) / 4) most = (tiles + 3) / 4;
     if (most > 128) most = 128;
@@ -818,9 +841,14 @@ uint32_t plan_f32_parts(uint64_t items, uint64_t tiles, uint32_t head_dim, uint6
     const long x = e ? strtol(e, nullptr, 10) : 0;
     if (x > 0) return (uint32_t)((uint64_t)x < most ? (uint64_t)x : most);
     if (!same) {
-        *part_tiles = 8;
-        const uint64_t p = 3 * slots / items > 1 ? 3 * slots / items : 1, by_tiles = (tiles + 7) / 8;
-        return (uint32_t)(p < most ? (p < by_tiles ? p : by_tiles) : (most < by_tiles ? most : by_tiles));
+        pl->part_tiles = 8;
+        if (items * 6 > slots) pl->far_tiles = 16;
+        pl->near_parts = (uint32_t)(slots / items > 1 ? slots / items : 1);
+        const uint64_t far_parts = items * 6 > slots ? (3 * slots / items > 1 ? 3 * slots / items : 1) : 1;
+        const uint64_t near = (tiles + 7) / 8 < pl->near_parts ? (tiles + 7) / 8 : pl->near_parts;
+        const uint64_t far = (tiles + 15) / 16 < far_parts ? (tiles + 15) / 16 : far_parts;
+        const uint64_t p = near > far ? near : far;
+        return (uint32_t)(p < most ? p : most);
     }
     const double lat = 0.8, bw = 2.75e-3 * head_dim / 128.0;
     const double busy = sqrt(lat * lat + (double)(slots * slots) * bw * bw);
@@ -839,23 +867,6 @@ uint32_t plan_f32_parts(uint64_t items, uint64_t tiles, uint32_t head_dim, uint6
     return parts;
 }
 
-struct DecodePlan {
-    bool merge;  // split MFMA kernels: some work item may span two workgroups (merge launch)
-    uint32_t part_tiles;  // least tiles per part of the item split
-    uint32_t item_parts;  // item split (kv_common.h): parts of a work item, 0: ranges of all items' tiles
-    uint32_t gw;
-    uint32_t gsplit;
-    size_t ws_bytes;
-    // MFMA kernels (f16 / int4 pools): tiles of all work items split over grid_x workgroups
-    bool split;
-    uint32_t grid_x;
-    uint32_t chunk_tiles;
-    uint64_t split_tiles;  // tiles the balanced split spreads over grid_x (upper bound)
-    uint32_t min_tiles;    // least tiles per workgroup of the balanced split
-    uint32_t max_tiles;
-    uint32_t old_permille;  // pair share of the first-half workgroups (500: equal shares)
-    uint32_t uniform_tiles; // tiles per work item when every context is known to be the same
-};
 
 // With every context known to be the same (min_ctx_len == the context bound), the split
 // of the MFMA kernels (kv_common.h work_split with equal shares, as for any batch whose
@@ -937,9 +948,11 @@ int plan_decode(const VspecPagedAttnDesc* d, DecodePlan* pl) {
     pl->split = d->kv.dtype != VSPEC_KV_F32;
     pl->item_parts = 0;
     pl->part_tiles = 4;  // one for each wave
-    pl->min_tiles = decode_min_tiles_per_wg((uint64_t)d->batch * hkv * pl->gsplit);
+    pl->near_parts = 0x7fffffffu;
+    pl->far_tiles = 0x40000000u;
     if (pl->split) {
         // every workgroup streams an equal share of all work items' tiles
+        pl->min_tiles = decode_min_tiles_per_wg((uint64_t)d->batch * hkv * pl->gsplit);
         const uint64_t bound = (uint64_t)d->batch * hkv * pl->gsplit * (max_tiles ? max_tiles : 1);
         if (bound > (uint64_t)INT32_MAX) {
             set_err("paged_decode: batch * work items * tiles exceeds 2^31");
@@ -1004,7 +1017,7 @@ int plan_decode(const VspecPagedAttnDesc* d, DecodePlan* pl) {
     } else if (d->batch) {
         pl->item_parts = plan_f32_parts((uint64_t)d->batch * hkv * pl->gsplit, max_tiles ? max_tiles : 1, d->kv.head_dim,
                                         2ull * (uint64_t)num_cus(), uniform_item_tiles(d, pl, ctx_bound) != 0, &ws_parts,
-                                        &pl->part_tiles);
+                                        pl);
     }
     if (!ws_parts) ws_parts = pl->item_parts;
     pl->ws_bytes = ws_parts > 1
@@ -1513,6 +1526,8 @@ int paged_decode(const VspecPagedAttnDesc* desc, const void* k_new, const void* 
     p.min_tiles = pl.split && !pl.chunk_tiles ? pl.min_tiles : 1u;
     p.item_parts = pl.item_parts;
     p.part_tiles = pl.part_tiles;
+    p.near_parts = pl.near_parts;
+    p.far_tiles = pl.far_tiles;
     p.seg_cost = !pl.split || pl.chunk_tiles ? 0u
                  : desc->kv.dtype == VSPEC_KV_F16 ? decode_segment_cost()
                  : desc->kv.dtype == VSPEC_KV_INT4 ? decode_segment_cost_int4() : 0u;
