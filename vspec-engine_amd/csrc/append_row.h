@@ -51,8 +51,7 @@ constexpr int append_ept(int dt) { return dt == VSPEC_KV_INT4 ? 32 : 8; }
 // Chunk c of the token-head row of K (which 0) or V (which 1) whose first source element
 // is src_el, written at position pos of block-table row `seq`, kv head h.  Positions past
 // the table, behind an invalid entry or (with rotary tables) past max_pos are not written.
-// A clamp-flag update held back by the caller: flag word `word` gets bit `bit` set or
-// cleared.
+// A clamp-flag update: flag word `word` gets bit `bit` set or cleared.
 struct FlagOp {
     uint32_t* word;
     uint32_t bit;
@@ -67,19 +66,17 @@ __device__ __forceinline__ void apply_flag(const FlagOp& f) {
 
 // int4 codec of one 32-element group: rep = 2nd-largest |x|, scale = rep/8 (1 if rep == 0),
 // floored at 1e-6, rounded to fp16 (saturating), codes rint(x/scale) in [-8,7]; element e
-// in nibble e%8 of w[e/8].  c1, c2, cm: sum, sum of squares and largest magnitude of the
-// codes.
+// in nibble e%8 of w[e/8].  top: the code of the largest |x|, as a positive value.
 struct Int4Group {
     uint32_t w[4];
     uint32_t s16;
     float sc;
-    int c1, c2, cm;
+    int top;
 };
-// the largest two |x| seen (a1 >= a2; equal values count twice), updated with a
+// the largest two |x| seen (a1 >= a2; equal values count twice, NaN not at all), updated with a
 __device__ __forceinline__ void int4_top2(float a, float& a1, float& a2) {
-    const bool gt1 = a > a1;
-    a2 = gt1 ? a1 : (a > a2 ? a : a2);
-    a1 = gt1 ? a : a1;
+    a2 = fminf(a1, fmaxf(a2, a));
+    a1 = fmaxf(a1, a);
 }
 // fp16 bits of a group's scale from its 2nd-largest |x|
 __device__ __forceinline__ uint32_t int4_scale_bits(float rep) {
@@ -93,6 +90,19 @@ __device__ __forceinline__ int int4_code(float x, float sc) {
     const float rr = rintf(x / sc);
     return rr > 7.0f ? 7 : (rr >= -8.0f ? (int)rr : -8);
 }
+// The same code as a two's complement nibble, for many elements of one scale: inv is 1 / sc
+// correctly rounded, and two Newton steps with exact remainders (Markstein) give x / sc correctly
+// rounded, 5 operations instead of a division's 10 or so.  x is held within 16 scales first: the
+// code is the same, nothing overflows, and NaN goes to -8 as above.  Adding 1.5 * 2^23 rounds to
+// the nearest even integer, whose low bits are the code's.
+__device__ __forceinline__ uint32_t int4_nibble(float x, float sc, float inv) {
+    const float lim = 16.0f * sc;
+    const float xc = fminf(fmaxf(x, -lim), lim);
+    const float q0 = xc * inv;
+    const float q1 = fmaf(fmaf(-q0, sc, xc), inv, q0);
+    const float q = fmaf(fmaf(-q1, sc, xc), inv, q1);
+    return __builtin_bit_cast(uint32_t, fminf(fmaxf(q, -8.0f), 7.0f) + 12582912.0f) & 0xfu;
+}
 __device__ __forceinline__ Int4Group int4_encode_group(const float (&x)[32]) {
     float a1 = 0.f, a2 = 0.f;
 #pragma unroll
@@ -100,17 +110,33 @@ __device__ __forceinline__ Int4Group int4_encode_group(const float (&x)[32]) {
     Int4Group q;
     q.s16 = int4_scale_bits(a2);
     q.sc = half_bits_to_float(q.s16);
+    const float inv = 1.0f / q.sc;
     q.w[0] = q.w[1] = q.w[2] = q.w[3] = 0u;
-    q.c1 = q.c2 = q.cm = 0;
 #pragma unroll
-    for (int e = 0; e < 32; ++e) {
-        const int code = int4_code(x[e], q.sc);
-        q.w[e / 8] |= ((uint32_t)code & 0xfu) << (4 * (e % 8));
-        q.c1 += code;
-        q.c2 += code * code;
-        q.cm = max(q.cm, code < 0 ? -code : code);
-    }
+    for (int e = 0; e < 32; ++e) q.w[e / 8] |= int4_nibble(x[e], q.sc, inv) << (4 * (e % 8));
+    q.top = (int)int4_nibble(a1, q.sc, inv);
     return q;
+}
+// sum, sum of squares and largest magnitude of a group's codes
+__device__ __forceinline__ void int4_code_sums(const Int4Group& q, int& c1, int& c2, int& cm) {
+    c1 = c2 = 0;
+    uint32_t m8 = 0;  // nibbles that hold -8
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t w = q.w[i];
+#if defined(__HIP_DEVICE_COMPILE__)
+        c1 = __builtin_amdgcn_sdot8((int)w, 0x11111111, c1, false);
+        c2 = __builtin_amdgcn_sdot8((int)w, (int)w, c2, false);
+#else
+        for (int e = 0; e < 8; ++e) {
+            const int code = (int32_t)(w << (28 - 4 * e)) >> 28;
+            c1 += code;
+            c2 += code * code;
+        }
+#endif
+        m8 |= w & ~(w << 1) & ~(w << 2) & ~(w << 3) & 0x88888888u;
+    }
+    cm = m8 ? 8 : q.top;
 }
 
 // The clamp flag of a key from its row's sums: s1 = sum x, s2 = sum x^2 (the groups' scaled
@@ -130,9 +156,11 @@ __device__ __forceinline__ bool int4_flag_from_sums(float s1, float s2, float m,
 // append work items of one row: all of these lanes call this together); the 2^-10 margins
 // cover the one-pass variance (the decode kernel's screen test, run once per key here).
 __device__ __forceinline__ bool int4_key_flag(const Int4Group& q, uint32_t head_dim) {
-    float s1 = q.sc * (float)q.c1;
-    float s2 = (q.sc * q.sc) * (float)q.c2;
-    float m = q.sc * (float)q.cm;
+    int c1, c2, cm;
+    int4_code_sums(q, c1, c2, cm);
+    float s1 = q.sc * (float)c1;
+    float s2 = (q.sc * q.sc) * (float)c2;
+    float m = q.sc * (float)cm;
     for (uint32_t o = 2; o < 2 * (head_dim / 32); o <<= 1) {
         s1 += __shfl_xor(s1, (int)o);
         s2 += __shfl_xor(s2, (int)o);
@@ -175,7 +203,7 @@ __device__ __forceinline__ void load_elements(const uint8_t* src, size_t el, flo
 // ROPE: the launch may carry rotary tables (without it their code and registers go)
 template <int DT, int SRC, bool ROPE = true>
 __device__ __forceinline__ void append_chunk(const AppendParams& p, uint32_t seq, uint32_t pos, uint32_t h,
-                                             uint32_t c, int which, size_t src_el, FlagOp* defer = nullptr) {
+                                             uint32_t c, int which, size_t src_el) {
     constexpr int EPT = append_ept(DT);
     const uint32_t lb = pos / p.block_tokens;
     if (lb >= p.max_blocks) return;
@@ -274,8 +302,7 @@ __device__ __forceinline__ void append_chunk(const AppendParams& p, uint32_t seq
             if (c == 0) {
                 const FlagOp op = {p.kf + ((size_t)phys * p.hkv + h) * (p.block_tokens / 16) + slot / 16,
                                    1u << (slot % 16), flag};
-                if (defer) *defer = op;
-                else apply_flag(op);
+                apply_flag(op);
             }
         }
         const size_t bh = (size_t)phys * p.hkv + h;
@@ -292,41 +319,6 @@ __device__ __forceinline__ void append_chunk(const AppendParams& p, uint32_t seq
             p.ks[int4_ks_index(bh, p.head_dim / 32, p.block_tokens, slot, c)] = (uint16_t)q.s16;
         }
     }
-}
-
-// The append of a decode kernel's fused decode step: each sequence's new token at position
-// ctx_lens[b] - 1.
-__device__ __forceinline__ AppendParams decode_step_append_params(const DecodeParams& p, uint32_t head_dim) {
-    AppendParams a;
-    a.k = const_cast<uint8_t*>(p.k);
-    a.v = const_cast<uint8_t*>(p.v);
-    a.ks = const_cast<uint16_t*>(p.ks);
-    a.vs = const_cast<uint16_t*>(p.vs);
-    a.kf = const_cast<uint32_t*>(p.kf);
-    a.block_tables = p.block_tables;
-    a.start_pos = nullptr;
-    a.token_item = nullptr;
-    a.token_pos = nullptr;
-    a.n_items = 0;
-    a.rope_cos = nullptr;
-    a.rope_sin = nullptr;
-    a.rope_dim = 0;
-    a.max_pos = 0;
-    a.rope_vec = false;
-    a.q_in = nullptr;
-    a.q_out = nullptr;
-    a.hq = 0;
-    a.ctx_lens = p.ctx_lens;
-    a.k_new = p.k_new;
-    a.v_new = p.v_new;
-    a.batch = p.batch;
-    a.n_new = 1;
-    a.hkv = p.hkv;
-    a.head_dim = head_dim;
-    a.block_tokens = p.block_tokens;
-    a.max_blocks = p.max_blocks;
-    a.num_blocks = p.num_blocks;
-    return a;
 }
 
 // Work items of one append launch: 2 (K, V) x chunks per row x kv heads x tokens.
@@ -529,65 +521,6 @@ __device__ __forceinline__ void rope_q_item(const AppendParams& p, uint32_t it) 
                                       x[h].z * cv.z - y[h].z * sv.z, x[h].w * cv.w - y[h].w * sv.w);
         out[h * d4 + c + half / 4] = make_float4(x[h].x * sv.x + y[h].x * cv.x, x[h].y * sv.y + y[h].y * cv.y,
                                                  x[h].z * sv.z + y[h].z * cv.z, x[h].w * sv.w + y[h].w * cv.w);
-    }
-}
-
-// Fused decode-step append of the MFMA decode kernels (p.k_new != null).  Every work
-// item whose last tile lies in this workgroup's range [ws.lo, ws.hi) -- exactly one
-// workgroup per work item -- gets its sequence's new token written for its kv head at
-// position ctx_lens[b] - 1, exactly as the append kernel writes it.  Threads below kItems
-// (the first lanes of wave 0) write the rows: with WAIT every thread calls this (it ends in a
-// barrier), without WAIT at least those, before the workgroup reads any tile the append may
-// write.  WAIT: it returns with the
-// stores complete and a barrier passed, so the workgroup's later loads of those tiles see
-// them; without WAIT it returns with the stores issued, and the caller waits for them (every
-// thread) and passes a barrier before such loads.  Other workgroups never read the rows
-// written here (they belong to the item's last tile), except the owners of the other
-// q-head groups of the same kv head, which write the same bytes themselves.
-template <int DT, int D, bool WAIT = true>
-__device__ void fused_append(const DecodeParams& p, const WorkSplit& ws, ItemCursor c, const int ips,
-                             FlagOp& pending, uint32_t* pend_lds) {
-    constexpr int EPT = append_ept(DT);
-    constexpr int kItems = D / EPT * 2;  // append work items per token-head row (K and V)
-    static_assert(kItems <= kWaves * 64, "one pass of the workgroup's threads");
-    const AppendParams a = decode_step_append_params(p, D);
-    const int t = (int)threadIdx.x;
-    // int4 clamp flags (thread 0 of each row): the first one is handed back to the caller,
-    // which applies it after the barrier below (so the barrier does not wait for it) and,
-    // with pend_lds, is published there as {word index, bit, set} for the tile loop to patch
-    // into the word it loads; any further ones are applied at once
-    pending = {nullptr, 0u, false};
-    while (true) {
-        const int last = c.item0 + c.U - 1;
-        if (last >= ws.lo && last < ws.hi) {
-            const int ctx = as_const(p.ctx_lens)[c.b];
-            if (ctx > 0 && t < kItems) {
-                const uint32_t hk = (uint32_t)c.y / p.gsplit;
-                const uint32_t ch = (uint32_t)t >> 1;
-                const size_t src_el = ((size_t)c.b * p.hkv + hk) * D + (size_t)ch * EPT;
-                FlagOp op = {nullptr, 0u, false};
-                if (p.append_src == VSPEC_KV_F32) {
-                    append_chunk<DT, VSPEC_KV_F32>(a, (uint32_t)c.b, (uint32_t)ctx - 1u, hk, ch, t & 1, src_el, &op);
-                } else {
-                    append_chunk<DT, VSPEC_KV_F16>(a, (uint32_t)c.b, (uint32_t)ctx - 1u, hk, ch, t & 1, src_el, &op);
-                }
-                if (op.word) {
-                    if (!pending.word) pending = op;
-                    else apply_flag(op);
-                }
-            }
-        }
-        if (c.item0 + c.U >= ws.hi) break;
-        cursor_next(p, ips, c);
-    }
-    if (pend_lds && t == 0) {
-        pend_lds[0] = pending.word ? (uint32_t)(pending.word - p.kf) : 0xffffffffu;
-        pend_lds[1] = pending.bit;
-        pend_lds[2] = pending.set ? pending.bit : 0u;
-    }
-    if constexpr (WAIT) {
-        __builtin_amdgcn_s_waitcnt(0);  // this thread's stores are done
-        __syncthreads();
     }
 }
 

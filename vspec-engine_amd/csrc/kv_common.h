@@ -820,6 +820,10 @@ __device__ __forceinline__ void finish_item(const DecodeParams& p, const float (
     }
 }
 
+// a partial state's max (log2 units) and sum
+struct alignas(8) MaxSum {
+    float m, l;
+};
 // Merge launch of an item split, one workgroup per work item (grid = (hkv * gsplit, batch)):
 // a lane takes 4 outputs of one head and every PS-th part; the PS sets meet in LDS.
 template <int D, int GW>
@@ -829,7 +833,7 @@ __global__ __launch_bounds__(256) void decode_merge_items(DecodeParams p) {
     constexpr int NBATCH = 4;
     static_assert(Q * PS <= 256, "lanes");
     __shared__ float4 sa[PS][Q];
-    __shared__ float2 sml[PS][Q];
+    __shared__ MaxSum sml[PS][Q];
     const int b = (int)blockIdx.y, y = (int)blockIdx.x;
     const int n = item_parts_of(p, item_tiles(p, b));
     if (n <= 1) return;  // written by the split kernel
@@ -837,7 +841,7 @@ __global__ __launch_bounds__(256) void decode_merge_items(DecodeParams p) {
     const int h = 4 * o / D;
     const size_t slot0 = ((size_t)b * gridDim.x + y) * p.item_parts;
     const float4* acc = reinterpret_cast<const float4*>(p.part_acc) + slot0 * Q + o;
-    const float2* ml = reinterpret_cast<const float2*>(p.part_ml) + slot0 * GW + h;
+    const MaxSum* ml = reinterpret_cast<const MaxSum*>(p.part_ml) + slot0 * GW + h;
     // -1e30 (not -inf) keeps exp2 finite
     float M = -1e30f, L = 0.f;
     float4 A = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -852,7 +856,7 @@ __global__ __launch_bounds__(256) void decode_merge_items(DecodeParams p) {
         M = nm;
     };
     for (int i = ps; ps < PS && i < n; i += PS * NBATCH) {
-        float2 mlv[NBATCH];
+        MaxSum mlv[NBATCH];
         float4 av[NBATCH];
 #pragma unroll
         for (int k = 0; k < NBATCH; ++k) {
@@ -862,19 +866,19 @@ __global__ __launch_bounds__(256) void decode_merge_items(DecodeParams p) {
         }
 #pragma unroll
         for (int k = 0; k < NBATCH; ++k) {
-            if (i + k * PS < n) add(mlv[k].x, mlv[k].y, av[k]);
+            if (i + k * PS < n) add(mlv[k].m, mlv[k].l, av[k]);
         }
     }
     if (ps > 0 && ps < PS) {
         sa[ps][o] = A;
-        sml[ps][o] = make_float2(M, L);
+        sml[ps][o] = MaxSum{M, L};
     }
     __syncthreads();
     if (ps != 0) return;
 #pragma unroll
     for (int s = 1; s < PS; ++s) {
         if (s >= n) break;  // (sets past the parts are empty)
-        add(sml[s][o].x, sml[s][o].y, sa[s][o]);
+        add(sml[s][o].m, sml[s][o].l, sa[s][o]);
     }
     reinterpret_cast<float4*>(p.out + ((size_t)b * p.hq + (size_t)y * GW) * D)[o] =
         L > 0.f ? make_float4(A.x / L, A.y / L, A.z / L, A.w / L) : make_float4(0.f, 0.f, 0.f, 0.f);
