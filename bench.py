@@ -715,7 +715,7 @@ def main():
                      "frac": achieved / PEAK_GBS, "traffic": traffic,
                      "kernel": ("kv_append + " if args.separate_append else "") +
                                {"f16": "decode_mfma_f16", "int4": "decode_mfma_i4",
-                                "f32": "decode_partial" + (" + decode_combine" if ws_bytes else "")}[wl["dtype"]],
+                                "f32": "decode_f32" + (" + decode_merge_items" if ws_bytes else "")}[wl["dtype"]],
                      "algorithmic_bytes_per_launch": alg,
                      "tiles_per_launch": tiles_per_launch(lens, Hq, Hkv)},
     }
