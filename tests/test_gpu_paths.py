@@ -204,3 +204,93 @@ def test_f32_step_parts(gpu, monkeypatch, lens, Hq, H, D, P, used, src):
             got = vr.paged_decode_step(pools[1], tables, ctx, q, *new, numerics=numerics, **hint)
             assert _same_pools(*pools)
             assert float((got - want).abs().max()) <= 6e-6
+
+
+def _attend_valid(vr, pool, tables, spans, used, q, numerics):
+    """Decode attention in 64 bits over the rows that the pool holds at the valid slots (read
+    back as fp32 rows by kv_gather_rows)."""
+    import ctypes as C
+    import torch
+
+    P, three = pool.block_tokens, numerics == vr.NUMERICS_3BIT
+    H, D = pool.num_kv_heads, pool.head_dim
+
+    def limited(x):
+        th = (4.5 * x.std(-1, correction=0, keepdim=True)).clamp(min=1e-6)
+        th = th.clamp(max=16.0) if three else th
+        return x.clamp(-th, th)
+
+    tab, use, out = tables.cpu(), used.cpu(), torch.zeros(q.shape, dtype=torch.float64)
+    for b, span in enumerate(spans):
+        at = [t for t in range(span) if t % P < int(use[b, t // P])]
+        if not at:
+            continue
+        pages = torch.tensor([int(tab[b, t // P]) for t in at], dtype=torch.int32, device=q.device)
+        slots = torch.tensor([t % P for t in at], dtype=torch.int32, device=q.device)
+        k, v = (torch.empty((len(at), H, D), device=q.device) for _ in range(2))
+        assert vr.lib().vspec_rocm_kv_gather_rows(C.byref(pool.desc()), len(at), pages.data_ptr(), slots.data_ptr(), k.data_ptr(),
+                                                  v.data_ptr(), torch.cuda.current_stream().cuda_stream), vr.last_error()
+        kc, vc, qc = limited(k.cpu().double()), v.cpu().double(), limited(q[b].cpu().double())
+        for h in range(q.shape[1]):
+            s = kc[:, h // (q.shape[1] // H)] @ qc[h] / D ** 0.5
+            s = s.clamp(-24, 24) if three else s
+            out[b, h] = s.softmax(0) @ vc[:, h // (q.shape[1] // H)]
+    return out
+
+
+@pytest.mark.parametrize("kind", ["f32", "f16", "int4"])
+@pytest.mark.parametrize("Hq,H,D,P,blocks", [
+    # used tokens of each block, the last one's span; tiles without a valid slot as a wave's only
+    # tile, as its first of two, as a whole part, and as a whole sequence
+    (8, 2, 128, 32, [[10, 32], [32, 16, 32, 3], [0, 0], [1]]), (8, 8, 64, 48, [[48, 5, 0, 48, 48, 20], [16, 47]]),
+    (6, 2, 64, 16, [[0, 16, 0, 16, 3], [16, 0, 0, 0, 16, 16, 16, 16, 1], [0]]), (32, 4, 128, 64, [[5, 64, 64, 9, 64, 64, 40]])])
+def test_decode_skips_tiles_without_valid_slots(gpu, monkeypatch, kind, Hq, H, D, P, blocks):
+    """block_used counts that leave whole tiles empty, for several splits, against 64-bit
+    attention over the valid rows (2e-5: the bar of the parity tests for f32 and f16; int4 also
+    rounds each weight x scale once to fp16, 2^-12 of |v| < 8)."""
+    import torch
+
+    n = max(len(b) for b in blocks)
+    spans = [(len(b) - 1) * P + b[-1] for b in blocks]
+    vr, pools, tables, ctx, q, new, _ = _decode_setup(gpu, kind, [n * P] * len(blocks), Hq, H, D, P)
+    used = torch.tensor([b + [0] * (n - len(b)) for b in blocks], dtype=torch.int32, device=gpu)
+    ctx = torch.tensor(spans, dtype=torch.int32, device=gpu)
+    tol = 8 * 2.0 ** -12 if kind == "int4" else 2e-5
+    for numerics in (vr.NUMERICS_PLAIN, vr.NUMERICS_3BIT):
+        want = _attend_valid(vr, pools[0], tables, spans, used, q, numerics)
+        for parts in ("", "0", "1", "2", "5"):
+            if parts:
+                monkeypatch.setenv("VSPEC_ROCM_DECODE_ITEM_PARTS", parts)
+            else:
+                monkeypatch.delenv("VSPEC_ROCM_DECODE_ITEM_PARTS", raising=False)
+            got = vr.paged_decode(pools[0], tables, ctx, q, numerics=numerics, block_used=used)
+            assert float((got.cpu().double() - want).abs().max()) <= tol, (numerics, parts)
+        # the step: each live sequence's last token replaced first
+        monkeypatch.delenv("VSPEC_ROCM_DECODE_ITEM_PARTS")
+        vr.paged_decode_step(pools[1], tables, ctx, q, *new, numerics=numerics, block_used=used)
+        want = _attend_valid(vr, pools[1], tables, spans, used, q, numerics)
+        got = vr.paged_decode_step(pools[1], tables, ctx, q, *new, numerics=numerics, block_used=used)
+        assert float((got.cpu().double() - want).abs().max()) <= tol, numerics
+
+
+@pytest.mark.parametrize("parts", ["1", "2"])
+def test_f32_scores_far_below_zero(gpu, monkeypatch, parts):
+    """f32 pools, plain numerics, every score below -1e30: the waves and the parts keep their
+    relative weights (tokens of tile 2 score -8e32, the others twice that: the output is
+    the mean of tile 2's V rows, up to 16 roundings of |v| < 6)."""
+    import torch
+    import vspec_rocm as vr
+
+    monkeypatch.setenv("VSPEC_ROCM_DECODE_ITEM_PARTS", parts)
+    T, D = 128, 64
+    g = torch.Generator(device=gpu).manual_seed(3)
+    u = torch.randint(0, 2, (D,), generator=g, device=gpu).float() * 2 - 1
+    k = 2e16 * u.repeat(1, T, 1, 1)  # [1][T][1][D]
+    k[:, 32:48] *= 0.5
+    v = torch.randn((1, T, 1, D), generator=g, device=gpu)
+    pool = vr.PagedPool(vr.KV_F32, T // 16, 16, 1, D, device=gpu)
+    tables = torch.arange(T // 16, dtype=torch.int32).view(1, -1)
+    vr.kv_append(pool, tables, torch.zeros(1, dtype=torch.int32), k, v)
+    out = vr.paged_decode(pool, tables, torch.tensor([T], dtype=torch.int32), (-1e16 * u).view(1, 1, D).contiguous())
+    want = v[0, 32:48, 0].double().mean(0)
+    assert float((out[0, 0].double() - want).abs().max()) <= 16 * 2.0 ** -24 * 6

@@ -148,6 +148,7 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
         // block's used count (a prefix of the block's slots)
         const int lim = p.block_used ? min(ctx - tok0, used_cap(as_const(p.block_used)[(size_t)c.b * p.max_blocks + lblock], slot0))
                                      : ctx - tok0;
+        if (lim <= 0) continue;  // (without a valid slot the weights would be exp2(-inf + inf))
 
         // V goes out with K where a wave's chain of round trips, not the memory rate, is what
         // it waits for: one tile per wave (89 x 1-26 tokens 19.2 -> 17.4 us), and 64-element
@@ -267,7 +268,7 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) comb[wave][h][2 + 8 * vc + e] = acc[h][e];
             if (vc == 0) {
-                comb[wave][h][0] = fmaxf(m_run[h], -1e30f);  // (finite: a wave without tokens)
+                comb[wave][h][0] = m_run[h];  // (-inf: a wave without tokens)
                 comb[wave][h][1] = l_run[h];
             }
         }

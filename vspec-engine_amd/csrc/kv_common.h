@@ -790,7 +790,7 @@ __device__ __forceinline__ ItemCursor item_part(const DecodeParams& p, int& lo, 
 }
 
 // Block-wide: merge the NW wave states of an item part and write the output rows (whole) or
-// the part's partial state.
+// the part's partial state.  A state of max -inf holds no token and is left out.
 template <int D, int GW, int NW>
 __device__ __forceinline__ void finish_item(const DecodeParams& p, const float (*st)[GW][D + 2], const ItemCursor& c,
                                             size_t slot, bool whole) {
@@ -804,7 +804,9 @@ __device__ __forceinline__ void finish_item(const DecodeParams& p, const float (
         float a = 0.f, l = 0.f;
 #pragma unroll
         for (int v = 0; v < NW; ++v) {
-            const float f = exp2f(st[v][h][0] - M);
+            const float m = st[v][h][0];
+            if (m == -INFINITY) continue;
+            const float f = exp2f(m - M);
             a = fmaf(st[v][h][2 + d], f, a);
             l = fmaf(st[v][h][1], f, l);
         }
@@ -842,10 +844,10 @@ __global__ __launch_bounds__(256) void decode_merge_items(DecodeParams p) {
     const size_t slot0 = ((size_t)b * gridDim.x + y) * p.item_parts;
     const float4* acc = reinterpret_cast<const float4*>(p.part_acc) + slot0 * Q + o;
     const MaxSum* ml = reinterpret_cast<const MaxSum*>(p.part_ml) + slot0 * GW + h;
-    // -1e30 (not -inf) keeps exp2 finite
-    float M = -1e30f, L = 0.f;
+    float M = -INFINITY, L = 0.f;
     float4 A = make_float4(0.f, 0.f, 0.f, 0.f);
     auto add = [&](float m, float l, float4 a) {
+        if (m == -INFINITY) return;  // a state without tokens
         const float nm = fmaxf(M, m);
         const float fo = exp2f(M - nm), fn = exp2f(m - nm);
         A.x = fmaf(a.x, fn, A.x * fo);
