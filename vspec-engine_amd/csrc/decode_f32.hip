@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
         // block's used count (a prefix of the block's slots)
         const int lim = p.block_used ? min(ctx - tok0, used_cap(as_const(p.block_used)[(size_t)c.b * p.max_blocks + lblock], slot0))
                                      : ctx - tok0;
-        if (lim <= 0) continue;  // (without a valid slot the weights would be exp2(-inf + inf))
+        if (lim <= 0) continue;
 
         // V goes out with K where a wave's chain of round trips, not the memory rate, is what
         // it waits for: one tile per wave (89 x 1-26 tokens 19.2 -> 17.4 us), and 64-element
@@ -216,7 +216,7 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
                         mv = m_run[h];
                     }
                 }
-                p_lds[wave][buf][kp * KPP + kk][sub] = exp2f(sv - mv);
+                p_lds[wave][buf][kp * KPP + kk][sub] = exp2f(sv - fmaxf(mv, kLowestMax));
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

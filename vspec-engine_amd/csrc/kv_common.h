@@ -735,6 +735,9 @@ __device__ __forceinline__ void finish_segment(const DecodeParams& p, const floa
 // others lie at item * parts + part, where decode_merge_items finds them without redoing a
 // split.
 // ---------------------------------------------------------------------------
+// Running maxima start here and not at -inf, which keeps exp2f(m - M) a number
+constexpr float kLowestMax = -3.402823466e38f;
+
 __device__ __forceinline__ int item_parts_of(const DecodeParams& p, int U) {
     const uint32_t u = (uint32_t)U;
     const uint32_t near = min(p.near_parts, (u + p.part_tiles - 1) / p.part_tiles);
@@ -790,7 +793,8 @@ __device__ __forceinline__ ItemCursor item_part(const DecodeParams& p, int& lo, 
 }
 
 // Block-wide: merge the NW wave states of an item part and write the output rows (whole) or
-// the part's partial state.  A state of max -inf holds no token and is left out.
+// the part's partial state.  A state of max -inf holds no token: against a finite M its weight
+// is 0.
 template <int D, int GW, int NW>
 __device__ __forceinline__ void finish_item(const DecodeParams& p, const float (*st)[GW][D + 2], const ItemCursor& c,
                                             size_t slot, bool whole) {
@@ -798,15 +802,13 @@ __device__ __forceinline__ void finish_item(const DecodeParams& p, const float (
     for (int idx = (int)threadIdx.x; idx < GW * D; idx += NW * 64) {
         const int h = idx / D;
         const int d = idx % D;
-        float M = -INFINITY;
+        float M = kLowestMax;
 #pragma unroll
         for (int v = 0; v < NW; ++v) M = fmaxf(M, st[v][h][0]);
         float a = 0.f, l = 0.f;
 #pragma unroll
         for (int v = 0; v < NW; ++v) {
-            const float m = st[v][h][0];
-            if (m == -INFINITY) continue;
-            const float f = exp2f(m - M);
+            const float f = exp2f(st[v][h][0] - M);
             a = fmaf(st[v][h][2 + d], f, a);
             l = fmaf(st[v][h][1], f, l);
         }
@@ -844,10 +846,9 @@ __global__ __launch_bounds__(256) void decode_merge_items(DecodeParams p) {
     const size_t slot0 = ((size_t)b * gridDim.x + y) * p.item_parts;
     const float4* acc = reinterpret_cast<const float4*>(p.part_acc) + slot0 * Q + o;
     const MaxSum* ml = reinterpret_cast<const MaxSum*>(p.part_ml) + slot0 * GW + h;
-    float M = -INFINITY, L = 0.f;
+    float M = kLowestMax, L = 0.f;
     float4 A = make_float4(0.f, 0.f, 0.f, 0.f);
     auto add = [&](float m, float l, float4 a) {
-        if (m == -INFINITY) return;  // a state without tokens
         const float nm = fmaxf(M, m);
         const float fo = exp2f(M - nm), fn = exp2f(m - nm);
         A.x = fmaf(a.x, fn, A.x * fo);
