@@ -294,3 +294,33 @@ def test_f32_scores_far_below_zero(gpu, monkeypatch, parts):
     out = vr.paged_decode(pool, tables, torch.tensor([T], dtype=torch.int32), (-1e16 * u).view(1, 1, D).contiguous())
     want = v[0, 32:48, 0].double().mean(0)
     assert float((out[0, 0].double() - want).abs().max()) <= 16 * 2.0 ** -24 * 6
+
+
+@pytest.mark.parametrize("sessions,rows,Hq,H,D,P", [
+    ([14], 5, 8, 2, 128, 16), ([30, 1, 250], 3, 6, 2, 64, 32), ([63, 500], 4, 32, 4, 128, 48), ([47, 130], 32, 4, 1, 64, 16),
+    ([15, 700, 63], 22, 8, 8, 64, 16)])
+def test_f32_step_rows_that_share_blocks(gpu, monkeypatch, sessions, rows, Hq, H, D, P):
+    """f32 pools, `rows` rows of the batch on one session's block table, each appending the
+    session's next token (across a tile and a block; up to and above the 64 rows that the decode
+    kernel looks after itself): every row sees the tokens of the rows before it, as after
+    kv_append (the same pool bytes; outputs within the rounding of f32 sums in another order)."""
+    import torch
+
+    lens = [n + r + 1 for n in sessions for r in range(rows)]
+    nblk = -(-max(lens) // P)
+    vr, pools, tables, _, _, _, _ = _decode_setup(gpu, "f32", [nblk * P] * len(sessions), Hq, H, D, P)
+    tables = tables.repeat_interleave(rows, 0).contiguous()
+    ctx = torch.tensor(lens, dtype=torch.int32, device=gpu)
+    g = torch.Generator(device=gpu).manual_seed(len(lens))
+    q = torch.randn((len(lens), Hq, D), generator=g, device=gpu)
+    for src in (torch.float32, torch.float16):
+        new = [torch.randn((len(lens), H, D), generator=g, device=gpu).to(src) for _ in range(2)]
+        vr.kv_append(pools[0], tables, ctx - 1, *(x[:, None].contiguous() for x in new))
+        monkeypatch.setenv("VSPEC_ROCM_DECODE_ITEM_PARTS", "1")
+        want = vr.paged_decode(pools[0], tables, ctx, q, numerics=vr.NUMERICS_3BIT)
+        for parts in ("1", "", "3"):
+            monkeypatch.setenv("VSPEC_ROCM_DECODE_ITEM_PARTS", parts)
+            vr.kv_append(pools[1], tables, ctx - 1, *(x[:, None].neg().contiguous() for x in new))  # what the step replaces
+            got = vr.paged_decode_step(pools[1], tables, ctx, q, *new, numerics=vr.NUMERICS_3BIT)
+            assert _same_pools(*pools)
+            assert float((got - want).abs().max()) <= 6e-6, (src, parts)

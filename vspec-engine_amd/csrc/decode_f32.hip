@@ -4,8 +4,9 @@
 //
 // One workgroup of 4 waves per part of a work item (item_part); wave w takes the part's
 // tiles w, w + 4, ...  D/16 lanes hold one key, 16 elements each (chunks of 4 elements
-// sub + j * D/16); D/8 lanes hold one token of V, 8 elements each.  The decode step's token is
-// taken from its source rows by every wave that reads its tile, so no launch precedes this one.
+// sub + j * D/16); D/8 lanes hold one token of V, 8 elements each.  The decode step's tokens are
+// taken from their source rows by every wave that reads their tiles, whichever row of the batch
+// they belong to, so no launch precedes this one.
 //
 // Bound by the memory rate at full batches (16 x 2049 tokens: 269 MB in 55.3 us with the merge
 // launch, 61 us with an append launch ahead and ordinary loads) and by a wave's chain of round
@@ -69,6 +70,13 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // The decode step's tokens, row i's in lane i (at most kStepRows rows).  Rows may share
+    // blocks, as two rows that verify two tokens of one session do: a tile can hold tokens that
+    // other rows' workgroups store while it is read here, so all of them are taken from the
+    // source rows.  The two dependent loads run beside those of the item's context and entry.
+    const int ctx_cap = (int)(p.max_blocks * p.block_tokens);
+    const int step_row = min(lane, (int)p.batch - 1);
+    const int step_ctx = p.k_new ? p.ctx_lens[step_row] : 0;
     int lo, hi;
     size_t part_slot;
     const ItemCursor c = item_part(p, lo, hi, part_slot);
@@ -76,7 +84,6 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
     const int hk = __builtin_amdgcn_readfirstlane(c.y / (int)p.gsplit);
     const int hq0 = c.y * GW;
     const int tiles_per_block = (int)p.block_tokens / kTile;
-    const int ctx_cap = (int)(p.max_blocks * p.block_tokens);
     const const_i32* table = as_const(p.block_tables) + (size_t)c.b * p.max_blocks;
 
     const int kk = lane / LPK;      // key within a K pass
@@ -95,11 +102,19 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
             qv[h][4 * j] = w.x; qv[h][4 * j + 1] = w.y; qv[h][4 * j + 2] = w.z; qv[h][4 * j + 3] = w.w;
         }
     }
+    int step_block = -1, step_slot = 0;
+    if (p.k_new) {
+        const int pos = min(max(step_ctx, 1), ctx_cap) - 1;
+        const int e = p.block_tables[(size_t)step_row * p.max_blocks + pos / (int)p.block_tokens];
+        const bool is = lane < (int)p.batch && step_ctx >= 1 && step_ctx <= ctx_cap && (uint32_t)e < p.num_blocks;
+        step_block = is ? e : -1;
+        step_slot = pos % (int)p.block_tokens;
+    }
     int tile = lo + wave;
     int entry = table[min(tile, hi - 1) / tiles_per_block];
     const int raw_ctx = as_const(p.ctx_lens)[c.b];
     const int ctx = min(max(raw_ctx, 0), ctx_cap);
-    // the decode step's new token: its position, and the decoded tile whose wave stores it
+    // the row's own new token: its position, and the decoded tile whose wave stores it
     const int papp = p.k_new && raw_ctx >= 1 && raw_ctx <= ctx_cap ? raw_ctx - 1 : -1;
     const int tnew = papp >= 0 ? min(papp / kTile, c.U - 1) : -1;
 #pragma unroll
@@ -130,12 +145,9 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
         const size_t row0 = ((size_t)(ok ? phys : 0) * p.hkv + hk) * p.block_tokens + slot0;
         const float* krow = reinterpret_cast<const float*>(p.k) + row0 * D;
         const float* vrow = reinterpret_cast<const float*>(p.v) + row0 * D;
-        // the new token: taken from its source rows wherever the tile is read, and written to
-        // the pool here (its block may be another one where the context exceeds the bound)
-        const bool here = tile == tnew;
-        const int ts = here && tile == papp / kTile ? papp % kTile : -1;  // its slot in this tile
-        const size_t new_el = ((size_t)c.b * p.hkv + hk) * D;
-        if (here && c.y % (int)p.gsplit == 0) {
+        // (its block may be another one where the context exceeds the bound)
+        if (tile == tnew && c.y % (int)p.gsplit == 0) {
+            const size_t new_el = ((size_t)c.b * p.hkv + hk) * D;
             const int e = table[papp / (int)p.block_tokens];
             if (e >= 0 && (uint32_t)e < p.num_blocks && lane < D / 4) {
                 const size_t row = ((size_t)e * p.hkv + hk) * p.block_tokens + papp % (int)p.block_tokens;
@@ -149,6 +161,8 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
         const int lim = p.block_used ? min(ctx - tok0, used_cap(as_const(p.block_used)[(size_t)c.b * p.max_blocks + lblock], slot0))
                                      : ctx - tok0;
         if (lim <= 0) continue;
+        // rows with a new token in this tile
+        const uint64_t fresh = p.k_new ? __ballot(step_block == phys && step_slot / kTile == slot0 / kTile) : 0ull;
 
         // V goes out with K where a wave's chain of round trips, not the memory rate, is what
         // it waits for: one tile per wave (89 x 1-26 tokens 19.2 -> 17.4 us), and 64-element
@@ -171,9 +185,17 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
             float x[16];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                float4 w = load_row4<ONCE>(krow + (size_t)slot * D + 4 * (sub + j * LPK));
-                if (slot == ts) w = load_new4(p.k_new, new_el + 4 * (sub + j * LPK), p.append_src);
+                const float4 w = load_row4<ONCE>(krow + (size_t)slot * D + 4 * (sub + j * LPK));
                 x[4 * j] = w.x; x[4 * j + 1] = w.y; x[4 * j + 2] = w.z; x[4 * j + 3] = w.w;
+            }
+            for (uint64_t m = fresh; m; m &= m - 1) {
+                const int r = __builtin_ctzll(m);
+                if (slot != __builtin_amdgcn_readlane(step_slot, r) % kTile) continue;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float4 w = load_new4(p.k_new, ((size_t)r * p.hkv + hk) * D + 4 * (sub + j * LPK), p.append_src);
+                    x[4 * j] = w.x; x[4 * j + 1] = w.y; x[4 * j + 2] = w.z; x[4 * j + 3] = w.w;
+                }
             }
             clamp_row<LPK, D>(x, p.alpha, p.input_clip);
             const bool valid = slot < lim;
@@ -230,9 +252,11 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
         for (int vp = 0; vp < VPASS; ++vp) {
             const int slot = vp * VTPP + vt;
             float4 a = va[vp], b = vb[vp];
-            if (slot == ts) {
-                a = load_new4(p.v_new, new_el + 8 * vc, p.append_src);
-                b = load_new4(p.v_new, new_el + 8 * vc + 4, p.append_src);
+            for (uint64_t m = fresh; m; m &= m - 1) {
+                const int r = __builtin_ctzll(m);
+                if (slot != __builtin_amdgcn_readlane(step_slot, r) % kTile) continue;
+                a = load_new4(p.v_new, ((size_t)r * p.hkv + hk) * D + 8 * vc, p.append_src);
+                b = load_new4(p.v_new, ((size_t)r * p.hkv + hk) * D + 8 * vc + 4, p.append_src);
             }
             float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
             if (tail && slot >= lim) {

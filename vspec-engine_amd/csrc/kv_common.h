@@ -253,9 +253,11 @@ struct DecodeParams {
     uint32_t batch;
     uint32_t max_tiles;    // tiles of the host's context bound (max_ctx_len)
     uint32_t chunk_tiles;  // tiles per workgroup, or 0: split evenly over gridDim.x
-    // fused decode-step append of the MFMA kernels (k_new != null): each sequence's new
-    // token, [batch][hkv][D] in append_src (VSPEC_KV_F32 / VSPEC_KV_F16), is written at
-    // position ctx_lens[b] - 1 before any tile is read
+    // fused decode-step append (k_new != null): each sequence's new token, [batch][hkv][D] in
+    // append_src (VSPEC_KV_F32 / VSPEC_KV_F16), goes to position ctx_lens[b] - 1.  The f16 and
+    // f32 kernels take it from these rows wherever its tile is read (the f32 kernel every row's
+    // token, the f16 kernel the sequence's own) and one wave stores it; the int4 kernel takes or
+    // stores it before the tile is read
     const uint8_t* k_new;
     const uint8_t* v_new;
     int32_t append_src;
@@ -274,6 +276,9 @@ struct DecodeParams {
     uint32_t near_parts;
     uint32_t far_tiles;  // least tiles per part with more parts
 };
+
+// Most rows of a fused decode step on f32 pools: one lane of a wave looks after each
+constexpr uint32_t kStepRows = 64;
 
 // Launch the decode kernels for f32 pools (decode_f32.hip), f16 pools (decode_mfma.hip) and
 // int4 pools (decode_mfma_int4.hip) of head_dim 64 or 128, each followed by its merge launch; they

@@ -1433,8 +1433,9 @@ size_t vspec_rocm_paged_decode_workspace_bytes(const VspecPagedAttnDesc* desc) {
 
 namespace {
 
-// Decode attention, with the decode step's append of k_new / v_new first when they are
-// given (one launch for the f16 and int4 kernels, an append launch before the f32 one).
+// Decode attention, with the decode step's append of k_new / v_new when they are given: by the
+// decode kernel itself, or for f32 pools and more than kStepRows rows by a launch before it
+// (the f32 kernel looks in every tile for the new tokens of all rows, which may share blocks).
 // noalloc: the partial states come from the file-scope scratch array
 // (no allocation, no library state beyond it); the descriptor's workspace is ignored.
 int paged_decode(const VspecPagedAttnDesc* desc, const void* k_new, const void* v_new, int32_t src_dtype,
@@ -1536,8 +1537,20 @@ int paged_decode(const VspecPagedAttnDesc* desc, const void* k_new, const void* 
                  : desc->kv.dtype == VSPEC_KV_INT4 ? decode_segment_cost_int4() : 0u;
 
     hipStream_t s = (hipStream_t)desc->stream;
-    p.k_new = (const uint8_t*)k_new;
-    p.v_new = (const uint8_t*)v_new;
+    if (k_new && !pl.split && desc->batch > kStepRows) {
+        AppendParams a = {};
+        a.block_tables = desc->block_tables;
+        a.ctx_lens = desc->ctx_lens;
+        a.k_new = (const uint8_t*)k_new;
+        a.v_new = (const uint8_t*)v_new;
+        a.batch = desc->batch;
+        a.n_new = 1;
+        a.max_blocks = desc->max_blocks_per_seq;
+        if (!append_launch("paged_decode_step append launch", &desc->kv, a, src_dtype, s)) return 0;
+    } else {
+        p.k_new = (const uint8_t*)k_new;
+        p.v_new = (const uint8_t*)v_new;
+    }
     if (pl.split) {
         // partial slots [grid][2][GW] of (max, sum) then of acc[D]
         p.part_acc = (float*)ws + (size_t)pl.grid_x * 2 * pl.gw * 2;
