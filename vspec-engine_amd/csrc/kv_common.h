@@ -735,7 +735,7 @@ __device__ __forceinline__ void finish_segment(const DecodeParams& p, const floa
 // ---------------------------------------------------------------------------
 // Item split (DecodeParams.item_parts): workgroup (y * parts + part, b) takes part `part` of
 // work item y of sequence b.  An item of U tiles is cut into n <= parts parts (item_parts_of),
-// of tiles [part * U / n, (part + 1) * U / n).  No pass over ctx_lens, no workgroup with two
+// of U / n tiles, the first U % n of them of one more.  No pass over ctx_lens, no workgroup with two
 // items; an item in one part goes straight to the output, and the partial states of the
 // others lie at item * parts + part, where decode_merge_items finds them without redoing a
 // split.
@@ -747,6 +747,16 @@ __device__ __forceinline__ int item_parts_of(const DecodeParams& p, int U) {
     const uint32_t u = (uint32_t)U;
     const uint32_t near = min(p.near_parts, (u + p.part_tiles - 1) / p.part_tiles);
     return (int)min(p.item_parts, max(near, (u + p.far_tiles - 1) / p.far_tiles));
+}
+
+// Tiles [lo, hi) of part `part` of an item of U tiles, none past its parts.  (Sums, not part * U / n:
+// that product passes 2^32 from 131072 tiles in parts of 4 on.)
+__device__ __forceinline__ void part_range(const DecodeParams& p, uint32_t part, uint32_t U, int& lo, int& hi) {
+    const uint32_t n = (uint32_t)item_parts_of(p, (int)U);
+    const uint32_t each = U / n, more = U - each * n;
+    const uint32_t l = part * each + min(part, more);
+    lo = part < n ? (int)l : 0;
+    hi = part < n ? (int)(l + each + (part < more ? 1u : 0u)) : 0;
 }
 
 // this workgroup's item (tile positions count from the item's first tile) and tiles [lo, hi);
@@ -783,11 +793,7 @@ __device__ __forceinline__ ItemCursor item_part(const DecodeParams& p, int& lo, 
     c.y = (int)(x * p.gsplit + g);
     c.U = item_tiles(p, c.b);
     int l = 0, h = c.U;
-    if (p.item_parts > 1) {
-        const uint32_t n = (uint32_t)item_parts_of(p, c.U);
-        l = part < n ? (int)(part * (uint32_t)c.U / n) : 0;
-        h = part < n ? (int)((part + 1) * (uint32_t)c.U / n) : 0;
-    }
+    if (p.item_parts > 1) part_range(p, part, (uint32_t)c.U, l, h);
     // wave-uniform values on the scalar unit (the divisions run on the vector one)
     c.y = __builtin_amdgcn_readfirstlane(c.y);
     c.U = __builtin_amdgcn_readfirstlane(c.U);
