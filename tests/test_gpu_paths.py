@@ -324,3 +324,37 @@ def test_f32_step_rows_that_share_blocks(gpu, monkeypatch, sessions, rows, Hq, H
             got = vr.paged_decode_step(pools[1], tables, ctx, q, *new, numerics=vr.NUMERICS_3BIT)
             assert _same_pools(*pools)
             assert float((got - want).abs().max()) <= 6e-6, (src, parts)
+
+
+@pytest.mark.parametrize("pt", [16, 48, 512])
+def test_f32_partition_tokens_is_the_part_size(gpu, pt):
+    """f32 pools: with partition_tokens every part of an item holds that many tokens, whatever the
+    longest context of the batch: the (max, sum) states in the workspace equal the exponential
+    sums over exactly those tokens, and the other slots stay as they were (sums of up to 512
+    exponentials <= 1 of scores with 2^-22 of error: 1e-5)."""
+    import ctypes as C
+    import torch
+
+    lens, H, D, P = [1049, 130, 16], 2, 64, 16
+    vr, pools, tables, ctx, q, _, _ = _decode_setup(gpu, "f32", lens, H, H, D, P)
+    out = torch.empty_like(q)
+    parts = -(-max(lens) // pt)
+    d = vr.make_decode_desc(pools[0], tables, ctx, q, out, max(lens), partition_tokens=pt)
+    assert vr.decode_workspace_bytes(d) == len(lens) * H * parts * (D + 2) * 4
+    ws = torch.full((len(lens) * H * parts * (D + 2),), 7e7, device=gpu)
+    d = vr.make_decode_desc(pools[0], tables, ctx, q, out, max(lens), partition_tokens=pt, workspace=ws)
+    assert vr.lib().vspec_rocm_paged_decode_attention(C.byref(d)), vr.last_error()
+    ml = ws[len(lens) * H * parts * D:].view(len(lens), H, parts, 2).cpu().double()
+    k, _, _, _ = vr.kv_gather(pools[0], tables, ctx, out_mode=vr.GATHER_F32)
+    k, at = k.cpu().double(), 0
+    limit = lambda x: torch.minimum(torch.maximum(x, -4.5 * x.std(-1, correction=0, keepdim=True)), 4.5 * x.std(-1, correction=0, keepdim=True))  # noqa: E731
+    for b, n in enumerate(lens):
+        for h in range(H):
+            s = limit(k[at:at + n, h]) @ limit(q[b, h].cpu().double()) / D ** 0.5
+            ranges = range(0, n, pt) if n > pt else []  # an item in one part has no state
+            for i, t in enumerate(ranges):
+                want = s[t:t + pt].logsumexp(0)
+                got = ml[b, h, i, 0] * 0.6931471805599453 + ml[b, h, i, 1].log()
+                assert abs(float(got - want)) <= 1e-5, (b, h, i)
+            assert bool((ml[b, h, len(ranges):] == 7e7).all())
+        at += n

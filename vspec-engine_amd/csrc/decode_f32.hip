@@ -79,7 +79,7 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
     const int step_ctx = p.k_new ? p.ctx_lens[step_row] : 0;
     int lo, hi;
     size_t part_slot;
-    const ItemCursor c = item_part(p, lo, hi, part_slot);
+    const ItemCursor c = item_part<true>(p, lo, hi, part_slot);
     if (lo >= hi) return;
     const int hk = __builtin_amdgcn_readfirstlane(c.y / (int)p.gsplit);
     const int hq0 = c.y * GW;

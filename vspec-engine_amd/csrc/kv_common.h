@@ -252,7 +252,7 @@ struct DecodeParams {
     bool merge;            // the host could not rule out work items spanning two workgroups
     uint32_t batch;
     uint32_t max_tiles;    // tiles of the host's context bound (max_ctx_len)
-    uint32_t chunk_tiles;  // tiles per workgroup, or 0: split evenly over gridDim.x
+    uint32_t chunk_tiles;  // tiles per workgroup, or 0: split evenly (f32 pools: tiles per part)
     // fused decode-step append (k_new != null): each sequence's new token, [batch][hkv][D] in
     // append_src (VSPEC_KV_F32 / VSPEC_KV_F16), goes to position ctx_lens[b] - 1.  The f16 and
     // f32 kernels take it from these rows wherever its tile is read (the f32 kernel every row's
@@ -750,9 +750,16 @@ __device__ __forceinline__ int item_parts_of(const DecodeParams& p, int U) {
 }
 
 // Tiles [lo, hi) of part `part` of an item of U tiles, none past its parts.  (Sums, not part * U / n:
-// that product passes 2^32 from 131072 tiles in parts of 4 on.)
+// that product passes 2^32 from 131072 tiles in parts of 4 on.)  CHUNKS: with chunk_tiles, that
+// many tiles a part, the last one's rest (part_tiles is the same number then).
+template <bool CHUNKS>
 __device__ __forceinline__ void part_range(const DecodeParams& p, uint32_t part, uint32_t U, int& lo, int& hi) {
     const uint32_t n = (uint32_t)item_parts_of(p, (int)U);
+    if (CHUNKS && p.chunk_tiles) {
+        lo = part < n ? (int)(part * p.chunk_tiles) : 0;
+        hi = part < n ? (int)min(U, part * p.chunk_tiles + p.chunk_tiles) : 0;
+        return;
+    }
     const uint32_t each = U / n, more = U - each * n;
     const uint32_t l = part * each + min(part, more);
     lo = part < n ? (int)l : 0;
@@ -761,6 +768,7 @@ __device__ __forceinline__ void part_range(const DecodeParams& p, uint32_t part,
 
 // this workgroup's item (tile positions count from the item's first tile) and tiles [lo, hi);
 // lo = hi when it has none; slot: the part's partial state
+template <bool CHUNKS = false>
 __device__ __forceinline__ ItemCursor item_part(const DecodeParams& p, int& lo, int& hi, size_t& slot) {
     ItemCursor c;
     c.seq0 = 0;
@@ -793,7 +801,7 @@ __device__ __forceinline__ ItemCursor item_part(const DecodeParams& p, int& lo, 
     c.y = (int)(x * p.gsplit + g);
     c.U = item_tiles(p, c.b);
     int l = 0, h = c.U;
-    if (p.item_parts > 1) part_range(p, part, (uint32_t)c.U, l, h);
+    if (p.item_parts > 1) part_range<CHUNKS>(p, part, (uint32_t)c.U, l, h);
     // wave-uniform values on the scalar unit (the divisions run on the vector one)
     c.y = __builtin_amdgcn_readfirstlane(c.y);
     c.U = __builtin_amdgcn_readfirstlane(c.U);

@@ -950,6 +950,7 @@ int plan_decode(const VspecPagedAttnDesc* d, DecodePlan* pl) {
     const uint32_t max_tiles = (uint32_t)((ctx_bound + kTile - 1) / kTile);
     pl->split = d->kv.dtype != VSPEC_KV_F32;
     pl->item_parts = 0;
+    pl->chunk_tiles = 0;
     pl->part_tiles = 4;  // one for each wave
     pl->near_parts = 0x7fffffffu;
     pl->far_tiles = 0x40000000u;
@@ -970,7 +971,6 @@ int plan_decode(const VspecPagedAttnDesc* d, DecodePlan* pl) {
             pl->chunk_tiles = d->partition_tokens / kTile;
             grid = (bound + pl->chunk_tiles - 1) / pl->chunk_tiles;
         } else {
-            pl->chunk_tiles = 0;
             // two workgroups per CU; small f16 batches (under 64 tiles per workgroup at two
             // per CU) take one, which halves the cross-workgroup merges per work item
             // (C2: 41.6 -> 38.9 us; the int4 kernel, bound by vector ALU work, needs both)
@@ -1016,6 +1016,7 @@ int plan_decode(const VspecPagedAttnDesc* d, DecodePlan* pl) {
             return 0;
         }
         const uint32_t tpp = d->partition_tokens / kTile;
+        pl->chunk_tiles = pl->part_tiles = tpp;
         if (max_tiles) pl->item_parts = (max_tiles + tpp - 1) / tpp;
     } else if (d->batch) {
         pl->item_parts = plan_f32_parts((uint64_t)d->batch * hkv * pl->gsplit, max_tiles ? max_tiles : 1, d->kv.head_dim,
@@ -1523,7 +1524,7 @@ int paged_decode(const VspecPagedAttnDesc* desc, const void* k_new, const void* 
     p.merge = pl.split && pl.merge;
     p.batch = desc->batch;
     p.max_tiles = pl.max_tiles;
-    p.chunk_tiles = pl.split ? pl.chunk_tiles : 0u;
+    p.chunk_tiles = pl.chunk_tiles;
     p.append_src = src_dtype;
     p.split_old_permille = pl.split ? pl.old_permille : 500u;
     p.uniform_tiles = pl.split ? pl.uniform_tiles : 0u;
