@@ -52,9 +52,15 @@ __device__ __forceinline__ void clamp_row(float* x, float alpha, float input_cli
     for (int e = 0; e < 16; ++e) x[e] = fminf(fmaxf(x[e], -th), th);
 }
 
-// ONCE: each tile is read by one work item, past the caches (16 x 2049 tokens 55.6 us, 59.0 with
-// ordinary loads); else the gsplit items of a kv head share it in their XCD's L2 (25 x 37-2392
-// tokens, 8 heads per kv head: 54.8 us, 57.5 past the caches)
+// ONCE: each tile is read by one work item; else the gsplit items of a kv head share it in their
+// XCD's L2 (25 x 37-2392 tokens, 8 heads per kv head: 54.8 us, 57.5 past the caches).  Read once,
+// K goes past the caches, and V too with 64-element heads.  First pass on a pool just written /
+// repeated passes on three pools in turn, us, K and V past the caches, K alone, neither:
+//   16 x 2049 tokens, D = 128         76 / 55.2   67 / 54.7   68 / 58.9
+//   64 x 1025, D = 128               129 / 93.2  118 / 91.3  159 / 100.1
+//   13 x 3101-6203, D = 128          130 / 106   159 / 104   171 / 108
+//   36 x 649-5195, D = 64             86 / 69.9   79 / 70.7   80 / 71.0
+// (the kernel before the item split: 70 / 61.2, 162 / 105.7, 158 / 105.2, 98 / 83.3)
 template <int D, int GW, bool ONCE>
 __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
     constexpr int LPK = D / 16;           // lanes per key
@@ -172,8 +178,8 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
         auto load_v = [&]() {
 #pragma unroll
             for (int vp = 0; vp < VPASS; ++vp) {
-                va[vp] = load_row4<ONCE>(vrow + (size_t)(vp * VTPP + vt) * D + 8 * vc);
-                vb[vp] = load_row4<ONCE>(vrow + (size_t)(vp * VTPP + vt) * D + 8 * vc + 4);
+                va[vp] = load_row4<ONCE && D == 64>(vrow + (size_t)(vp * VTPP + vt) * D + 8 * vc);
+                vb[vp] = load_row4<ONCE && D == 64>(vrow + (size_t)(vp * VTPP + vt) * D + 8 * vc + 4);
             }
         };
         if (v_early) load_v();
