@@ -8,7 +8,7 @@
 // taken from their source rows by every wave that reads their tiles, whichever row of the batch
 // they belong to, so no launch precedes this one.
 //
-// Bound by the memory rate at full batches (16 x 2049 tokens: 269 MB in 55.3 us with the merge
+// Bound by the memory rate at full batches (16 x 2049 tokens: 269 MB in 53.3 us with the merge
 // launch, 61 us with an append launch ahead and ordinary loads) and by a wave's chain of round
 // trips per tile (about 3 us) at small ones.
 #include "kv_common.h"
@@ -97,6 +97,22 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
     const int vc = lane % VLPT;     // V chunk
     const int vt = lane / VLPT;     // token within a V pass
 
+    int tile = lo + wave;
+    int entry = table[min(tile, hi - 1) / tiles_per_block];
+    const int raw_ctx = as_const(p.ctx_lens)[c.b];
+    const int ctx = min(max(raw_ctx, 0), ctx_cap);
+    // the row's own new token: its position, and the decoded tile whose wave stores it
+    const int papp = p.k_new && raw_ctx >= 1 && raw_ctx <= ctx_cap ? raw_ctx - 1 : -1;
+    const int tnew = papp >= 0 ? min(papp / kTile, c.U - 1) : -1;
+    int step_block = -1, step_slot = 0;
+    if (p.k_new) {
+        const int pos = min(max(step_ctx, 1), ctx_cap) - 1;
+        const int e = p.block_tables[(size_t)step_row * p.max_blocks + pos / (int)p.block_tokens];
+        const bool is = lane < (int)p.batch && step_ctx >= 1 && step_ctx <= ctx_cap && (uint32_t)e < p.num_blocks;
+        step_block = is ? e : -1;
+        step_slot = pos % (int)p.block_tokens;
+    }
+
     // q' = clip(q) * scale * log2(e), in the K-side lane layout
     float qv[GW][16];
 #pragma unroll
@@ -108,21 +124,6 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
             qv[h][4 * j] = w.x; qv[h][4 * j + 1] = w.y; qv[h][4 * j + 2] = w.z; qv[h][4 * j + 3] = w.w;
         }
     }
-    int step_block = -1, step_slot = 0;
-    if (p.k_new) {
-        const int pos = min(max(step_ctx, 1), ctx_cap) - 1;
-        const int e = p.block_tables[(size_t)step_row * p.max_blocks + pos / (int)p.block_tokens];
-        const bool is = lane < (int)p.batch && step_ctx >= 1 && step_ctx <= ctx_cap && (uint32_t)e < p.num_blocks;
-        step_block = is ? e : -1;
-        step_slot = pos % (int)p.block_tokens;
-    }
-    int tile = lo + wave;
-    int entry = table[min(tile, hi - 1) / tiles_per_block];
-    const int raw_ctx = as_const(p.ctx_lens)[c.b];
-    const int ctx = min(max(raw_ctx, 0), ctx_cap);
-    // the row's own new token: its position, and the decoded tile whose wave stores it
-    const int papp = p.k_new && raw_ctx >= 1 && raw_ctx <= ctx_cap ? raw_ctx - 1 : -1;
-    const int tnew = papp >= 0 ? min(papp / kTile, c.U - 1) : -1;
 #pragma unroll
     for (int h = 0; h < GW; ++h) {
         clamp_row<LPK, D>(qv[h], p.alpha, p.input_clip);
@@ -167,8 +168,6 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
         const int lim = p.block_used ? min(ctx - tok0, used_cap(as_const(p.block_used)[(size_t)c.b * p.max_blocks + lblock], slot0))
                                      : ctx - tok0;
         if (lim <= 0) continue;
-        // rows with a new token in this tile
-        const uint64_t fresh = p.k_new ? __ballot(step_block == phys && step_slot / kTile == slot0 / kTile) : 0ull;
 
         // V goes out with K where a wave's chain of round trips, not the memory rate, is what
         // it waits for: one tile per wave (89 x 1-26 tokens 19.2 -> 17.4 us), and 64-element
@@ -184,32 +183,40 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
         };
         if (v_early) load_v();
         // ---- scores ----
-        float s[KPASS][GW];
+        float s[KPASS][GW], x[KPASS][16];
 #pragma unroll
         for (int kp = 0; kp < KPASS; ++kp) {
-            const int slot = kp * KPP + kk;
-            float x[16];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const float4 w = load_row4<ONCE>(krow + (size_t)slot * D + 4 * (sub + j * LPK));
-                x[4 * j] = w.x; x[4 * j + 1] = w.y; x[4 * j + 2] = w.z; x[4 * j + 3] = w.w;
+                const float4 w = load_row4<ONCE>(krow + (size_t)(kp * KPP + kk) * D + 4 * (sub + j * LPK));
+                x[kp][4 * j] = w.x; x[kp][4 * j + 1] = w.y; x[kp][4 * j + 2] = w.z; x[kp][4 * j + 3] = w.w;
             }
-            for (uint64_t m = fresh; m; m &= m - 1) {
-                const int r = __builtin_ctzll(m);
-                if (slot != __builtin_amdgcn_readlane(step_slot, r) % kTile) continue;
+        }
+        // rows with a new token in this tile (looked up once the tile is on its way)
+        const uint64_t fresh = p.k_new ? __ballot(step_block == phys && step_slot / kTile == slot0 / kTile) : 0ull;
+        for (uint64_t m = fresh; m; m &= m - 1) {
+            const int r = __builtin_ctzll(m);
+            const int at = __builtin_amdgcn_readlane(step_slot, r) % kTile;
+#pragma unroll
+            for (int kp = 0; kp < KPASS; ++kp) {
+                if (kp * KPP + kk != at) continue;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const float4 w = load_new4(p.k_new, ((size_t)r * p.hkv + hk) * D + 4 * (sub + j * LPK), p.append_src);
-                    x[4 * j] = w.x; x[4 * j + 1] = w.y; x[4 * j + 2] = w.z; x[4 * j + 3] = w.w;
+                    x[kp][4 * j] = w.x; x[kp][4 * j + 1] = w.y; x[kp][4 * j + 2] = w.z; x[kp][4 * j + 3] = w.w;
                 }
             }
-            clamp_row<LPK, D>(x, p.alpha, p.input_clip);
+        }
+#pragma unroll
+        for (int kp = 0; kp < KPASS; ++kp) {
+            const int slot = kp * KPP + kk;
+            clamp_row<LPK, D>(x[kp], p.alpha, p.input_clip);
             const bool valid = slot < lim;
 #pragma unroll
             for (int h = 0; h < GW; ++h) {
                 float d = 0.f;
 #pragma unroll
-                for (int e = 0; e < 16; ++e) d = fmaf(qv[h][e], x[e], d);
+                for (int e = 0; e < 16; ++e) d = fmaf(qv[h][e], x[kp][e], d);
                 d = group_sum<LPK>(d);
                 d = fminf(fmaxf(d, -p.logit_clip), p.logit_clip);
                 s[kp][h] = valid ? d : -INFINITY;
