@@ -201,3 +201,30 @@ def test_missing_library_fails_loudly(tmp_path):
                PYTHONPATH=str(ROOT / "vspec-engine_amd" / "python"))
     r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=300)
     assert r.returncode == 0 and "raised" in r.stdout, r.stderr[-2000:]
+
+
+@pytest.mark.parametrize("wgs,fits", [(2, True), (3, True), (5, True), (6, False)])
+def test_noalloc_scratch_holds_plans_of_8_heads(wgs, fits):
+    """f16 pools, 8 query heads per kv head of 128 elements: up to 5 workgroups per CU (of 256, what
+    the plan assumes without a GPU) the plan fits the no-allocation step's scratch, so that the
+    call gets past that check to the missing device; 6 are refused.  In a process of its own: the
+    setting is read once."""
+    code = """
+import ctypes as C, sys
+import vspec_rocm as vr
+d = vr.VspecPagedAttnDesc()
+d.kv.dtype, d.kv.num_blocks, d.kv.block_tokens, d.kv.num_kv_heads, d.kv.head_dim = vr.KV_F16, 1 << 14, 16, 4, 128
+d.kv.k_data = d.kv.v_data = 1 << 20
+d.batch, d.num_q_heads, d.max_blocks_per_seq, d.max_ctx_len = 64, 32, 256, 4096
+d.block_tables = d.ctx_lens = d.q = d.out = 1 << 20
+assert vr.lib().vspec_rocm_paged_decode_step_noalloc(C.byref(d), 1 << 20, 1 << 20, vr.KV_F16) == 0
+print(vr.last_error())
+"""
+    import os
+    import sys
+
+    env = dict(os.environ, VSPEC_ROCM_DECODE_WGS_PER_CU=str(wgs), HIP_VISIBLE_DEVICES="", ROCR_VISIBLE_DEVICES="",
+               PYTHONPATH=str(ROOT / "vspec-engine_amd" / "python"))
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, env=env)
+    assert r.returncode == 0, r.stderr[-2000:]
+    assert ("no current device" if fits else "more than the") in r.stdout, r.stdout

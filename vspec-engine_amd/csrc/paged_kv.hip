@@ -916,7 +916,8 @@ bool uniform_split_has_partials(const VspecPagedAttnDesc* d, const DecodePlan* p
     return false;
 }
 
-int plan_decode(const VspecPagedAttnDesc* d, DecodePlan* pl) {
+// most_heads: query heads that one work item may hold, 8 or 4
+int plan_decode(const VspecPagedAttnDesc* d, DecodePlan* pl, uint32_t most_heads = 8) {
     pl->merge = true;
     const uint32_t hkv = d->kv.num_kv_heads;
     if (d->num_q_heads == 0 || d->num_q_heads % hkv != 0) {
@@ -927,7 +928,7 @@ int plan_decode(const VspecPagedAttnDesc* d, DecodePlan* pl) {
     if (g <= 4) {
         pl->gw = g;
         pl->gsplit = 1;
-    } else if (g % 8 == 0 && d->kv.dtype == VSPEC_KV_F16) {
+    } else if (g % 8 == 0 && d->kv.dtype == VSPEC_KV_F16 && most_heads >= 8) {
         // f16: the score MFMA's 16 columns hold 8 heads as well as 4, so that a tile is read
         // and multiplied once for all of them (64 x 4097 tokens, 32/4 heads: 172 us with two
         // items of 4 heads, 142 with the two on one XCD, 89.5 with one of 8)
@@ -1463,6 +1464,9 @@ int paged_decode(const VspecPagedAttnDesc* desc, const void* k_new, const void* 
     if (!plan_decode(desc, &pl)) return 0;
     void* ws = nullptr;
     if (noalloc) {
+        // a workgroup's two partial states are twice as large with 8 heads to a work item as with
+        // 4: plans of many workgroups (VSPEC_ROCM_DECODE_WGS_PER_CU 3 to 5) fit only with 4
+        if (pl.ws_bytes > kScratchBytes && pl.gw == 8 && !plan_decode(desc, &pl, 4)) return 0;
         if (pl.ws_bytes > kScratchBytes) {
             set_err("paged_decode_step_noalloc: the plan needs %zu bytes of partial states, more than the "
                     "%zu-byte scratch (use vspec_rocm_paged_decode_step with a workspace)",
