@@ -228,3 +228,25 @@ print(vr.last_error())
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, env=env)
     assert r.returncode == 0, r.stderr[-2000:]
     assert ("no current device" if fits else "more than the") in r.stdout, r.stdout
+
+
+@pytest.mark.parametrize("heads,kv_heads,D,batch,parts", [(32, 8, 128, 64, 3), (32, 8, 128, 16, 12), (8, 8, 64, 1, 128), (32, 4, 128, 128, 2),
+                                                          (32, 8, 128, 300, 1)])
+def test_f32_workspace_follows_the_context_bound(heads, kv_heads, D, batch, parts):
+    """f32 pools: the workspace holds the partial states of three rounds of workgroups (`parts` per
+    work item on 256 CUs at long contexts), never falls as the context bound rises and does not
+    depend on the lower bound."""
+    import vspec_rocm as vr
+
+    d = vr.VspecPagedAttnDesc()
+    d.kv.dtype, d.kv.num_blocks, d.kv.block_tokens, d.kv.num_kv_heads, d.kv.head_dim = vr.KV_F32, 1 << 16, 16, kv_heads, D
+    d.kv.k_data = d.kv.v_data = 1 << 20
+    d.batch, d.num_q_heads, d.max_blocks_per_seq = batch, heads, 4096
+    last = 0
+    for bound in list(range(1, 700, 5)) + [1025, 4097, 65536]:
+        d.max_ctx_len, d.min_ctx_len = bound, 0
+        need = vr.decode_workspace_bytes(d)
+        d.min_ctx_len = bound
+        assert need == vr.decode_workspace_bytes(d) and need >= last
+        last = need
+    assert last == (batch * heads * parts * (D + 2) * 4 if parts > 1 else 0)

@@ -827,15 +827,18 @@ struct DecodePlan {
 // once, and where that cuts an item in fewer than 6, up to three times as many of at least 16
 // tiles, so that the longest context's parts do not outlast the others (36 x 649-5195 tokens,
 // 144 items: 76 us with 3 parts, 61 with 10; 8 x 773-4188, 64 items: 49 us with 8, 56-66 with
-// more; 35 x 128-1024: 25 us, 31 in parts of 8 tiles).  *ws_parts:
-// what the workspace is sized for, which never falls as the bound on the contexts rises, so
-// that a workspace for the longest contexts serves every shorter one.
+// more; 35 x 128-1024: 25 us, 31 in parts of 8 tiles).  *ws_parts: what the workspace is sized
+// for.  It never falls as the bound on the contexts rises and does not depend on `same`, so that
+// a workspace for the longest contexts serves every shorter one of as many sequences (not every
+// smaller batch: fewer items are cut into more parts).  Neither rule goes past three rounds of
+// workgroups, which is what is reserved.
 // Measured at 1 / 2 / 4 / 8 / 16 / 32 parts: 1 x 4097 tokens (8 items) 227 / 122 / 69 / 42 / 29 / 24
 // us, 16 x 2049 (128) 126 / 75 / 56 / 65, 36 x 649-5195 (144, D = 64) 189 / 107 / 76 / 64, 64 x 1025
 // (512) 95 / 107.
 uint32_t plan_f32_parts(uint64_t items, uint64_t tiles, uint32_t head_dim, uint64_t slots, bool same, uint32_t* ws_parts,
                         DecodePlan* pl) {
-    uint64_t most = 4 * slots / items;
+    uint64_t most = (3 * slots + items - 1) / items;
+    if (most > 4 * slots / items) most = 4 * slots / items;
     if (most > (tiles + 3) / 4) most = (tiles + 3) / 4;
     if (most > 128) most = 128;
     if (most < 1) most = 1;
