@@ -706,8 +706,7 @@ bool balanced_split_env() {
 
 // Parts of a work item under the item split (kv_common.h item_part), or 0 for the balanced
 // split of all items' tiles.  Read on every call: VSPEC_ROCM_DECODE_ITEM_PARTS 0 never, 1..64
-// that many (as far as the workspace holds them); VSPEC_ROCM_DECODE_WIDE=2 whole items
-// wherever they fit the CUs.
+// that many (as far as the workspace holds them).
 //
 // Else the cheaper one by a cost model in us, fitted to both splits over 30 shapes (1-128
 // sequences of 19-16k tokens): `slots` workgroups run at a time; with k of them running, a
@@ -736,8 +735,6 @@ uint32_t plan_item_parts(const VspecPagedAttnDesc* d, uint64_t items, uint64_t t
         return x <= 0 ? 0u : (uint32_t)((uint64_t)x < most ? (x < 64 ? x : 64) : (most < 64 ? most : 64));
     }
     if (balanced_split_env()) return 0;
-    e = getenv("VSPEC_ROCM_DECODE_WIDE");
-    if (e && strtol(e, nullptr, 10) == 2 && same && items <= slots / 2) return 1;
     const bool i4 = d->kv.dtype == VSPEC_KV_INT4;
     const double size = d->kv.head_dim / 128.0;
     const SplitCost c = i4 ? SplitCost{0.15, 2.6e-4 * (1 + size) / 2, 7.0, 4.2e-4 * (1 + size) / 2, 19.0}
