@@ -1,7 +1,7 @@
 // append_row.h -- block-table append of one chunk of a token-head row of K or V
-// (kv_paged_cache.c:292-303 in the reference, with quantise-on-write for int4 pools),
-// shared by the append kernels (paged_kv.hip) and the decode kernels' fused decode-step
-// append (decode_mfma.hip, decode_mfma_int4.hip).
+// (kv_paged_cache.c:292-303 in the reference, with quantise-on-write for int4 pools):
+// the items of the append kernels (paged_kv.hip), and the int4 codec, which the int4
+// decode's fused append uses as well (decode_mfma_int4.hip).
 #pragma once
 #include "kv_common.h"
 
@@ -31,7 +31,7 @@ struct AppendParams {
     float* q_out;
     uint32_t hq;
     // with start_pos and token_item null: source token b goes to position ctx_lens[b] - 1
-    // (the decode step's append; a context of 0 appends nothing)
+    // (the append of an f32 decode step of many rows; a context of 0 appends nothing)
     const int32_t* ctx_lens;
     const uint8_t* k_new;
     const uint8_t* v_new;
@@ -48,9 +48,6 @@ struct AppendParams {
 // 8 elements (16 or 32 bytes) otherwise.
 constexpr int append_ept(int dt) { return dt == VSPEC_KV_INT4 ? 32 : 8; }
 
-// Chunk c of the token-head row of K (which 0) or V (which 1) whose first source element
-// is src_el, written at position pos of block-table row `seq`, kv head h.  Positions past
-// the table, behind an invalid entry or (with rotary tables) past max_pos are not written.
 // A clamp-flag update: flag word `word` gets bit `bit` set or cleared.
 struct FlagOp {
     uint32_t* word;
@@ -200,6 +197,9 @@ __device__ __forceinline__ void load_elements(const uint8_t* src, size_t el, flo
     }
 }
 
+// Chunk c of the token-head row of K (which 0) or V (which 1) whose first source element
+// is src_el, written at position pos of block-table row `seq`, kv head h.  Positions past
+// the table, behind an invalid entry or (with rotary tables) past max_pos are not written.
 // ROPE: the launch may carry rotary tables (without it their code and registers go)
 template <int DT, int SRC, bool ROPE = true>
 __device__ __forceinline__ void append_chunk(const AppendParams& p, uint32_t seq, uint32_t pos, uint32_t h,

@@ -311,7 +311,7 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
         }
     }
     __syncthreads();
-    finish_item<D, GW, kWaves>(p, comb, c, part_slot, hi - lo == c.U);
+    finish_item<D, GW>(p, comb, c, part_slot, hi - lo == c.U);
 }
 
 template <int D, int GW>

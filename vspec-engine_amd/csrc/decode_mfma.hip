@@ -55,27 +55,27 @@ struct Frags {
 // scan and one item's set-up: what bounds short and few contexts is the chain of dependent
 // round trips (context scan, q rows, table entries, tiles, merge), 17-34 us of kernel plus a
 // 5-7 us merge launch at 1 x 21 and 53 x 19 tokens against 7.4 and 8.2 us in all here.
-template <int D, int GW, int PB, int NB, bool USED, int NW, bool ITEMS>
-__global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams p) {
+template <int D, int GW, int PB, int NB, bool USED, bool ITEMS>
+__global__ __launch_bounds__(kWaves * 64, 2) void decode_mfma_f16(DecodeParams p) {
     constexpr int NQK = D / 32;   // QK MFMAs per tile (each on 32 d)
     constexpr int NDT = D / 16;   // PV d-tiles
     constexpr int kQStage = ITEMS ? 1 : 4;  // item segments whose q rows are staged up front
     constexpr int kSlots = ITEMS ? 1 : 2;   // item segments being merged at once
     __shared__ float qraw[ITEMS ? 1 : kQStage][ITEMS ? 1 : GW][ITEMS ? 1 : D];
-    __shared__ float qs[ITEMS ? 1 : NW][GW][D];  // per wave: q' of its current item (ITEMS: for all)
+    __shared__ float qs[ITEMS ? 1 : kWaves][GW][D];  // per wave: q' of its current item (ITEMS: for all)
     __shared__ int qexp[GW];                     // ITEMS: per head, the q' operand shift (qnorm_shift)
     // per wave: QK B operands (hi, lo for each 32-wide d chunk), read back every tile
-    __shared__ float comb[kSlots][NW][GW][D + 2];
-    __shared__ float patch_val[NW][kTile][GW];
-    __shared__ int patch_flag[NW][kTile];
+    __shared__ float comb[kSlots][kWaves][GW][D + 2];
+    __shared__ float patch_val[kWaves][kTile][GW];
+    __shared__ int patch_flag[kWaves][kTile];
     __shared__ int slot_cnt[kSlots];
     __shared__ int slot_seg[kSlots];
     // fused decode step: the new token's K and V rows (f16 bits, two per word) of segment s
     // in row s < kQStage (staged up front), of a later segment in row kQStage + wave (staged
     // by the wave itself); the wave that processes the tile holding the token patches them
     // into its fragments and stores them to the pool, so no wave waits for those stores
-    __shared__ uint32_t newtok[kQStage + NW][2][D / 2];
-    __shared__ SplitSharedN<NW> split_sh;
+    __shared__ uint32_t newtok[kQStage + kWaves][2][D / 2];
+    __shared__ SplitShared split_sh;
 
     const int lane = threadIdx.x & 63;
     // wave index as a scalar: tile loop control and block-table reads stay on the
@@ -91,7 +91,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
     if constexpr (ITEMS) {
         first = item_part(p, ws.lo, ws.hi, part_slot);
     } else {
-        ws = work_split<kSplitRagged, NW>(p, ips, split_sh);
+        ws = work_split<kSplitRagged>(p, ips, split_sh);
     }
     if (ws.lo >= ws.hi) return;
     if constexpr (!ITEMS) first = cursor_at(p, ws);
@@ -433,7 +433,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
     };
 
     // Hand this wave's state for segment s (work item c) to merge slot s % kSlots; the
-    // last of the NW waves to hand in merges their states.  A slot serves segment
+    // last of the kWaves waves to hand in merges their states.  A slot serves segment
     // s once segment s - kSlots is merged; waves hand in segments in order, so the wave
     // furthest behind never waits here and every wait ends.
     auto arrive = [&](const int s, const ItemCursor& c) {
@@ -458,10 +458,10 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
         int before = 0;
         if (lane == 0) before = __hip_atomic_fetch_add(&slot_cnt[slot], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         before = __builtin_amdgcn_readfirstlane(before);
-        if (before == NW - 1) {
+        if (before == kWaves - 1) {
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
             const bool whole = c.item0 >= ws.lo && c.item0 + c.U <= ws.hi;
-            merge_segment<D, GW, NW>(p, comb[slot], lane, (size_t)c.b * p.hq + (size_t)c.y * GW, whole, s == 0 ? 0 : 1);
+            merge_segment<D, GW>(p, comb[slot], lane, (size_t)c.b * p.hq + (size_t)c.y * GW, whole, s == 0 ? 0 : 1);
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
             if (lane == 0) {
                 slot_cnt[slot] = 0;
@@ -550,7 +550,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
     int papp = new_pos(pc.b);
     const int len = ws.hi - ws.lo;
     const int t0 = ws.lo + wave;
-    const int nt = wave < len ? (len - wave + NW - 1) / NW : 0;
+    const int nt = wave < len ? (len - wave + kWaves - 1) / kWaves : 0;
     Frags<D> f[NB];
     int ok[NB];
     if constexpr (ITEMS) {
@@ -558,11 +558,11 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
         // waves, each wave's first tiles are on their way while head w is prepared by wave w,
         // one barrier publishes them, and all waves merge after another.
         constexpr int E = D / 64;
-        constexpr int HPW = (GW + NW - 1) / NW;  // heads per wave: w, w + NW
+        constexpr int HPW = (GW + kWaves - 1) / kWaves;  // heads per wave: w, w + kWaves
         float x[HPW][E];
 #pragma unroll
         for (int i = 0; i < HPW; ++i) {
-            const int h = wave + i * NW;
+            const int h = wave + i * kWaves;
             if (h < GW) {
                 const float* qrow = p.q + ((size_t)pc.b * p.hq + (size_t)pc.y * GW + h) * D;
 #pragma unroll
@@ -574,20 +574,20 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
         size_t erow[NB];
 #pragma unroll
         for (int u = 0; u < NB; ++u) {
-            erow[u] = (size_t)pc.b * p.max_blocks + min(t0 + u * NW, ws.hi - 1) / tiles_per_block;
+            erow[u] = (size_t)pc.b * p.max_blocks + min(t0 + u * kWaves, ws.hi - 1) / tiles_per_block;
             entry[u] = as_const(p.block_tables)[erow[u]];
         }
         const int tnew = papp >= 0 ? min(papp / kTile, pc.U - 1) : -1;  // the tile whose wave stores the token
-        const bool stage = tnew >= ws.lo && tnew < ws.hi && wave == NW - 1;
+        const bool stage = tnew >= ws.lo && tnew < ws.hi && wave == kWaves - 1;
         NewRow row;
         if (stage) row = newrow_load(pc);
 #pragma unroll
         for (int u = 0; u < NB; ++u) {
-            if (u < nt) ok[u] = load_entry(t0 + u * NW, true, t0 + u * NW, erow[u], entry[u], f[u]);
+            if (u < nt) ok[u] = load_entry(t0 + u * kWaves, true, t0 + u * kWaves, erow[u], entry[u], f[u]);
         }
 #pragma unroll
         for (int i = 0; i < HPW; ++i) {
-            const int h = wave + i * NW;
+            const int h = wave + i * kWaves;
             if (h < GW) {
                 const int e = qhead(h, x[i]);
                 if (lane == 0) qexp[h] = e;
@@ -608,14 +608,14 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
         for (; k + NB < nt; k += NB) {
 #pragma unroll
             for (int u = 0; u < NB; ++u) {
-                const int t = t0 + (k + u) * NW;
+                const int t = t0 + (k + u) * kWaves;
                 step(u, t);
-                ok[u] = load(t + NB * NW, f[u]);
+                ok[u] = load(t + NB * kWaves, f[u]);
             }
         }
 #pragma unroll
         for (int u = 0; u < NB; ++u) {
-            if (k + u < nt) step(u, t0 + (k + u) * NW);
+            if (k + u < nt) step(u, t0 + (k + u) * kWaves);
         }
         const float l = add_rows(l_run);
         if (n < GW) {
@@ -630,7 +630,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
             }
         }
         __syncthreads();
-        finish_item<D, GW, NW>(p, comb[0], pc, part_slot, ws.hi - ws.lo == pc.U);
+        finish_item<D, GW>(p, comb[0], pc, part_slot, ws.hi - ws.lo == pc.U);
         return;
     }
     // Set-up.  Wave 0 loads the q rows of the range's first kQStage segments (rows GW*y ..
@@ -688,14 +688,14 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
         }
     }
 #pragma unroll
-    for (int u = 0; u < NB; ++u) ok[u] = load(t0 + u * NW, f[u]);
+    for (int u = 0; u < NB; ++u) ok[u] = load(t0 + u * kWaves, f[u]);
     __syncthreads();
     reset();
     qprep(0, pc);
     for (int k = 0; k < nt; k += NB) {
 #pragma unroll
         for (int u = 0; u < NB; ++u) {
-            const int t = t0 + (k + u) * NW;
+            const int t = t0 + (k + u) * kWaves;
             if (t < ws.hi && t >= pc.item0 + pc.U) {
                 do {
                     arrive(seg, pc);
@@ -713,7 +713,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void decode_mfma_f16(DecodeParams 
                 store_new(pc, seg, papp);
             }
             process(f[u], ok[u], t - pc.item0, pctx);
-            ok[u] = load(t + NB * NW, f[u]);
+            ok[u] = load(t + NB * kWaves, f[u]);
         }
     }
     // hand in the current segment and every later one of the workgroup (empty states)
@@ -734,9 +734,9 @@ template <int D, int GW, bool USED, int PB>
 void launch_pb(const DecodeParams& p, dim3 grid, hipStream_t s) {
     constexpr int NB = VSPEC_F16_TILES_IN_FLIGHT;
     if (p.item_parts) {
-        hipLaunchKernelGGL((decode_mfma_f16<D, GW, PB, NB, USED, kWaves, true>), grid, dim3(kWaves * 64), 0, s, p);
+        hipLaunchKernelGGL((decode_mfma_f16<D, GW, PB, NB, USED, true>), grid, dim3(kWaves * 64), 0, s, p);
     } else {
-        hipLaunchKernelGGL((decode_mfma_f16<D, GW, PB, NB, USED, kWaves, false>), grid, dim3(kWaves * 64), 0, s, p);
+        hipLaunchKernelGGL((decode_mfma_f16<D, GW, PB, NB, USED, false>), grid, dim3(kWaves * 64), 0, s, p);
     }
 }
 

@@ -993,7 +993,7 @@ __global__ __launch_bounds__(256, VSPEC_I4_MIN_WG_PER_CU) void decode_mfma_i4(De
         }
         __syncthreads();
         if constexpr (ITEMS) {
-            finish_item<D, GW, kWaves>(p, comb, c0, part_slot, tile_end - tile_begin == U);
+            finish_item<D, GW>(p, comb, c0, part_slot, tile_end - tile_begin == U);
             return;
         }
         finish_segment<D, GW>(p, comb, b, hq0, U, tile_begin, tile_end, pos == ws.lo ? 0 : 1);

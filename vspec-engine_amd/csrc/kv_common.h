@@ -336,17 +336,15 @@ struct WorkSplit {
     int seq0;    // index of that sequence's first tile
 };
 
-template <int NW>
-struct SplitSharedN {
-    int wsum[NW];
-    int umin[NW];  // per wave: least and greatest tiles per work item (U_b)
-    int umax[NW];
-    int wpre[NW];  // merge launch: per wave, tiles of the sequences before the item's
+struct SplitShared {
+    int wsum[kWaves];
+    int umin[kWaves];  // per wave: least and greatest tiles per work item (U_b)
+    int umax[kWaves];
+    int wpre[kWaves];  // merge launch: per wave, tiles of the sequences before the item's
     int b;
     int seq0;
     int lo_t, hi_t;  // balanced split with a segment cost: the range in tiles
 };
-using SplitShared = SplitSharedN<kWaves>;
 
 __device__ __forceinline__ int item_tiles(const DecodeParams& p, int b) {
     if (p.uniform_tiles) return (int)p.uniform_tiles;
@@ -443,10 +441,10 @@ __device__ __forceinline__ void split_range(const DecodeParams& p, WorkSplit& r)
     }
 }
 
-// Block-wide over NW waves (every thread calls it; the result is uniform).  The host keeps
+// Block-wide over kWaves waves (every thread calls it; the result is uniform).  The host keeps
 // T = hkv * gsplit * sum U_b below 2^31.
-template <int UNEVEN, int NW = kWaves>
-__device__ __forceinline__ WorkSplit work_split(const DecodeParams& p, int ips, SplitSharedN<NW>& sh) {
+template <int UNEVEN>
+__device__ __forceinline__ WorkSplit work_split(const DecodeParams& p, int ips, SplitShared& sh) {
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int nb = (int)p.batch;
@@ -463,7 +461,7 @@ __device__ __forceinline__ WorkSplit work_split(const DecodeParams& p, int ips, 
         r.seq0 = r.b * per_seq;
         return r;
     }
-    if (nb <= NW * 64) {
+    if (nb <= kWaves * 64) {
         // one sequence per thread: the total and the search come from one scan
         const int b = (int)threadIdx.x;
         const int u = b < nb ? item_tiles(p, b) : 0;
@@ -491,7 +489,7 @@ __device__ __forceinline__ WorkSplit work_split(const DecodeParams& p, int ips, 
         umin = 0x7fffffff;
         umax = 0;
 #pragma unroll
-        for (int w = 0; w < NW; ++w) {
+        for (int w = 0; w < kWaves; ++w) {
             before += w < wave ? sh.wsum[w] : 0;
             all += sh.wsum[w];
             if constexpr (UNEVEN != 0) {
@@ -537,7 +535,7 @@ __device__ __forceinline__ WorkSplit work_split(const DecodeParams& p, int ips, 
         return r;
     }
     int s = 0, umin = 0x7fffffff, umax = 0;
-    for (int b = threadIdx.x; b < nb; b += NW * 64) {
+    for (int b = threadIdx.x; b < nb; b += kWaves * 64) {
         const int u = item_tiles(p, b);
         s += u;
         if constexpr (UNEVEN != 0) {
@@ -563,7 +561,7 @@ __device__ __forceinline__ WorkSplit work_split(const DecodeParams& p, int ips, 
     umin = 0x7fffffff;
     umax = 0;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) {
+    for (int w = 0; w < kWaves; ++w) {
         units += sh.wsum[w];
         umin = min(umin, sh.umin[w]);
         umax = max(umax, sh.umax[w]);
@@ -578,7 +576,7 @@ __device__ __forceinline__ WorkSplit work_split(const DecodeParams& p, int ips, 
     if (r.lo >= r.hi) return r;
     // the sequence holding tile lo: exclusive prefix of U_b * ips, 256 sequences a pass
     int carry = 0;
-    for (int base = 0; base < nb; base += NW * 64) {
+    for (int base = 0; base < nb; base += kWaves * 64) {
         const int b = base + (int)threadIdx.x;
         const int u = b < nb ? item_tiles(p, b) : 0;
         int x = u;
@@ -592,7 +590,7 @@ __device__ __forceinline__ WorkSplit work_split(const DecodeParams& p, int ips, 
         __syncthreads();
         int before = 0, all = 0;
 #pragma unroll
-        for (int w = 0; w < NW; ++w) {
+        for (int w = 0; w < kWaves; ++w) {
             before += w < wave ? sh.wsum[w] : 0;
             all += sh.wsum[w];
         }
@@ -659,10 +657,10 @@ __device__ __forceinline__ void cursor_next(const DecodeParams& p, int ips, Item
     }
 }
 
-// One wave merges the NW states of one item segment held in LDS (st[w][h] = {max, sum,
+// One wave merges the kWaves states of one item segment held in LDS (st[w][h] = {max, sum,
 // acc[D]}, written by wave w) and writes the output rows of a whole work item, or else the
 // workgroup's partial `pslot` (0: its first segment, 1: its last).
-template <int D, int GW, int NW = kWaves>
+template <int D, int GW>
 __device__ __forceinline__ void merge_segment(const DecodeParams& p, const float (*st)[GW][D + 2], int lane,
                                               size_t row0, bool whole, int pslot) {
     float* pacc = p.part_acc + ((size_t)blockIdx.x * 2 + pslot) * GW * D;
@@ -672,10 +670,10 @@ __device__ __forceinline__ void merge_segment(const DecodeParams& p, const float
         const int d = idx % D;
         float M = -INFINITY;
 #pragma unroll
-        for (int v = 0; v < NW; ++v) M = fmaxf(M, st[v][h][0]);
+        for (int v = 0; v < kWaves; ++v) M = fmaxf(M, st[v][h][0]);
         float a = 0.f, l = 0.f;
 #pragma unroll
-        for (int v = 0; v < NW; ++v) {
+        for (int v = 0; v < kWaves; ++v) {
             const float f = exp2f(st[v][h][0] - M);
             a = fmaf(st[v][h][2 + d], f, a);
             l = fmaf(st[v][h][1], f, l);
@@ -811,22 +809,22 @@ __device__ __forceinline__ ItemCursor item_part(const DecodeParams& p, int& lo, 
     return c;
 }
 
-// Block-wide: merge the NW wave states of an item part and write the output rows (whole) or
+// Block-wide: merge the kWaves wave states of an item part and write the output rows (whole) or
 // the part's partial state.  A state of max -inf holds no token: against a finite M its weight
 // is 0.
-template <int D, int GW, int NW>
+template <int D, int GW>
 __device__ __forceinline__ void finish_item(const DecodeParams& p, const float (*st)[GW][D + 2], const ItemCursor& c,
                                             size_t slot, bool whole) {
     const size_t row0 = (size_t)c.b * p.hq + (size_t)c.y * GW;
-    for (int idx = (int)threadIdx.x; idx < GW * D; idx += NW * 64) {
+    for (int idx = (int)threadIdx.x; idx < GW * D; idx += kWaves * 64) {
         const int h = idx / D;
         const int d = idx % D;
         float M = kLowestMax;
 #pragma unroll
-        for (int v = 0; v < NW; ++v) M = fmaxf(M, st[v][h][0]);
+        for (int v = 0; v < kWaves; ++v) M = fmaxf(M, st[v][h][0]);
         float a = 0.f, l = 0.f;
 #pragma unroll
-        for (int v = 0; v < NW; ++v) {
+        for (int v = 0; v < kWaves; ++v) {
             const float f = exp2f(st[v][h][0] - M);
             a = fmaf(st[v][h][2 + d], f, a);
             l = fmaf(st[v][h][1], f, l);
