@@ -8,7 +8,7 @@
 // taken from their source rows by every wave that reads their tiles, whichever row of the batch
 // they belong to, so no launch precedes this one.
 //
-// Bound by the memory rate at full batches (16 x 2049 tokens: 269 MB in 53.3 us with the merge
+// Bound by the memory rate at full batches (16 x 2049 tokens: 269 MB in 52.7 us with the merge
 // launch, 61 us with an append launch ahead and ordinary loads) and by a wave's chain of round
 // trips per tile (about 3 us) at small ones.
 #include "kv_common.h"
@@ -61,7 +61,8 @@ __device__ __forceinline__ void clamp_row(float* x, float alpha, float input_cli
 //   13 x 3101-6203, D = 128          130 / 106   159 / 104   171 / 108
 //   36 x 649-5195, D = 64             86 / 69.9   79 / 70.7   80 / 71.0
 // (the kernel before the item split: 70 / 61.2, 162 / 105.7, 158 / 105.2, 98 / 83.3)
-template <int D, int GW, bool ONCE>
+// STEP: the decode step's tokens come with the launch (k_new).
+template <int D, int GW, bool ONCE, bool STEP>
 __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
     constexpr int LPK = D / 16;           // lanes per key
     constexpr int KPP = 64 / LPK;         // keys per K pass
@@ -82,7 +83,7 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
     // source rows.  The two dependent loads run beside those of the item's context and entry.
     const int ctx_cap = (int)(p.max_blocks * p.block_tokens);
     const int step_row = min(lane, (int)p.batch - 1);
-    const int step_ctx = p.k_new ? p.ctx_lens[step_row] : 0;
+    const int step_ctx = STEP ? p.ctx_lens[step_row] : 0;
     int lo, hi;
     size_t part_slot;
     const ItemCursor c = item_part<true>(p, lo, hi, part_slot);
@@ -102,16 +103,8 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
     const int raw_ctx = as_const(p.ctx_lens)[c.b];
     const int ctx = min(max(raw_ctx, 0), ctx_cap);
     // the row's own new token: its position, and the decoded tile whose wave stores it
-    const int papp = p.k_new && raw_ctx >= 1 && raw_ctx <= ctx_cap ? raw_ctx - 1 : -1;
+    const int papp = STEP && raw_ctx >= 1 && raw_ctx <= ctx_cap ? raw_ctx - 1 : -1;
     const int tnew = papp >= 0 ? min(papp / kTile, c.U - 1) : -1;
-    int step_block = -1, step_slot = 0;
-    if (p.k_new) {
-        const int pos = min(max(step_ctx, 1), ctx_cap) - 1;
-        const int e = p.block_tables[(size_t)step_row * p.max_blocks + pos / (int)p.block_tokens];
-        const bool is = lane < (int)p.batch && step_ctx >= 1 && step_ctx <= ctx_cap && (uint32_t)e < p.num_blocks;
-        step_block = is ? e : -1;
-        step_slot = pos % (int)p.block_tokens;
-    }
 
     // q' = clip(q) * scale * log2(e), in the K-side lane layout
     float qv[GW][16];
@@ -123,6 +116,17 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
             const float4 w = *reinterpret_cast<const float4*>(qrow + 4 * (sub + j * LPK));
             qv[h][4 * j] = w.x; qv[h][4 * j + 1] = w.y; qv[h][4 * j + 2] = w.z; qv[h][4 * j + 3] = w.w;
         }
+    }
+    // (behind the query rows, which are waited for first.  What it costs, a step of one tile or two
+    // pays: 3 x 40 tokens 7.9 -> 8.3 us, 60 x 20-100 9.6 -> 10.3; one gather per workgroup through
+    // LDS instead of one per wave 8.5 and 10.6)
+    int step_block = -1, step_slot = 0;
+    if constexpr (STEP) {
+        const int pos = min(max(step_ctx, 1), ctx_cap) - 1;
+        const int e = p.block_tables[(size_t)step_row * p.max_blocks + pos / (int)p.block_tokens];
+        const bool is = lane < (int)p.batch && step_ctx >= 1 && step_ctx <= ctx_cap && (uint32_t)e < p.num_blocks;
+        step_block = is ? e : -1;
+        step_slot = pos % (int)p.block_tokens;
     }
 #pragma unroll
     for (int h = 0; h < GW; ++h) {
@@ -152,9 +156,9 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
         const size_t row0 = ((size_t)(ok ? phys : 0) * p.hkv + hk) * p.block_tokens + slot0;
         const float* krow = reinterpret_cast<const float*>(p.k) + row0 * D;
         const float* vrow = reinterpret_cast<const float*>(p.v) + row0 * D;
+        const size_t new_el = ((size_t)c.b * p.hkv + hk) * D;
         // (its block may be another one where the context exceeds the bound)
         if (tile == tnew && c.y % (int)p.gsplit == 0) {
-            const size_t new_el = ((size_t)c.b * p.hkv + hk) * D;
             const int e = table[papp / (int)p.block_tokens];
             if (e >= 0 && (uint32_t)e < p.num_blocks && lane < D / 4) {
                 const size_t row = ((size_t)e * p.hkv + hk) * p.block_tokens + papp % (int)p.block_tokens;
@@ -184,6 +188,7 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
         if (v_early) load_v();
         // ---- scores ----
         float s[KPASS][GW], x[KPASS][16];
+        const int ts = STEP && tile == papp / kTile ? papp % kTile : -1;  // the row's own token's slot
 #pragma unroll
         for (int kp = 0; kp < KPASS; ++kp) {
 #pragma unroll
@@ -192,20 +197,24 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
                 x[kp][4 * j] = w.x; x[kp][4 * j + 1] = w.y; x[kp][4 * j + 2] = w.z; x[kp][4 * j + 3] = w.w;
             }
         }
-        // rows with a new token in this tile (looked up once the tile is on its way)
-        const uint64_t fresh = p.k_new ? __ballot(step_block == phys && step_slot / kTile == slot0 / kTile) : 0ull;
-        for (uint64_t m = fresh; m; m &= m - 1) {
-            const int r = __builtin_ctzll(m);
-            const int at = __builtin_amdgcn_readlane(step_slot, r) % kTile;
+        auto take_k = [&](const int at, const size_t el) {
 #pragma unroll
             for (int kp = 0; kp < KPASS; ++kp) {
                 if (kp * KPP + kk != at) continue;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const float4 w = load_new4(p.k_new, ((size_t)r * p.hkv + hk) * D + 4 * (sub + j * LPK), p.append_src);
+                    const float4 w = load_new4(p.k_new, el + 4 * (sub + j * LPK), p.append_src);
                     x[kp][4 * j] = w.x; x[kp][4 * j + 1] = w.y; x[kp][4 * j + 2] = w.z; x[kp][4 * j + 3] = w.w;
                 }
             }
+        };
+        if (STEP && ts >= 0) take_k(ts, new_el);
+        // the rows with another new token in this tile (looked up once the tile is on its way)
+        const uint64_t fresh =
+            STEP ? __ballot(step_block == phys && step_slot / kTile == slot0 / kTile && (ts < 0 || lane != c.b)) : 0ull;
+        for (uint64_t m = fresh; m; m &= m - 1) {
+            const int r = __builtin_ctzll(m);
+            take_k(__builtin_amdgcn_readlane(step_slot, r) % kTile, ((size_t)r * p.hkv + hk) * D);
         }
 #pragma unroll
         for (int kp = 0; kp < KPASS; ++kp) {
@@ -265,6 +274,10 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
         for (int vp = 0; vp < VPASS; ++vp) {
             const int slot = vp * VTPP + vt;
             float4 a = va[vp], b = vb[vp];
+            if (STEP && slot == ts) {
+                a = load_new4(p.v_new, new_el + 8 * vc, p.append_src);
+                b = load_new4(p.v_new, new_el + 8 * vc + 4, p.append_src);
+            }
             for (uint64_t m = fresh; m; m &= m - 1) {
                 const int r = __builtin_ctzll(m);
                 if (slot != __builtin_amdgcn_readlane(step_slot, r) % kTile) continue;
@@ -314,10 +327,16 @@ __global__ __launch_bounds__(256, 2) void decode_f32(DecodeParams p) {
     finish_item<D, GW>(p, comb, c, part_slot, hi - lo == c.U);
 }
 
+template <int D, int GW, bool STEP>
+void launch_decode(const DecodeParams& p, dim3 grid, hipStream_t s) {
+    if (p.gsplit == 1) hipLaunchKernelGGL((decode_f32<D, GW, true, STEP>), grid, dim3(kWaves * 64), 0, s, p);
+    else hipLaunchKernelGGL((decode_f32<D, GW, false, STEP>), grid, dim3(kWaves * 64), 0, s, p);
+}
+
 template <int D, int GW>
 void launch(const DecodeParams& p, dim3 grid, hipStream_t s) {
-    if (p.gsplit == 1) hipLaunchKernelGGL((decode_f32<D, GW, true>), grid, dim3(kWaves * 64), 0, s, p);
-    else hipLaunchKernelGGL((decode_f32<D, GW, false>), grid, dim3(kWaves * 64), 0, s, p);
+    if (p.k_new) launch_decode<D, GW, true>(p, grid, s);
+    else launch_decode<D, GW, false>(p, grid, s);
     if (p.item_parts > 1) {
         hipLaunchKernelGGL((decode_merge_items<D, GW>), dim3(p.hkv * p.gsplit, p.batch), dim3(256), 0, s, p);
     }
