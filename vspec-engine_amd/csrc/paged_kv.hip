@@ -821,10 +821,15 @@ struct DecodePlan {
 // context to be the same, by the same kind of model: a part of n tiles takes n * hypot(0.8, k *
 // 16 KB / 5.9 TB/s) us with k workgroups running.  Else an item's parts follow from its own
 // context, not from the host's bound: enough workgroups of at least 8 tiles to fill the card
-// once, and where that cuts an item in fewer than 6, up to three times as many of at least 16
-// tiles, so that the longest context's parts do not outlast the others (36 x 649-5195 tokens,
-// 144 items: 76 us with 3 parts, 61 with 10; 8 x 773-4188, 64 items: 49 us with 8, 56-66 with
-// more; 35 x 128-1024: 25 us, 31 in parts of 8 tiles).  *ws_parts: what the workspace is sized
+// once, and where that cuts an item in fewer than 4, up to three times as many of at least 16
+// tiles, so that the longest context's parts do not outlast the others.  Once / three times, us, at
+// 64, 86, 104, 128, 144 and 280 items (4 heads of 128):
+//   500-4000 tokens    41/46  54/62  64/64    73/77    84/81    208/144
+//   2000-4000          44/49  59/68  70/76    80/86    93/96    218/162
+//   100-1600           25/25  30/27  33/35    36/39    41/42    87/64
+//   120-7700           61/59  89/78  117/99   118/111  144/122  361/209
+// (64-element heads alike; from 86 items on three times was slower than the kernel before the item
+// split, 500-4000 tokens in heads of 64: 49 us against 38, 39 once).  *ws_parts: what the workspace is sized
 // for.  It never falls as the bound on the contexts rises and does not depend on `same`, so that
 // a workspace for the longest contexts serves every shorter one of as many sequences (not every
 // smaller batch: fewer items are cut into more parts).  Neither rule goes past three rounds of
@@ -845,9 +850,9 @@ uint32_t plan_f32_parts(uint64_t items, uint64_t tiles, uint32_t head_dim, uint6
     if (x > 0) return (uint32_t)((uint64_t)x < most ? (uint64_t)x : most);
     if (!same) {
         pl->part_tiles = 8;
-        if (items * 6 > slots) pl->far_tiles = 16;
+        if (items * 4 > slots) pl->far_tiles = 16;
         pl->near_parts = (uint32_t)(slots / items > 1 ? slots / items : 1);
-        const uint64_t far_parts = items * 6 > slots ? (3 * slots / items > 1 ? 3 * slots / items : 1) : 1;
+        const uint64_t far_parts = items * 4 > slots ? (3 * slots / items > 1 ? 3 * slots / items : 1) : 1;
         const uint64_t near = (tiles + 7) / 8 < pl->near_parts ? (tiles + 7) / 8 : pl->near_parts;
         const uint64_t far = (tiles + 15) / 16 < far_parts ? (tiles + 15) / 16 : far_parts;
         const uint64_t p = near > far ? near : far;
