@@ -64,7 +64,6 @@ __global__ __launch_bounds__(kWaves * 64, 2) void decode_mfma_f16(DecodeParams p
     __shared__ float qraw[ITEMS ? 1 : kQStage][ITEMS ? 1 : GW][ITEMS ? 1 : D];
     __shared__ float qs[ITEMS ? 1 : kWaves][GW][D];  // per wave: q' of its current item (ITEMS: for all)
     __shared__ int qexp[GW];                     // ITEMS: per head, the q' operand shift (qnorm_shift)
-    // per wave: QK B operands (hi, lo for each 32-wide d chunk), read back every tile
     __shared__ float comb[kSlots][kWaves][GW][D + 2];
     __shared__ float patch_val[kWaves][kTile][GW];
     __shared__ int patch_flag[kWaves][kTile];

@@ -1,9 +1,14 @@
 // paged_kv.hip -- gfx950 kernels and C-ABI for the Vspec paged KV-cache decode path.
 //
 // Kernels (all wave64):
-//   kv_append      block-table append of new K/V; int4 pools quantise on write
-//   kv_gather      block-table gather into [T][H][D] (raw bytes or dequantised f32)
-//   kv_compact     whole-block moves (compaction after eviction)
+//   kv_append_rows   block-table append of new K/V to f16 and f32 pools, with rotary k and q
+//   kv_append        the same to int4 pools, which quantise on write
+//   rope_q_rows, rope_q   the query rows of appends that do not carry them
+//   kv_gather_quads, kv_gather   block-table gather into [T][H][D] (raw bytes or dequantised f32)
+//   kv_gather_rows   single tokens by page and slot
+//   kv_compact       whole-block moves (compaction after eviction)
+// and the plan of a decode, whose kernels are in decode_f32.hip, decode_mfma.hip and
+// decode_mfma_int4.hip.
 //
 // The C-ABI is declared in include/vspec_rocm.h.
 #include <hip/hip_runtime.h>
@@ -874,7 +879,6 @@ uint32_t plan_f32_parts(uint64_t items, uint64_t tiles, uint32_t head_dim, uint6
     }
     return parts;
 }
-
 
 // With every context known to be the same (min_ctx_len == the context bound), the split
 // of the MFMA kernels (kv_common.h work_split with equal shares, as for any batch whose
