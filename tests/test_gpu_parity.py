@@ -898,10 +898,9 @@ def _fused_step_case(oracle, gpu, dtype, Hq, Hkv, D, P, pt, src16, ctx, seed):
 @pytest.mark.parametrize("dtype", [DTYPE_F16, DTYPE_INT4])
 def test_decode_step_in_hip_graph(oracle, gpu, flag_gate, dtype):
     """A decode step (fused append + attention) captured into a HIP graph after one eager
-    call on the capture stream (which sets up that stream's merge counters and the
-    workspace): every replay, with eager decodes of another batch and synchronisations in
-    between, equals the eager step bit for bit, and the pool bytes stay those of the eager
-    append (every launch returns the counters to zero; no memset is recorded)."""
+    call on the capture stream: every replay, with eager decodes of another batch and
+    synchronisations in between, equals the eager step bit for bit, and the pool bytes stay
+    those of the eager append (no memset is recorded, no state outlives a launch)."""
     import torch
     import vspec_rocm as vr
 
@@ -928,7 +927,7 @@ def test_decode_step_in_hip_graph(oracle, gpu, flag_gate, dtype):
 
     s.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(s):
-        step()  # eager: counters and workspace exist before capture
+        step()  # eager first
     torch.cuda.synchronize()
     want = out.clone()
     want_pool = [None if a is None else a.copy() for a in pool_bytes(pool)]

@@ -358,3 +358,40 @@ def test_f32_partition_tokens_is_the_part_size(gpu, pt):
                 assert abs(float(got - want)) <= 1e-5, (b, h, i)
             assert bool((ml[b, h, len(ranges):] == 7e7).all())
         at += n
+
+
+@pytest.mark.parametrize("rows", [7, 66])
+def test_f32_step_in_hip_graph(gpu, rows):
+    """f32 pools, items cut into parts, the append in the decode's launch (up to 64 rows) and ahead of
+    it (more), captured: every replay, with the step's tokens replaced in the pool and eager work
+    in between, equals the eager step bit for bit, pool bytes included."""
+    import torch
+
+    lens = [1 + (211 * b) % 900 for b in range(rows)]
+    vr, pools, tables, ctx, q, new, _ = _decode_setup(gpu, "f32", lens, 8, 2, 128, 16)
+    want = vr.paged_decode_step(pools[0], tables, ctx, q, *new, max_ctx_len=max(lens))
+    out = torch.empty_like(q)
+    d = vr.make_decode_desc(pools[1], tables, ctx, q, out, max(lens))
+    ws = torch.empty(vr.decode_workspace_bytes(d), dtype=torch.uint8, device=gpu)
+    assert ws.numel()
+    s = torch.cuda.Stream()
+
+    def step():
+        vr.paged_decode_step(pools[1], tables, ctx, q, *new, max_ctx_len=max(lens), out=out, workspace=ws, stream=s.cuda_stream)
+
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        step()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        step()
+    for rep in range(4):
+        vr.kv_append(pools[1], tables, ctx - 1, *(x[:, None].neg().contiguous() for x in new))  # what the step replaces
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), rep
+        assert _same_pools(*pools), rep
+        vr.paged_decode(pools[0], tables, ctx, q, max_ctx_len=max(lens))
