@@ -653,7 +653,7 @@ def main():
     # timed steps run in the card's steady state.  Timed straight after the pool set-up, a
     # short run lands in the card's transient at the start of a load (north star: launches of
     # ~166 us, then ~185-190 us for a few ms, then ~170 us), so 20 steps read 3 % slower and
-    # vary more between boxes.
+    # vary more from run to run.
     pc = None
     if not args.no_probe:
         log("probe ceilings ...")
